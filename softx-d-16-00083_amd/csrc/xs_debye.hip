@@ -27,6 +27,7 @@
 #include <mutex>
 #include <vector>
 
+#include "xs_debye_moments.h"
 #include "xs_internal.h"
 #include "xs_sincos.h"
 
@@ -58,33 +59,6 @@ struct MeshInfo {
   double dq;
   uint32_t uniform, pad;
 };
-
-// sin and cos of 2 pi r for any double r, from a table of the 64 points
-// k/64 of a turn (tab[k] = (sin, cos) of 2 pi k/64, within an ulp) and a
-// short series: t = r - rint(r) and u = t - n/64 with n = rint(64 t) are
-// exact (u is a multiple of ulp(t), |u| <= |t|), |u| <= 1/128, so
-// x = 2 pi u lies within 0.0491 rad, where sin through x^9 and cos through
-// x^8 leave truncation errors below 1e-19 relative; then
-// sin(a + x) = sin a cos x + cos a sin x and likewise for cos.  24 VALU
-// instructions and one LDS read against 37 for the quarter-turn series of
-// sincos_2pi, with the same few-ulp result.
-__device__ __forceinline__ void sincos_2pi_tab(double r, const double2 *tab, double *s, double *c) {
-  const double t = r - rint(r);
-  const double n = rint(64.0 * t);
-  const double x = kTwoPi * fma(n, -1.0 / 64.0, t);
-  const double x2 = x * x;
-  double ps = fma_k(x2, inv_factorial(9), -inv_factorial(7));
-  ps = fma_k(ps, x2, inv_factorial(5));
-  ps = fma_k(ps, x2, -inv_factorial(3));
-  const double sx = fma(x * x2, ps, x);
-  double pc = fma_k(x2, inv_factorial(8), -inv_factorial(6));
-  pc = fma_k(pc, x2, inv_factorial(4));
-  pc = fma_k(pc, x2, -inv_factorial(2));
-  const double cx = fma(x2, pc, 1.0);
-  const double2 a = tab[(int)n & 63];
-  *s = fma(a.x, cx, a.y * sx);
-  *c = fma(a.y, cx, -(a.x * sx));
-}
 
 // S[p][k] /= q[k] (0 where q[k] = 0): debye_kernel adds up
 // q sin(q r)/(q r + 1e-8) and leaves the division by q to this pass.
@@ -262,14 +236,114 @@ __global__ __launch_bounds__(kBlock) void debye_kernel(const double *__restrict_
   }
 }
 
-static bool uniform_mesh(const std::vector<double> &q, double *dq) {
-  const size_t n = q.size();
-  *dq = n > 1 ? (q[n - 1] - q[0]) / (double)(n - 1) : 0.0;
-  double scale = 0.0;
-  for (double v : q) scale = std::max(scale, std::fabs(v));
-  for (size_t k = 0; k < n; ++k)
-    if (std::fabs(q[k] - (q[0] + (double)k * *dq)) > 1e-13 * scale) return false;
-  return true;
+// Bounding box of the atoms (partials of blocks 0..kBoxBlocks-1: low and high
+// x, y, z; NaN in any coordinate makes all six NaN) and, in the last block,
+// the mesh: its step, max |q|, and whether it is uniform and finite.
+constexpr int kBoxBlocks = 64;
+struct BoxOut {
+  double lo_hi[kBoxBlocks][6];
+  double dq, qmax;
+  int32_t uniform, finite;
+};
+
+__global__ __launch_bounds__(256) void box_kernel(const double *__restrict__ xyz, size_t n,
+                                                  const double *__restrict__ q, unsigned nq,
+                                                  BoxOut *__restrict__ out) {
+  __shared__ double sh[256];
+  if (blockIdx.x == kBoxBlocks) {
+    const double dq = nq > 1 ? (q[nq - 1] - q[0]) / (double)(nq - 1) : 0.0;
+    double m = 0.0;
+    int bad = 0;
+    for (unsigned k = threadIdx.x; k < nq; k += 256) {
+      m = fmax(m, fabs(q[k]));
+      bad |= !(fabs(q[k]) < HUGE_VAL);
+    }
+    sh[threadIdx.x] = m;
+    bad = __syncthreads_or(bad);
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + w]);
+      __syncthreads();
+    }
+    m = sh[0];
+    int off = 0;
+    for (unsigned k = threadIdx.x; k < nq; k += 256)
+      off |= fabs(q[k] - (q[0] + (double)k * dq)) > 1e-13 * m;
+    off = __syncthreads_or(off);
+    if (threadIdx.x == 0) {
+      out->dq = dq;
+      out->qmax = m;
+      out->uniform = !off;
+      out->finite = !bad;
+    }
+    return;
+  }
+  // v: low x, y, z and minus high x, y, z
+  double v[6];
+  for (int c = 0; c < 6; ++c) v[c] = HUGE_VAL;
+  int bad = 0;
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)kBoxBlocks * 256)
+    for (int c = 0; c < 3; ++c) {
+      const double u = xyz[c * n + i];
+      v[c] = fmin(v[c], u);
+      v[3 + c] = fmin(v[3 + c], -u);
+      bad |= !(fabs(u) < HUGE_VAL);
+    }
+  for (int c = 0; c < 6; ++c) {
+    for (int w = 32; w > 0; w >>= 1) v[c] = fmin(v[c], __shfl_down(v[c], w, 64));
+    if ((threadIdx.x & 63) == 0) sh[(threadIdx.x >> 6) * 6 + c] = v[c];
+  }
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x < 6) {
+    const int c = threadIdx.x;
+    const double m = fmin(fmin(sh[c], sh[6 + c]), fmin(sh[12 + c], sh[18 + c]));
+    out->lo_hi[blockIdx.x][c % 3 * 2 + c / 3] = bad ? __builtin_nan("") : c < 3 ? m : -m;
+  }
+}
+
+static MeshBox mesh_box(const BoxOut &o) {
+  MeshBox in;
+  in.dq = o.dq;
+  in.Q = o.qmax;
+  in.uniform = o.uniform != 0;
+  in.finite = o.finite != 0;
+  double r2 = 0.0;
+  for (int c = 0; c < 3; ++c) {
+    double lo = HUGE_VAL, hi = -HUGE_VAL;
+    for (int b = 0; b < kBoxBlocks; ++b) {
+      if (std::isnan(o.lo_hi[b][2 * c])) in.finite = false;
+      lo = std::min(lo, o.lo_hi[b][2 * c]);
+      hi = std::max(hi, o.lo_hi[b][2 * c + 1]);
+    }
+    if (hi >= lo) r2 += (hi - lo) * (hi - lo);
+  }
+  in.R = std::sqrt(r2);
+  return in;
+}
+
+// Tiles that stay inside one (element, block) segment and their pairs.
+static void tile_tables(const std::vector<uint32_t> &seg_cnt, unsigned n_el, unsigned nblocks,
+                        std::vector<Tile> *tiles, std::vector<Item> *items) {
+  std::vector<uint32_t> el_first(n_el + 1);
+  uint32_t off = 0;
+  for (unsigned e = 0; e < n_el; ++e) {
+    el_first[e] = (uint32_t)tiles->size();
+    for (unsigned b = 0; b < nblocks; ++b) {
+      const uint32_t cnt = seg_cnt[e * nblocks + b];
+      for (uint32_t t = 0; t < cnt; t += kTT)
+        tiles->push_back(Tile{off + t, std::min<uint32_t>(kTT, cnt - t), e, b});
+      off += cnt;
+    }
+  }
+  el_first[n_el] = (uint32_t)tiles->size();
+  unsigned p = 0;
+  for (unsigned a = 0; a < n_el; ++a)
+    for (unsigned b = a; b < n_el; ++b, ++p)
+      for (uint32_t ti = el_first[a]; ti < el_first[a + 1]; ++ti)
+        for (uint32_t tj = (a == b ? ti : el_first[b]); tj < el_first[b + 1]; ++tj) {
+          const uint32_t bi = (*tiles)[ti].blk, bj = (*tiles)[tj].blk;
+          const uint32_t lo = std::min(bi, bj), hi = std::max(bi, bj);
+          items->push_back(Item{ti, tj, p, nblocks * lo - (lo * (lo + 1)) / 2 + hi});
+        }
 }
 
 static int run(xs_ctx *ctx, const double *xyz_in, size_t n, const unsigned *el_count, unsigned n_el,
@@ -278,44 +352,13 @@ static int run(xs_ctx *ctx, const double *xyz_in, size_t n, const unsigned *el_c
   const unsigned ntypes = ntypes_of(n_el);
   const unsigned nparts = nblocks * (nblocks + 1) / 2;
   const size_t ssize = (size_t)ntypes * nparts * nq;
-  // tiles that stay inside one (element, block) segment
-  std::vector<Tile> tiles;
-  std::vector<uint32_t> el_first(n_el + 1);
-  uint32_t off = 0;
-  for (unsigned e = 0; e < n_el; ++e) {
-    el_first[e] = (uint32_t)tiles.size();
-    for (unsigned b = 0; b < nblocks; ++b) {
-      const uint32_t cnt = blk_count ? blk_count[e * nblocks + b] : el_count[e];
-      for (uint32_t t = 0; t < cnt; t += kTT)
-        tiles.push_back(Tile{off + t, std::min<uint32_t>(kTT, cnt - t), e, b});
-      off += cnt;
-    }
-  }
-  el_first[n_el] = (uint32_t)tiles.size();
-  std::vector<Item> items;
-  unsigned p = 0;
-  for (unsigned a = 0; a < n_el; ++a)
-    for (unsigned b = a; b < n_el; ++b, ++p)
-      for (uint32_t ti = el_first[a]; ti < el_first[a + 1]; ++ti)
-        for (uint32_t tj = (a == b ? ti : el_first[b]); tj < el_first[b + 1]; ++tj) {
-          const uint32_t bi = tiles[ti].blk, bj = tiles[tj].blk;
-          const uint32_t lo = std::min(bi, bj), hi = std::max(bi, bj);
-          items.push_back(Item{ti, tj, p, nblocks * lo - (lo * (lo + 1)) / 2 + hi});
-        }
-  std::vector<double> qh(nq);
-  if (device) {
-    XS_HIP_CHECK(hipMemcpyAsync(qh.data(), q_in, (size_t)nq * 8, hipMemcpyDeviceToHost, ctx->stream));
-    XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-  } else {
-    std::memcpy(qh.data(), q_in, (size_t)nq * 8);
-  }
-  double dq = 0.0;
-  const bool uniform = uniform_mesh(qh, &dq);
-
-  const size_t tb = tiles.size() * sizeof(Tile), ib = items.size() * sizeof(Item);
-  XS_TRY(ensure_workspace(ctx, Carver::need({device ? 0 : 3 * n * 8, device ? 0 : (size_t)nq * 8,
-                                             device ? 0 : ssize * 8, tb, ib})));
+  const std::vector<uint32_t> seg_cnt(blk_count ? blk_count : el_count,
+                                      blk_count ? blk_count + (size_t)n_el * nblocks
+                                                : el_count + n_el);
+  XS_TRY(ensure_workspace(ctx, Carver::need({sizeof(BoxOut), device ? 0 : 3 * n * 8,
+                                             device ? 0 : (size_t)nq * 8, device ? 0 : ssize * 8})));
   Carver cv(ctx->ws);
+  BoxOut *box_d = cv.take<BoxOut>(1);
   const double *xyz = xyz_in, *qd = q_in;
   double *Sd = S_out;
   if (!device) {
@@ -327,38 +370,54 @@ static int run(xs_ctx *ctx, const double *xyz_in, size_t n, const unsigned *el_c
     xyz = x2;
     qd = q2;
   }
-  Tile *td = cv.take<Tile>(tiles.size());
-  Item *idv = cv.take<Item>(items.size());
-  XS_TRY(ensure_pinned(ctx, tb + ib + 256));
-  // the pinned buffer may still feed an earlier upload: wait for the stream
+  XS_TRY(ensure_pinned(ctx, sizeof(BoxOut)));
+  hipLaunchKernelGGL(box_kernel, dim3(kBoxBlocks + 1), dim3(256), 0, ctx->stream, xyz, n, qd, nq,
+                     box_d);
+  XS_HIP_CHECK(hipGetLastError());
+  XS_HIP_CHECK(hipMemcpyAsync(ctx->pin, box_d, sizeof(BoxOut), hipMemcpyDeviceToHost, ctx->stream));
+  // also frees the pinned staging of an earlier upload
   XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-  std::memcpy(ctx->pin, tiles.data(), tb);
-  std::memcpy(static_cast<char *>(ctx->pin) + align_up(tb, 256), items.data(), ib);
-  if (tb) XS_HIP_CHECK(hipMemcpyAsync(td, ctx->pin, tb, hipMemcpyHostToDevice, ctx->stream));
-  if (ib)
-    XS_HIP_CHECK(hipMemcpyAsync(idv, static_cast<char *>(ctx->pin) + align_up(tb, 256), ib,
-                                hipMemcpyHostToDevice, ctx->stream));
-  XS_HIP_CHECK(hipMemsetAsync(Sd, 0, ssize * 8, ctx->stream));
-  if (!items.empty()) {
-    hipEvent_t ev;
-    XS_TRY(prof_begin(ctx, "debye", &ev));
-    dim3 grid((unsigned)items.size(), (nq + kQBlock - 1) / kQBlock);
-    if (uniform)
-      hipLaunchKernelGGL(debye_kernel<true>, grid, dim3(kBlock), 0, ctx->stream, xyz, xyz + n,
-                         xyz + 2 * n, td, idv, qd, nq, dq, nparts, Sd, nullptr);
-    else
-      hipLaunchKernelGGL(debye_kernel<false>, grid, dim3(kBlock), 0, ctx->stream, xyz, xyz + n,
-                         xyz + 2 * n, td, idv, qd, nq, dq, nparts, Sd, nullptr);
-    hipLaunchKernelGGL(divide_by_q_kernel, dim3((unsigned)std::min<size_t>((ssize + 255) / 256, 4096)),
-                       dim3(256), 0, ctx->stream, Sd, qd, nq, ssize);
-    XS_HIP_CHECK(hipGetLastError());
-    XS_TRY(prof_end(ctx, "debye", ev));
+  const MeshBox in = mesh_box(*static_cast<const BoxOut *>(ctx->pin));
+
+  MomentPlan mp;
+  if (plan_moments(in, seg_cnt, n_el, nblocks, nq, ctx->cu_count, &mp)) {
+    XS_TRY(ensure_aux(ctx, moments_table_bytes(seg_cnt, n_el, nblocks, ctx->cu_count)));
+    XS_TRY(run_moments(ctx, mp, xyz, n, seg_cnt, n_el, nblocks, in, qd, nq, Sd, ctx->aux));
+  } else {
+    std::vector<Tile> tiles;
+    std::vector<Item> items;
+    tile_tables(seg_cnt, n_el, nblocks, &tiles, &items);
+    const size_t tb = tiles.size() * sizeof(Tile), ib = items.size() * sizeof(Item);
+    XS_TRY(ensure_aux(ctx, align_up(tb, 256) + ib + 256));
+    Tile *td = static_cast<Tile *>(ctx->aux);
+    Item *idv = reinterpret_cast<Item *>(static_cast<char *>(ctx->aux) + align_up(tb, 256));
+    XS_TRY(ensure_pinned(ctx, align_up(tb, 256) + ib));
+    std::memcpy(ctx->pin, tiles.data(), tb);
+    std::memcpy(static_cast<char *>(ctx->pin) + align_up(tb, 256), items.data(), ib);
+    if (tb) XS_HIP_CHECK(hipMemcpyAsync(td, ctx->pin, tb, hipMemcpyHostToDevice, ctx->stream));
+    if (ib)
+      XS_HIP_CHECK(hipMemcpyAsync(idv, static_cast<char *>(ctx->pin) + align_up(tb, 256), ib,
+                                  hipMemcpyHostToDevice, ctx->stream));
+    XS_HIP_CHECK(hipMemsetAsync(Sd, 0, ssize * 8, ctx->stream));
+    if (!items.empty()) {
+      hipEvent_t ev;
+      XS_TRY(prof_begin(ctx, "debye", &ev));
+      dim3 grid((unsigned)items.size(), (nq + kQBlock - 1) / kQBlock);
+      if (in.uniform)
+        hipLaunchKernelGGL(debye_kernel<true>, grid, dim3(kBlock), 0, ctx->stream, xyz, xyz + n,
+                           xyz + 2 * n, td, idv, qd, nq, in.dq, nparts, Sd, nullptr);
+      else
+        hipLaunchKernelGGL(debye_kernel<false>, grid, dim3(kBlock), 0, ctx->stream, xyz, xyz + n,
+                           xyz + 2 * n, td, idv, qd, nq, in.dq, nparts, Sd, nullptr);
+      hipLaunchKernelGGL(divide_by_q_kernel,
+                         dim3((unsigned)std::min<size_t>((ssize + 255) / 256, 4096)), dim3(256), 0,
+                         ctx->stream, Sd, qd, nq, ssize);
+      XS_HIP_CHECK(hipGetLastError());
+      XS_TRY(prof_end(ctx, "debye", ev));
+    }
   }
   if (!device) {
     XS_HIP_CHECK(hipMemcpyAsync(S_out, Sd, ssize * 8, hipMemcpyDeviceToHost, ctx->stream));
-    XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-  } else {
-    // keep the pinned staging alive until the uploads have been consumed
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   }
   return XS_OK;

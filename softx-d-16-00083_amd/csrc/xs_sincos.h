@@ -57,4 +57,32 @@ __device__ __forceinline__ void sincos_2pi(double r, double *s, double *c) {
   *c = ((q ^ (q >> 1)) & 1) ? -cc : cc;
 }
 
+// sin and cos of 2 pi r for any double r, from a table of the 64 points
+// k/64 of a turn (tab[k] = (sin, cos) of 2 pi k/64, within an ulp) and a
+// short series: t = r - rint(r) and u = t - n/64 with n = rint(64 t) are
+// exact (u is a multiple of ulp(t), |u| <= |t|), |u| <= 1/128, so
+// x = 2 pi u lies within 0.0491 rad, where sin through x^9 and cos through
+// x^8 leave truncation errors below 1e-19 relative; then
+// sin(a + x) = sin a cos x + cos a sin x and likewise for cos.  24 VALU
+// instructions and one LDS read against 37 for the quarter-turn series of
+// sincos_2pi, with the same few-ulp result.
+__device__ __forceinline__ void sincos_2pi_tab(double r, const double2 *tab, double *s, double *c) {
+  const double t = r - rint(r);
+  const double n = rint(64.0 * t);
+  constexpr double kTwoPi = 6.283185307179586476925286766559;
+  const double x = kTwoPi * fma(n, -1.0 / 64.0, t);
+  const double x2 = x * x;
+  double ps = fma_k(x2, inv_factorial(9), -inv_factorial(7));
+  ps = fma_k(ps, x2, inv_factorial(5));
+  ps = fma_k(ps, x2, -inv_factorial(3));
+  const double sx = fma(x * x2, ps, x);
+  double pc = fma_k(x2, inv_factorial(8), -inv_factorial(6));
+  pc = fma_k(pc, x2, inv_factorial(4));
+  pc = fma_k(pc, x2, -inv_factorial(2));
+  const double cx = fma(x2, pc, 1.0);
+  const double2 a = tab[(int)n & 63];
+  *s = fma(a.x, cx, a.y * sx);
+  *c = fma(a.y, cx, -(a.x * sx));
+}
+
 }  // namespace xs

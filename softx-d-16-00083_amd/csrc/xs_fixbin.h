@@ -69,5 +69,54 @@ XS_FIX_HD inline uint32_t fix_from_rsq(double s, double y, double inv_bin, doubl
   return (uint32_t)(w >> 32);
 }
 
+// The same floor with a window slot folded in, for squared distances in units
+// of (2 bins)^2.  y ~ 1/sqrt(s) within 2^-23, g = s y, and
+// g (3 - g y) = 2 sqrt(s) (1 - 3e^2/2 - e^3/2) is the distance in bins in
+// three operations, the last of them adding m = 2^18 + off + eff, where
+// slot = bin + off lies in [0, 2^18): T = RN(estimate + m) lies in
+// [2^18, 2^19), where the ulp of a double is 2^-34, so T's high word is
+// 0x41100000 + 4 slot + (2 bits of fraction), a byte offset after one AND, and
+// its low word the rest of the fraction.  off is any integer below 2^31 (the
+// grid may be wider than 2^18 bins), so off + eff can round: eff is requested
+// larger by more than that rounding and then taken as what m holds,
+// eff = m - (2^18 + off) exactly, eff >= E + 2^-33.  With phi the whole
+// fraction, phi >= 2 eff + 2^-34 puts the IEEE quotient t into
+// (slot - off, slot - off + 1):
+//   t >= K + phi - eff - 2^-35 - E > K,
+//   t <= K + 1 - 2^-34 - eff + 2^-35 + E < K + 1.
+// The low word alone is compared with lm1 >= 2 eff 2^34: a smaller phi always
+// has a low word at most lm1 (and so have three more intervals of phi, whose
+// pairs the exact evaluation takes for nothing).
+struct FixSlot {
+  double m;      // 2^18 + off + eff
+  uint32_t lm1;  // the estimate is floored directly when the low word > lm1
+};
+
+XS_FIX_HD inline FixSlot fix_slot(double band, int32_t off) {
+  const double E = 0.5 - band;
+  const double base = 0x1p18 + (double)off;
+  if (!(E >= 0.0 && E <= 0x1p-6)) return FixSlot{base, 0xffffffffu};
+  const double m = base + (E + 0x1p-32 + (base < 0.0 ? -base : base) * 0x1p-52);
+  const double eff = m - base;
+  return FixSlot{m, (uint32_t)__builtin_ceil(2.0 * eff * 0x1p34) + 1u};
+}
+
+// High word of T; its low word in lo.
+XS_FIX_HD inline uint32_t split_fixed(double T, uint32_t &lo) {
+  uint64_t w;
+  __builtin_memcpy(&w, &T, sizeof w);
+  lo = (uint32_t)w;
+  return (uint32_t)(w >> 32);
+}
+
+// T's high word from s and y ~ 1/sqrt(s); its low word in lo.
+XS_FIX_HD inline uint32_t fix_slot_from_rsq(double s, double y, double m, uint32_t &lo) {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+  const double g = s * y;
+  return split_fixed(__builtin_fma(g, __builtin_fma(-g, y, 3.0), m), lo);
+}
+
 }  // namespace hist
 }  // namespace xs

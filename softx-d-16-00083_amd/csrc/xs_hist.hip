@@ -10,11 +10,11 @@
 //
 // Kernel.  One work item = (pair type of a structure, I unit, run of J
 // tiles); an I unit is one tile (FP32 binning) or two neighbouring tiles
-// (FP64 binning, two I atoms per thread, so each J atom read from LDS serves
-// two pairs).  The I atoms sit in registers; J tiles are sorted by the
+// (FP64 binning, whose squared distances come from the matrix instruction, see
+// hist_kernel_f64).  The I atoms sit in registers; J tiles are sorted by the
 // lowest bin their pairs with the I unit can reach (from the boxes) and
-// swept in that order; J atoms are staged 256 at a time in LDS and read by
-// every lane at the same address.  Counts go to a circular LDS window of
+// swept in that order; with FP32 binning J atoms are staged 256 at a time in
+// LDS and read by every lane at the same address.  Counts go to an LDS window of
 // WCAP uint32 bins that only slides up; bins the remaining J tiles cannot
 // reach are flushed to the uint64 histogram with one atomic per non-zero bin,
 // so flush traffic per item is at most nhist + WCAP whatever the pair count.
@@ -59,7 +59,6 @@ namespace hist {
 
 constexpr int kStage = 256;      // J atoms staged in LDS per step
 constexpr int kBoxBlocks = 512;  // partial bounding boxes
-constexpr int kChunk = 256;      // FP64 binning: J atoms between barriers (8 KB of records)
 constexpr double kFill = 0.94 * kTile;  // target atoms in the fullest cell
 constexpr uint32_t kMaxCellsPerAxis = 256;
 
@@ -80,7 +79,7 @@ struct Args {
   unsigned long long *overflow;
   const double *rec;  // FP64 binning: J records, 4 per atom (hist_tile_records)
   uint32_t quot_f32;  // FP32 binning: the bin passed quot_f32_check_kernel
-  uint32_t narrow;    // FP64 binning: every pair type has at most kNarrowMax bins
+  double scale;       // FP64 binning: 1/(2 bin), the unit of the records
 };
 
 // ---------------------------------------------------------------- prep kernels
@@ -358,19 +357,6 @@ __device__ __forceinline__ double sqrt_over_bin(double s, double inv_bin) {
   return g * fma(t, -0.5 * inv_bin, 1.5 * inv_bin);
 }
 
-template <class T>
-__device__ __forceinline__ uint32_t bin_index(T s, T bin, double inv_bin, double band,
-                                              uint32_t nhist);
-
-template <>
-__device__ __forceinline__ uint32_t bin_index<double>(double s, double bin, double inv_bin,
-                                                      double band, uint32_t nhist) {
-  const double kd = sqrt_over_bin(s, inv_bin);
-  if (__builtin_expect(fabs(__builtin_amdgcn_fract(kd) - 0.5) < band, 1)) return (uint32_t)kd;
-  const double t = __builtin_sqrt(s) / bin;
-  return t < (double)nhist ? (uint32_t)t : nhist;
-}
-
 // float: (unsigned)(sqrtf(s) / bin) of the reference GPU kernel in IEEE
 // single precision.  sqrtf is the IEEE one; the division is evaluated as
 // (float)(r * inv_bin) in double, inv_bin = RN(1 / (double)bin).  That
@@ -471,34 +457,22 @@ __global__ void sqrt_f32_check_kernel(unsigned long long *bad) {
   if (b2) atomicAdd(&bad[2], b2);
 }
 
-template <>
-__device__ __forceinline__ uint32_t bin_index<float>(float s, float bin, double inv_bin,
-                                                     double band, uint32_t nhist) {
-  (void)bin;
-  (void)band;
+__device__ __forceinline__ uint32_t bin_index_f32(float s, double inv_bin, uint32_t nhist) {
   const float t = dist_over_bin_f32(s, inv_bin);
   return t < (float)nhist ? (uint32_t)t : nhist;
 }
 
-// Fast part of the FP64 bin_index: the estimate's floor and whether it may
-// differ from the IEEE result (then exact_bin decides).
+// The estimate's floor and whether it may differ from the IEEE result (then
+// exact_bin decides).
 __device__ __forceinline__ uint32_t fast_bin(double s, double inv_bin, double band, bool &bad) {
   const double kd = sqrt_over_bin(s, inv_bin);
   bad = !(fabs(__builtin_amdgcn_fract(kd) - 0.5) < band);
   return (uint32_t)kd;
 }
 
-// The same fast path in fixed point (xs_fixbin.h) for grids of at most
-// kNarrowMax bins: T's high word kFixHi + bin, its low word L; the estimate
-// is floored directly when L > FixBand::lm1.
-__device__ __forceinline__ uint32_t fix_bin(double s, double inv_bin, double m, uint32_t &lo) {
-  return fix_from_rsq(s, __builtin_amdgcn_rsq(s), inv_bin, m, lo);
-}
-
-template <class T>
-__device__ __forceinline__ uint32_t exact_bin(T s, T bin, uint32_t nhist) {
-  const T t = (T)__builtin_sqrt((double)s) / bin;
-  return t < (T)nhist ? (uint32_t)t : nhist;
+__device__ __forceinline__ uint32_t exact_bin(double s, double bin, uint32_t nhist) {
+  const double t = __builtin_sqrt(s) / bin;
+  return t < (double)nhist ? (uint32_t)t : nhist;
 }
 
 // An atom index the compiler cannot see through, so that coordinates read
@@ -509,30 +483,28 @@ __device__ __forceinline__ size_t opaque_index(size_t g) {
   return g;
 }
 
-// FP64 fast path of one I atom: its coordinates relative to the centre c of
-// a J tile's box times -2, and its squared distance from c.  With the J
-// atoms' coordinates relative to c (rj') and their squared norms (nj) in the
-// J records, |ri - rj|^2 = n + nj + (-2 ri').rj' costs one add and three
-// FMAs.
-struct IAtom {
-  double ax, ay, az, n;
-};
-
 // Centre c of a J tile's box (bi, 6 doubles) and the half-width of the FP64
 // fast path's band for pairs formed relative to c.  The bound below is
 // symmetric in the two atoms, so it holds with the J box as the one of
 // radius rho.
 // Relative to IEEE sqrt(s)/bin the estimate errs by (a) below nhist 2^-45.3
 // bins from v_rsq_f64, the Newton step and the roundings of the reference
-// expression, and (b) below u (64 R^2 + 36 R + 10 T) bins from forming s as
+// expression, and (b) below u (32 R^2 / D + 44 R + 14 T) bins from forming s as
 // |ri'|^2 + |rj'|^2 - 2 ri'.rj' with shifted, rounded coordinates, where
-// u = 2^-53, R bounds |ri - c| in bins and T = distance in bins <= nhist + 1
-// where it matters: the rounding error of s is below
-// u (32 rho^2 + 36 rho d + 10 d^2) for |ri - c| <= rho, |rj - c| <= rho + d,
+// u = 2^-53, R bounds |ri - c| in bins, T = distance in bins <= nhist + 1
+// where it matters, and D = max(1/2, dmin) with dmin a lower bound of the
+// distance in bins (from the boxes): the rounding error of s is below
+// u (32 rho^2 + 44 rho d + 14 d^2) for |ri - c| <= rho, |rj - c| <= rho + d,
 // and divides by d to give the error of the root for d >= bin / 2 (below
-// that, both floors are 0).  Both bounds are taken 16-fold.
+// that, both floors are 0).  (The product's FMAs run over x, y, z, then
+// |ri'|^2, from |rj'|^2: partial sums below 3 rho^2 + 2 rho d.  The
+// coordinates' rounding to units of 2 bins adds one more shift rounding.)
+// Both bounds are taken 16-fold.  (With D = 1/2 for every tile pair, the R^2
+// term sent 3% of the J blocks of a 366,000-atom cube to the exact path, for
+// nothing: 18.1 cycles a wave of pairs against 16.6.)
 __device__ __forceinline__ double tile_band(const double *bi, double band0, double inv_bin,
-                                            uint32_t nhist, double c[3]) {
+                                            uint32_t nhist, double dmin, double c[3],
+                                            double &R) {
   double h2 = 0.0, cm = 0.0;
   for (int a = 0; a < 3; ++a) {
     c[a] = 0.5 * (bi[a] + bi[3 + a]);
@@ -540,8 +512,8 @@ __device__ __forceinline__ double tile_band(const double *bi, double band0, doub
     h2 = fma(e, e, h2);
     cm = fmax(cm, fabs(c[a]));
   }
-  const double R = (0.5 * sqrt(h2) * (1.0 + 0x1p-20) + 0x1p-40 * cm) * inv_bin;
-  return band0 - 0x1p-49 * (fma(64.0 * R, R, 36.0 * R) + 10.0 * ((double)nhist + 1.0));
+  R = (0.5 * sqrt(h2) * (1.0 + 0x1p-20) + 0x1p-40 * cm) * inv_bin;
+  return band0 - 0x1p-49 * (fma(32.0 * R / fmax(dmin, 0.5), R, 44.0 * R) + 14.0 * ((double)nhist + 1.0));
 }
 
 // FP32 groups of 8 J atoms (not the like-element diagonal tile): the
@@ -593,23 +565,24 @@ __device__ __forceinline__ void pair_group8_f32(float xi, float yi, float zi, co
   }
 }
 
-template <class T, int WCAP, bool DIAG>
-__device__ __forceinline__ void pair_block(T xi, T yi, T zi, uint32_t il, const T *sx,
-                                           const T *sy, const T *sz, uint32_t cn,
-                                           uint32_t jbase, T bin, double inv_bin, double band,
-                                           uint32_t nhist, uint32_t B, uint32_t wlim, uint32_t D,
-                                           uint32_t *win, unsigned long long *__restrict__ hp,
-                                           unsigned long long *__restrict__ ovf) {
+// FP32: J atoms one at a time (the like-element diagonal, the last of a stage).
+template <int WCAP, bool DIAG>
+__device__ __forceinline__ void pair_block_f32(float xi, float yi, float zi, uint32_t il,
+                                               const float *sx, const float *sy, const float *sz,
+                                               uint32_t cn, uint32_t jbase, double inv_bin,
+                                               uint32_t nhist, uint32_t B, uint32_t wlim, uint32_t D,
+                                               uint32_t *win, unsigned long long *__restrict__ hp,
+                                               unsigned long long *__restrict__ ovf) {
 #pragma clang fp contract(off)
 #pragma unroll 4
   for (uint32_t j = 0; j < cn; ++j) {
     if (DIAG && jbase + j <= il) continue;
-    const T dx = xi - sx[j];
-    const T dy = yi - sy[j];
-    const T dz = zi - sz[j];
-    T s = dx * dx + dy * dy;
+    const float dx = xi - sx[j];
+    const float dy = yi - sy[j];
+    const float dz = zi - sz[j];
+    float s = dx * dx + dy * dy;
     s = s + dz * dz;
-    const uint32_t k = bin_index<T>(s, bin, inv_bin, band, nhist);
+    const uint32_t k = bin_index_f32(s, inv_bin, nhist);
     if (__builtin_expect(k - B < wlim, 1)) {
       atomicAdd(&win[(k + D) & (WCAP - 1)], 1u);
     } else if (k < nhist) {
@@ -643,7 +616,7 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
     zi = A.z[gi];
   }
   const T bin = (T)td.bin;
-  const double inv_bin32 = 1.0 / (double)bin;  // for bin_index<float>
+  const double inv_bin32 = 1.0 / (double)bin;  // for bin_index_f32
   const float yb = recip_f32(bin);              // for quot_f32
   const uint32_t nhist = td.nhist;
   const double *bi = A.boxes + 6 * (size_t)tiI;
@@ -726,8 +699,8 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
       __syncthreads();
       if (ivalid) {
         if (diag) {
-          pair_block<T, WCAP, true>(xi, yi, zi, tid, sx, sy, sz, cn, s0, bin, inv_bin32, td.band,
-                                    nhist, B, wlim, D, win, hp, ovf);
+          pair_block_f32<WCAP, true>(xi, yi, zi, tid, sx, sy, sz, cn, s0, inv_bin32, nhist, B, wlim,
+                                     D, win, hp, ovf);
         } else {
           const uint32_t ng = cn & ~7u;
           if (safe)
@@ -736,8 +709,8 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
           else
             pair_group8_f32<WCAP, false, FQ>(xi, yi, zi, sx, sy, sz, ng, bin, inv_bin32, yb, nhist, B,
                                              wlim, D, off, win, hp, ovf);
-          pair_block<T, WCAP, false>(xi, yi, zi, tid, sx + ng, sy + ng, sz + ng, cn - ng, s0 + ng, bin,
-                                     inv_bin32, td.band, nhist, B, wlim, D, win, hp, ovf);
+          pair_block_f32<WCAP, false>(xi, yi, zi, tid, sx + ng, sy + ng, sz + ng, cn - ng, s0 + ng,
+                                      inv_bin32, nhist, B, wlim, D, win, hp, ovf);
         }
       }
       __syncthreads();
@@ -746,125 +719,21 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
   flush_window<WCAP>(win, B, min(B + (uint32_t)WCAP, nhist), D, hp);
 }
 
-// Loads through the constant address space: with a uniform address they
-// become scalar loads into SGPRs (the J records below), read-only data.
-typedef const double __attribute__((address_space(4))) cdouble;
-
-// FP64 groups of 4 J atoms against the thread's two I atoms a and b (8
-// independent chains; each J record serves two pairs).  The J records (x',
-// y', z', |r'|^2, relative to the centre of the J tile's box; rec) are read
-// with scalar loads: the address is the same for every lane, so they take
-// SGPRs and no LDS.  Counts of an I atom that does not exist (va / vb false)
-// are dropped.  The exact evaluation reads the coordinates again (xg, yg, zg
-// at ga, gb for the I atoms, jg + j for the J atoms).
-// NARROW: the fixed-point fast path (fix_bin; nhist <= kNarrowMax), k[] then
-// holding kFixHi + bin.
-template <int WCAP, bool SAFE, bool NARROW>
-__device__ __forceinline__ void pair_group4x2(const IAtom &ia, const IAtom &ib, bool va, bool vb,
-                                              const double *xg, const double *yg,
-                                              const double *zg, size_t ga, size_t gb, size_t jg,
-                                              const double *rec, uint32_t ng, double bin,
-                                              double inv_bin, double band, const FixBand &fb,
-                                              uint32_t nhist, uint32_t B, uint32_t wlim,
-                                              uint32_t D, uint32_t off, uint32_t *win,
-                                              unsigned long long *__restrict__ hp,
-                                              unsigned long long *__restrict__ ovf) {
-#pragma clang fp contract(off)
-  constexpr uint32_t kb = NARROW ? kFixHi : 0u;  // offset of k[] from the bin
-  // (opaque, so that the slot address stays one shift-add of k[])
-  uint32_t offk = off - kb;
-  asm volatile("" : "+v"(offk));
-  // SAFE: every lane increments for every pair, by 1 or, for an I atom that
-  // does not exist (a stand-in whose bins lie in the J tile's range), by 0
-  const uint32_t inca = va, incb = vb;
-  cdouble *jr = (cdouble *)rec;
-  for (uint32_t j0 = 0; j0 < ng; j0 += 4) {
-    uint32_t k[8];
-    bool bad[8], any = false;
-    uint32_t lo[8];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const double rx = jr[4 * (j0 + p)], ry = jr[4 * (j0 + p) + 1], rz = jr[4 * (j0 + p) + 2],
-                   rn = jr[4 * (j0 + p) + 3];
-      double s = ia.n + rn;
-      s = __builtin_fma(ia.az, rz, s);
-      s = __builtin_fma(ia.ay, ry, s);
-      s = __builtin_fma(ia.ax, rx, s);
-      double t = ib.n + rn;
-      t = __builtin_fma(ib.az, rz, t);
-      t = __builtin_fma(ib.ay, ry, t);
-      t = __builtin_fma(ib.ax, rx, t);
-      if constexpr (NARROW) {
-        k[p] = fix_bin(s, inv_bin, fb.m, lo[p]);
-        k[4 + p] = fix_bin(t, inv_bin, fb.m, lo[4 + p]);
-      } else {
-        k[p] = fast_bin(s, inv_bin, band, bad[p]);
-        k[4 + p] = fast_bin(t, inv_bin, band, bad[4 + p]);
-        any |= bad[p] | bad[4 + p];
-      }
-    }
-    if constexpr (NARROW) {
-      // one test of the smallest low word; then all 8 pairs take the exact
-      // path (its result equals the fast one wherever that one holds)
-      const uint32_t m = min(min(min(lo[0], lo[1]), min(lo[2], lo[3])),
-                             min(min(lo[4], lo[5]), min(lo[6], lo[7])));
-      any = m <= fb.lm1;
-#pragma unroll
-      for (int p = 0; p < 8; ++p) bad[p] = true;
-    }
-    if (__builtin_expect(any, 0)) {
-#pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        if (bad[p]) {
-          const size_t g = opaque_index(p < 4 ? ga : gb), h = jg + j0 + (p & 3);
-          const double dx = xg[g] - xg[h];
-          const double dy = yg[g] - yg[h];
-          const double dz = zg[g] - zg[h];
-          double s = dx * dx + dy * dy;
-          s = s + dz * dz;
-          k[p] = exact_bin<double>(s, bin, nhist) + kb;
-        }
-      }
-    }
-    if constexpr (SAFE) {
-      // slot k - kb + off, a window index (32-bit wrap-around)
-#pragma unroll
-      for (int p = 0; p < 8; ++p) atomicAdd(&win[k[p] + offk], p < 4 ? inca : incb);
-    } else {
-#pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        if (!(p < 4 ? va : vb)) continue;
-        const uint32_t kp = k[p] - kb;
-        if (kp - B < wlim)
-          atomicAdd(&win[(kp + D) & (WCAP - 1)], 1u);
-        else if (kp < nhist)
-          atomicAdd(&hp[kp], 1ull);
-        else
-          atomicAdd(ovf, 1ull);
-      }
-    }
-  }
-}
-
-// I atom relative to a centre c, for the fast path.
-__device__ __forceinline__ IAtom centred(double x, double y, double z, const double c[3]) {
-  const double u = x - c[0], v = y - c[1], w = z - c[2];
-  return IAtom{-2.0 * u, -2.0 * v, -2.0 * w, fma(w, w, fma(v, v, u * u))};
-}
-
 // Records of the FP64 kernel's J atoms: each atom relative to the centre c
-// of its tile's box (the centre tile_band takes), (x - c, y - c, z - c,
-// |r - c|^2), four doubles per atom in the sorted order.
+// of its tile's box (the centre tile_band takes) in units of 2 bins
+// (scale = 1/(2 bin)), (x', y', z', |r'|^2), four doubles per atom in the
+// sorted order.
 __global__ void hist_tile_records(const double *__restrict__ x, const double *__restrict__ y,
                                   const double *__restrict__ z, const Tile *__restrict__ tiles,
-                                  const double *__restrict__ boxes, double *__restrict__ rec) {
+                                  const double *__restrict__ boxes, double scale,
+                                  double *__restrict__ rec) {
   const Tile t = tiles[blockIdx.x];
   const double *b = boxes + 6 * (size_t)blockIdx.x;
   double c[3];
   for (int a = 0; a < 3; ++a) c[a] = 0.5 * (b[a] + b[3 + a]);
   for (uint32_t i = threadIdx.x; i < t.cnt; i += blockDim.x) {
     const size_t g = (size_t)t.off + i;
-    const double u = x[g] - c[0], v = y[g] - c[1], w = z[g] - c[2];
+    const double u = (x[g] - c[0]) * scale, v = (y[g] - c[1]) * scale, w = (z[g] - c[2]) * scale;
     double *r = rec + 4 * g;
     r[0] = u;
     r[1] = v;
@@ -874,38 +743,63 @@ __global__ void hist_tile_records(const double *__restrict__ x, const double *__
 }
 
 // FP64 binning: one work item = (pair type, I tile pair {2 ti, 2 ti + 1},
-// run of J tiles), two I atoms per thread (atom tid of each tile).  The J
+// run of J tiles), of each J tile the share blockIdx.y of gridDim.y.  The J
 // tiles are sorted and the window managed for the union box of the two I
-// tiles.  Distances are formed relative to the centre of each J tile's box:
-// the J records hold the J atoms relative to it (A.rec), and the I atoms are
-// taken relative to it once per J tile.  Like-element types visit tile pairs
-// by a half rotation over I tile pairs (add_items), so within the item's own
-// tile pair the J tile 2 ti pairs with I tile 2 ti only (j > i) and J tile
-// 2 ti + 1 with I tile 2 ti fully and with 2 ti + 1 for j > i; those two J
-// tiles take the per-pair loop.  No J atoms are staged in LDS, so the work
-// group synchronises only where the window moves.
-template <int WCAP, bool NARROW>
-__global__ __launch_bounds__(kTile) void hist_kernel_f64(Args<double> A) {
-  __shared__ uint32_t win[WCAP];
+// tiles.  Like-element types visit tile pairs by a half rotation over I tile
+// pairs (add_items), so within the item's own tile pair the J tile 2 ti pairs
+// with I tile 2 ti only (j > i) and J tile 2 ti + 1 with I tile 2 ti fully and
+// with 2 ti + 1 for j > i.
+//
+// Squared distances come from the FP64 matrix instruction, 16 I x 16 J atoms
+// at a time: with the atoms relative to the J tile's centre in units of 2 bins
+// (A.rec), s = |ri'|^2 + |rj'|^2 - 2 ri'.rj' is a product over K = 4, A row
+// (-2 x', -2 y', -2 z', |ri'|^2), B column (x', y', z', 1), accumulator
+// |rj'|^2.  It issues the same FP64 FMAs as the vector units (v_mfma_f64
+// 16x16x4 holds the port 64-70 cycles for 16 waves' worth of FMAs; the two do
+// not overlap), but one instruction feeds them from 12 registers, the add of
+// |ri'|^2 is gone, and J atoms come by vector loads: scalar loads shared their
+// wait counter with the LDS increments (issue filled 82% of the cycles).
+// A wave holds up to 4 blocks of 16 atoms of each I tile (blocks wave + 16 p)
+// and all waves walk the same J blocks, so their loads hit the L1 cache.
+// Each lane then has 4 pairs per product: row (lane >> 4) + 4 r, column
+// lane & 15.
+// Increments are issued before the fixed-point test of the bin: one running
+// minimum of the low words over a J block's 32 pairs per lane, and only when it
+// fails (a few J blocks in 10^4) is the block gone through again, the doubtful
+// pairs' increments taken back and made from the exact evaluation.  A row or
+// column without an atom (the last block of a tile) carries a squared distance
+// that puts its pairs into kTrash slots past the window, so that partial blocks
+// cost nothing.
+typedef double double4v __attribute__((ext_vector_type(4)));
+constexpr uint32_t kTrash = 4032;  // slots past the window
+
+// One of four values (by value: an indexed array would live in scratch memory).
+__device__ __forceinline__ double pick(uint32_t p, double a, double b, double c, double d) {
+  const double x = (p & 1) ? b : a, y = (p & 1) ? d : c;
+  return (p & 2) ? y : x;
+}
+
+template <int WCAP>
+__global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) void hist_kernel_f64(
+    Args<double> A) {
+#pragma clang fp contract(off)
+  __shared__ uint32_t win[WCAP + kTrash];
   __shared__ unsigned long long keys[kSortCap];
 
   const Item it = A.items[blockIdx.x];
   const TypeDesc td = A.types[it.type];
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, col = lane & 15u, kc = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t tA = 2 * it.ti, tB = tA + 1;
   const bool hasB = tB < td.a_n;
   const Tile IA = A.tiles[td.a_base + tA];
   const Tile IB = hasB ? A.tiles[td.a_base + tB] : Tile{0u, 0u};
   if (IA.cnt == 0) return;
-  const bool va = tid < IA.cnt, vb = tid < IB.cnt;
-  // an I atom that does not exist stands in as the first atom of tile tA:
-  // its counts are dropped, and its bins lie inside every J tile's range
-  const size_t ga = (size_t)IA.off + (va ? tid : 0u);
-  const size_t gb = vb ? (size_t)IB.off + tid : (size_t)IA.off;
-  const double xa = A.x[ga], ya = A.y[ga], za = A.z[ga];
-  const double xb = A.x[gb], yb = A.y[gb], zb = A.z[gb];
   const uint32_t nhist = td.nhist;
   const double bin = td.bin;
+  // I blocks of this wave: 16 atoms each, blocks wave + 16 p of both tiles
+  const uint32_t nbI = (max(IA.cnt, IB.cnt) + 15) / 16;
+  const uint32_t np = nbI > wave ? (nbI - wave + 15) / 16 : 0u;
   // union box of the two I tiles
   double bu[6];
   {
@@ -955,8 +849,8 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f64(Args<double> A) {
     }
   }
 
+  // The window holds bins [B, B + WCAP), bin k in slot k - B.
   uint32_t B = (uint32_t)(keys[0] >> 32);
-  uint32_t D = 0u;  // bin k is counted in slot (k + D) mod WCAP
   for (uint32_t s = 0; s < n; ++s) {
     const uint32_t m = (uint32_t)(keys[s] & 0xffffffffu);
     const uint32_t tj = (it.jstart + m) % td.b_n;
@@ -968,81 +862,209 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f64(Args<double> A) {
     uint32_t wlim = 0;
     const bool span_ok = ku - kl + 1 <= (uint32_t)WCAP;
     if (span_ok) {
-      const uint32_t nb = ku + 1 > (uint32_t)WCAP ? ku + 1 - WCAP : 0u;
-      if (nb > B) {
+      if (ku - B >= (uint32_t)WCAP) {
+        // no later tile reaches below kl (they are sorted by it): the window
+        // moves up to there at once, so it moves rarely, and the waves meet
+        // only here and not at every tile
         __syncthreads();
-        flush_window<WCAP>(win, B, min(min(nb, B + (uint32_t)WCAP), nhist), D, hp);
-        B = nb;
-        __syncthreads();
+        flush_window<WCAP>(win, B, min(min(kl, B + (uint32_t)WCAP), nhist), 0u - B, hp);
+        rotate_window<WCAP>(win, kl, 0u - B);
+        B = kl;
       }
       wlim = min((uint32_t)WCAP, nhist - B);
     }
-    const bool safe = span_ok && fits;
-    uint32_t off = 0u;
-    if (safe) {
-      if (((kl + D) ^ (ku + D)) >= (uint32_t)WCAP) {
-        rotate_window<WCAP>(win, B, D);
-        D = 0u - B;
-      }
-      off = D - ((kl + D) & ~(uint32_t)(WCAP - 1));
-    }
     const Tile J = A.tiles[tjg];
-    const double *jx = A.x + J.off, *jy = A.y + J.off, *jz = A.z + J.off;
-    // like-element types: J tiles of the item's own tile pair.  The I
-    // coordinates are read again where the per-pair loop needs them, so that
-    // they take no registers in the grouped loop.
+    // like-element types: J tiles of the item's own tile pair
     const bool jA = td.same && tj == tA, jB = td.same && hasB && tj == tB;
-    if (jA) {
-      const size_t g = opaque_index(ga);
-      if (va)
-        pair_block<double, WCAP, true>(A.x[g], A.y[g], A.z[g], tid, jx, jy, jz, J.cnt, 0u, bin,
-                                       td.inv_bin, td.band, nhist, B, wlim, D, win, hp, ovf);
-    } else if (jB) {
-      const size_t g = opaque_index(ga), h = opaque_index(gb);
-      if (va)
-        pair_block<double, WCAP, false>(A.x[g], A.y[g], A.z[g], tid, jx, jy, jz, J.cnt, 0u, bin,
-                                        td.inv_bin, td.band, nhist, B, wlim, D, win, hp, ovf);
-      if (vb)
-        pair_block<double, WCAP, true>(A.x[h], A.y[h], A.z[h], tid, jx, jy, jz, J.cnt, 0u, bin,
-                                       td.inv_bin, td.band, nhist, B, wlim, D, win, hp, ovf);
-    } else {
-      double c[3];
-      const double band = tile_band(bj, td.band, td.inv_bin, nhist, c);
-      const FixBand fb = fix_band(band);
-      const IAtom ia = centred(xa, ya, za, c), ib = centred(xb, yb, zb, c);
-      const uint32_t ng = J.cnt & ~3u;
-      // chunks of kChunk J atoms with a barrier between them: the work
-      // group's waves read the same records, which the scalar cache then
-      // serves once rather than once per wave
-      for (uint32_t c0 = 0; c0 < ng; c0 += kChunk) {
-        const uint32_t cn = min((uint32_t)kChunk, ng - c0);
-        const size_t jg = (size_t)J.off + c0;
-        const double *rec = A.rec + 4 * jg;
-        if (va || vb) {
-          if (safe)
-            pair_group4x2<WCAP, true, NARROW>(ia, ib, va, vb, A.x, A.y, A.z, ga, gb, jg, rec, cn,
-                                              bin, td.inv_bin, band, fb, nhist, B, wlim, D, off,
-                                              win, hp, ovf);
-          else
-            pair_group4x2<WCAP, false, NARROW>(ia, ib, va, vb, A.x, A.y, A.z, ga, gb, jg, rec, cn,
-                                               bin, td.inv_bin, band, fb, nhist, B, wlim, D, off,
-                                               win, hp, ovf);
-        }
-        if (c0 + kChunk < ng) __syncthreads();
+    const uint32_t njb = (J.cnt + 15) / 16;
+    const uint32_t jb0 = (uint32_t)((uint64_t)njb * blockIdx.y / gridDim.y);
+    const uint32_t jb1 = (uint32_t)((uint64_t)njb * (blockIdx.y + 1) / gridDim.y);
+    if (np == 0 || jb0 == jb1) continue;
+    double c[3], R;
+    const double band = tile_band(bj, td.band, td.inv_bin, nhist, (double)kl, c, R);
+    // pairs without an atom: 16.3 bins past the window for the columns, up to
+    // R^2 / (2 * that) more for the rows
+    const double far = (double)(WCAP + 16) + 0.3 + (double)B;
+    const double q0 = 0.25 * far * far;
+    const bool safe = span_ok && fits && sqrt(far * far + R * R) - (double)B < WCAP + kTrash - 2.0;
+    // A operands: component kc of atom col of each block (p < 4 in tile A, the
+    // rest in tile B), or the squared norm (kc = 3).  The coordinates are read
+    // for every J tile, so that they take no registers in between.
+    double a[8];
+    {
+      const double *comp = kc == 0 ? A.x : kc == 1 ? A.y : A.z;
+      const double ck = kc == 0 ? c[0] : kc == 1 ? c[1] : c[2];
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        const Tile T = p < 4 ? IA : IB;
+        const uint32_t i = (wave + 16 * (p & 3)) * 16 + col;
+        const bool ok = i < T.cnt;
+        const size_t g = opaque_index((size_t)T.off + (ok ? i : 0u));
+        const double u = kc < 3 && ok ? (comp[g] - ck) * A.scale : 0.0;
+        double q = u * u;
+        q += __shfl_xor(q, 16, 64);
+        q += __shfl_xor(q, 32, 64);
+        a[p] = kc < 3 ? -2.0 * u : ok ? q : q0;
       }
-      const size_t g = opaque_index(ga), h = opaque_index(gb);
-      if (va)
-        pair_block<double, WCAP, false>(A.x[g], A.y[g], A.z[g], tid, jx + ng, jy + ng, jz + ng,
-                                        J.cnt - ng, ng, bin, td.inv_bin, td.band, nhist, B, wlim,
-                                        D, win, hp, ovf);
-      if (vb)
-        pair_block<double, WCAP, false>(A.x[h], A.y[h], A.z[h], tid, jx + ng, jy + ng, jz + ng,
-                                        J.cnt - ng, ng, bin, td.inv_bin, td.band, nhist, B, wlim,
-                                        D, win, hp, ovf);
     }
-    __syncthreads();
+    const double *rec = A.rec + 4 * (size_t)J.off;
+    // Pair i of a J block's 32 (8 p + 4 (tile B) + r) of this lane
+    auto valid = [&](uint32_t jb, uint32_t p, uint32_t i) {
+      const uint32_t blk = wave + 16 * p, row = blk * 16 + kc + 4 * (i & 3), j = jb * 16 + col;
+      const bool b = (i & 4) != 0;
+      // a tile against itself takes j > i, tile B's own J tile tile A whole
+      return j < J.cnt && row < (b ? IB.cnt : IA.cnt) && !(b && jA) &&
+             !((b ? jB : jA) && j <= row);
+    };
+    auto exact = [&](uint32_t jb, uint32_t p, uint32_t i) {
+      const size_t g = (size_t)((i & 4) ? IB.off : IA.off) + (wave + 16 * p) * 16 + kc + 4 * (i & 3);
+      const size_t h = (size_t)J.off + jb * 16 + col;
+      const double dx = A.x[g] - A.x[h];
+      const double dy = A.y[g] - A.y[h];
+      const double dz = A.z[g] - A.z[h];
+      double q = dx * dx + dy * dy;
+      q = q + dz * dz;
+      return exact_bin(q, bin, nhist);
+    };
+    if (safe) {
+      const FixSlot fs = fix_slot(band, (int32_t)(0u - B));
+      constexpr uint32_t kMask = (WCAP > 16384 ? 65536 : 16384) * 4 - 4;
+      static_assert(WCAP + kTrash <= kMask / 4 + 1, "slots");
+      auto add = [&](uint32_t at, uint32_t v) {
+        atomicAdd(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(win) + at), v);
+      };
+      double bv, nj;
+      {
+        const uint32_t j = min(jb0 * 16 + col, J.cnt - 1);
+        bv = rec[4 * j + kc];
+        nj = rec[4 * j + 3];
+      }
+      for (uint32_t jb = jb0; jb < jb1; ++jb) {
+        const bool jok = jb * 16 + col < J.cnt;
+        const double b = jok ? (kc < 3 ? bv : 1.0) : 0.0;
+        const double cj = jok ? nj : q0;
+        const double4v C = {cj, cj, cj, cj};
+        if (jb + 1 < jb1) {
+          const uint32_t j = min((jb + 1) * 16 + col, J.cnt - 1);
+          bv = rec[4 * j + kc];
+          nj = rec[4 * j + 3];
+        }
+        uint32_t low = 0xffffffffu;
+        // I blocks p of both tiles against the J block: two products, 8 pairs
+        auto two = [&](int p) {
+          const double4v d0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[p], b, C, 0, 0, 0);
+          const double4v d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[4 + p], b, C, 0, 0, 0);
+          uint32_t k[8], lo[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const double q = i < 4 ? d0[i & 3] : d1[i & 3];
+            k[i] = fix_slot_from_rsq(q, __builtin_amdgcn_rsq(q), fs.m, lo[i]) & kMask;
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) add(k[i], 1u);
+#pragma unroll
+          for (int i = 0; i < 8; i += 2) low = min(min(lo[i], lo[i + 1]), low);
+        };
+        if (!jA && !jB) {
+          if (np == 4) {
+            two(0);
+            two(1);
+            two(2);
+            two(3);
+          } else {
+            two(0);
+            if (np > 1) two(1);
+            if (np > 2) two(2);
+          }
+        } else {
+          // the item's own tiles: one product at a time, those below the
+          // diagonal left out
+#pragma unroll
+          for (int p = 0; p < 8; ++p) {
+            const uint32_t blk = wave + 16 * (p & 3);
+            if ((uint32_t)(p & 3) >= np || (p < 4 ? jA && jb < blk : jA || jb < blk)) continue;
+            const bool diag = (p < 4 ? jA : jB) && jb == blk;
+            const double4v d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[p], b, C, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              uint32_t l;
+              const uint32_t k = fix_slot_from_rsq(d[r], __builtin_amdgcn_rsq(d[r]), fs.m, l) & kMask;
+              const bool use = !diag || col > kc + 4 * r;
+              // (an atom with itself has a doubtful bin, which is not counted)
+              low = min(low, use ? l : 0xffffffffu);
+              add(use ? k : (uint32_t)WCAP * 4, 1u);
+            }
+          }
+        }
+        if (__builtin_expect(__ballot(low <= fs.lm1) != 0, 0)) {
+          uint32_t bits = 0;
+#pragma unroll 1
+          for (uint32_t p = 0; p < np; ++p) {
+            const double4v d0 = __builtin_amdgcn_mfma_f64_16x16x4f64(pick(p, a[0], a[1], a[2], a[3]), b, C, 0, 0, 0);
+            const double4v d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(pick(p, a[4], a[5], a[6], a[7]), b, C, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const double q = i < 4 ? d0[i & 3] : d1[i & 3];
+              uint32_t l;
+              const uint32_t k = fix_slot_from_rsq(q, __builtin_amdgcn_rsq(q), fs.m, l) & kMask;
+              if (l <= fs.lm1 && valid(jb, p, i)) {
+                add(k, 0xffffffffu);
+                bits |= 1u << (8 * p + i);
+              }
+            }
+          }
+          while (__ballot(bits != 0) != 0) {
+            if (bits) {
+              const uint32_t i = __builtin_ctz(bits);
+              bits &= bits - 1;
+              add(((exact(jb, i >> 3, i & 7) - B) & (WCAP - 1)) << 2, 1u);
+            }
+          }
+        }
+      }
+    } else {
+      // tile pairs that reach past nhist, or wider than the window: every pair
+      // is tested for where its count belongs
+      const FixBand fb = fix_band(band);
+      const bool narrow = nhist <= kNarrowMax;
+      for (uint32_t jb = jb0; jb < jb1; ++jb) {
+        const uint32_t j = min(jb * 16 + col, J.cnt - 1);
+        const double b = kc < 3 ? rec[4 * j + kc] : 1.0, nj = rec[4 * j + 3];
+        const double4v C = {nj, nj, nj, nj};
+#pragma unroll 1
+        for (uint32_t p = 0; p < np; ++p) {
+          const double4v d0 = __builtin_amdgcn_mfma_f64_16x16x4f64(pick(p, a[0], a[1], a[2], a[3]), b, C, 0, 0, 0);
+          const double4v d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(pick(p, a[4], a[5], a[6], a[7]), b, C, 0, 0, 0);
+#pragma unroll 1
+          for (uint32_t i = 0; i < 8; ++i) {
+            const uint32_t r = i & 3;
+            const double qa = pick(r, d0[0], d0[1], d0[2], d0[3]);
+            const double qb = pick(r, d1[0], d1[1], d1[2], d1[3]);
+            const double q = i < 4 ? qa : qb;
+            if (!valid(jb, p, i)) continue;
+            uint32_t k;
+            bool bad;
+            if (narrow) {
+              uint32_t l;
+              k = fix_from_rsq(q, __builtin_amdgcn_rsq(q), 2.0, fb.m, l) - kFixHi;
+              bad = l <= fb.lm1;
+            } else {
+              k = fast_bin(q, 2.0, band, bad);
+            }
+            if (__builtin_expect(bad, 0)) k = exact(jb, p, i);
+            if (k - B < wlim)
+              atomicAdd(&win[k - B], 1u);
+            else if (k < nhist)
+              atomicAdd(&hp[k], 1ull);
+            else
+              atomicAdd(ovf, 1ull);
+          }
+        }
+      }
+    }
   }
-  flush_window<WCAP>(win, B, min(B + (uint32_t)WCAP, nhist), D, hp);
+  __syncthreads();
+  flush_window<WCAP>(win, B, min(B + (uint32_t)WCAP, nhist), 0u - B, hp);
 }
 
 // ---------------------------------------------------------------- host planning
@@ -1250,32 +1272,53 @@ static void sort_structure_host(const T *xyz, size_t n, const unsigned *el_count
 // J records of the FP64 kernel (no-op for FP32 binning).
 template <class T>
 static void launch_records(hipStream_t st, const T *x, const T *y, const T *z, const Tile *tiles,
-                           const double *boxes, size_t ntiles, double *rec) {
+                           const double *boxes, size_t ntiles, double bin, double *rec) {
   if constexpr (sizeof(T) == 8) {
     if (ntiles)
       hipLaunchKernelGGL(hist_tile_records, dim3((unsigned)ntiles), dim3(256), 0, st, x, y, z,
-                         tiles, boxes, rec);
+                         tiles, boxes, 0.5 / bin, rec);
   }
 }
 
+// Shares that the J tiles of every FP64 item are cut into (hist_kernel_f64's
+// grid.y), so that a small structure's few items fill the chip: an item of
+// 2,048 x 1,024 pairs keeps one CU busy for 0.2 ms (16.6 cycles per 64 pairs),
+// while a work group costs some 4 or 20 us more than its pairs (window cleared
+// and flushed, J tiles sorted).  The estimate is rounds x work group time, half
+// a work group for the uneven end.  Measured with 1, 2, 4, 8, 16, 32 shares:
+// 2,000 atoms (2 items) 205, 130, 85, 59, 47, 40 us; 8,000 atoms (20 items)
+// 248, 143, 91, 59, 76, 92; 22,000 atoms (156 items) 235, 231, 217, 237, 319,
+// 584; 60,000 atoms (930 items) 880, 913, 944, 1,069, 1,343, 1,883.
+static unsigned item_shares(size_t nitems, double pairs, uint32_t wcap, int cus) {
+  const double w = pairs / (double)nitems / 64.0 * 16.6 / 2400.0;  // us
+  const double fixed = wcap > 8192 ? 20.0 : 4.0;
+  unsigned best = 1;
+  double bt = INFINITY;
+  for (unsigned s = 1; s <= 32; s *= 2) {
+    const double rounds = std::ceil((double)nitems * s / cus);
+    const double t = (rounds + 0.5) * (w / s + fixed);
+    if (t < bt) {
+      bt = t;
+      best = s;
+    }
+  }
+  return best;
+}
+
 template <class T>
-static int launch_hist(xs_ctx *ctx, const Args<T> &A, size_t nitems, uint32_t wcap, bool prof) {
+static int launch_hist(xs_ctx *ctx, const Args<T> &A, size_t nitems, double pairs, uint32_t wcap,
+                       bool prof) {
   if (!nitems) return XS_OK;
   hipEvent_t ev = nullptr;
   if (prof) XS_TRY(prof_begin(ctx, "hist", &ev));
-  const dim3 grid((unsigned)nitems), block(kTile);
+  dim3 grid((unsigned)nitems);
+  const dim3 block(kTile);
   if constexpr (sizeof(T) == 8) {
-    if (wcap == 8192) {
-      if (A.narrow)
-        hipLaunchKernelGGL((hist_kernel_f64<8192, true>), grid, block, 0, ctx->stream, A);
-      else
-        hipLaunchKernelGGL((hist_kernel_f64<8192, false>), grid, block, 0, ctx->stream, A);
-    } else {
-      if (A.narrow)
-        hipLaunchKernelGGL((hist_kernel_f64<32768, true>), grid, block, 0, ctx->stream, A);
-      else
-        hipLaunchKernelGGL((hist_kernel_f64<32768, false>), grid, block, 0, ctx->stream, A);
-    }
+    grid.y = item_shares(nitems, pairs, wcap, ctx->cu_count);
+    if (wcap == 8192)
+      hipLaunchKernelGGL((hist_kernel_f64<8192>), grid, block, 0, ctx->stream, A);
+    else
+      hipLaunchKernelGGL((hist_kernel_f64<32768>), grid, block, 0, ctx->stream, A);
   } else {
     if (wcap == 8192) {
       if (A.quot_f32)
@@ -1528,6 +1571,14 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
   add_types(n_el, ebase, en, nhist, bin, 0ull, 0u, types);
   std::vector<Item> items;
   add_items(types, 0, (uint32_t)types.size(), items, sizeof(T) == 8, kSingleSplit);
+  if (sizeof(T) == 8 && items.size() < 8192) {
+    // fewer, longer items: each flushes its window once, with one atomic per
+    // bin it touched, and launch_hist shares them out again where they are few
+    // (62,000 atoms, 47,000 bins: 1.19 -> 1.13 ms; 980,219 atoms, 30,380
+    // items: 197 ms, 201 with half as many)
+    items.clear();
+    add_items(types, 0, (uint32_t)types.size(), items, true, kSingleSplit / 2);
+  }
   order_items(items, types, tiles, sizeof(T) == 8);
 
   // 4. tables (exact sizes) in the table buffer; the stream is idle here
@@ -1556,7 +1607,7 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
   if (!tiles.empty())
     hipLaunchKernelGGL((hist_tile_boxes<T>), dim3((unsigned)tiles.size()), dim3(256), 0, ctx->stream,
                        sxp, syp, szp, tiles_d, boxes);
-  launch_records<T>(ctx->stream, sxp, syp, szp, tiles_d, boxes, tiles.size(), rec);
+  launch_records<T>(ctx->stream, sxp, syp, szp, tiles_d, boxes, tiles.size(), bin, rec);
   XS_HIP_CHECK(hipGetLastError());
   if (equal_count && std::isfinite(cap) && !tiles.empty()) {
     // equal-count tiles of a structure far from uniform density can be wider
@@ -1576,8 +1627,8 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
   XS_TRY(prof_end(ctx, "hist_prep", ev));
   Args<T> A{sxp, syp, szp, tiles_d, boxes, types_d, items_d, hist_d, ovf_d, rec};
   A.quot_f32 = quot;
-  A.narrow = nhist <= kNarrowMax;
-  return launch_hist<T>(ctx, A, items.size(), wcap, true);
+  A.scale = 0.5 / bin;
+  return launch_hist<T>(ctx, A, items.size(), 0.5 * (double)n * (double)n, wcap, true);
 }
 
 // Host coordinates: one synchronous copy to the device (a buffer of the
@@ -1645,6 +1696,12 @@ static int plan_finish(xs_ctx *ctx, xs_batch *b, const std::vector<Tile> &tiles,
   order_items(large, types, tiles, sizeof(T) == 8);
   b->items8192 = small.size();
   b->items32768 = large.size();
+  for (const TypeDesc &d : types) {
+    double na = 0.0, nb = 0.0;
+    for (uint32_t t = 0; t < d.a_n; ++t) na += tiles[d.a_base + t].cnt;
+    for (uint32_t t = 0; t < d.b_n; ++t) nb += tiles[d.b_base + t].cnt;
+    (d.nhist <= 8192 ? b->pairs8192 : b->pairs32768) += na * nb * (d.same ? 0.5 : 1.0);
+  }
   small.insert(small.end(), large.begin(), large.end());
   const size_t nc = b->natoms;
   const bool ok =
@@ -1674,7 +1731,7 @@ static int plan_finish(xs_ctx *ctx, xs_batch *b, const std::vector<Tile> &tiles,
     e = hipMemcpy(b->items, small.data(), small.size() * sizeof(Item), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     launch_records<T>(ctx->stream, c, c + nc, c + 2 * nc, static_cast<const Tile *>(b->tiles),
-                      static_cast<const double *>(b->boxes), tiles.size(),
+                      static_cast<const double *>(b->boxes), tiles.size(), b->bin,
                       static_cast<double *>(b->recs));
     e = hipGetLastError();
   }
@@ -2279,10 +2336,10 @@ static int plan_hist(xs_batch *b, unsigned long long *hist_d, bool prof) {
             b->ovf,
             static_cast<const double *>(b->recs)};
   A.quot_f32 = b->quot_f32;
-  A.narrow = std::all_of(b->nhist.begin(), b->nhist.end(), [](unsigned h) { return h <= kNarrowMax; });
-  XS_TRY(launch_hist<T>(ctx, A, b->items8192, 8192, prof));
+  A.scale = 0.5 / b->bin;
+  XS_TRY(launch_hist<T>(ctx, A, b->items8192, b->pairs8192, 8192, prof));
   A.items = items + b->items8192;
-  XS_TRY(launch_hist<T>(ctx, A, b->items32768, 32768, prof));
+  XS_TRY(launch_hist<T>(ctx, A, b->items32768, b->pairs32768, 32768, prof));
   return XS_OK;
 }
 

@@ -117,9 +117,9 @@ int xs_hist(xs_ctx *ctx, const void *xyz, size_t n_atoms,
             uint64_t *hist, uint64_t *overflow, unsigned flags);
 
 /* H3: histogram pair sums S[p*nq+iq] = sum_k h_p[k] sin(q r_k)/(q r_k + 1e-8),
- * r_k = (k+1/2) bin, empty bins skipped, S = 0 where q = 0.  FP64 terms,
- * sin advanced from bin to bin by Reinsch's form of the three-term
- * recurrence, FP64 atomics across blocks.
+ * r_k = (k+1/2) bin, S = 0 where q = 0.  FP64: groups of bins act through 64
+ * Chebyshev nodes each, to FP64 rounding (every bin by itself where they are
+ * wider than ~0.6 / max |q|); the sums over the nodes are matrix products.
  * Replaces the bin loop of calcInt1DHist (CalcFunctions.cpp:844-871) and
  * calcIntHistKernelXray/Neutron (CalcFunctionsCUDA.cu:923-985).
  * XS_PAIRSUM_MFMA evaluates the same sums as one product S = H A^T on the

@@ -6,7 +6,7 @@
 // sorted coordinates, tiles and work items of all structures on the device,
 // so a run is a fixed sequence of launches with no host work:
 //   zero fills -> histogram kernels (8192- then 32768-bin windows)
-//   -> zero fill + pair-sum kernel over all (pair type, 2048-bin chunk)
+//   -> pair sums of all pair types over Chebyshev nodes
 //   -> PDF kernel over all structures' bins.
 // With XS_BATCH_GRAPH the sequence is captured once into a hipGraph on the
 // context's stream and replayed while the output pointers, nq, the PDF type
@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "xs_internal.h"
+#include "xs_nodesum.h"
 
 namespace xs {
 
@@ -31,12 +32,12 @@ void release_batch_run(BatchRunState &r) {
 namespace {
 
 struct RunLayout {
-  size_t chunks, pdfdesc, q, hist, S, pdf, mm_cols, mm_tiles, mm_a, mm_b, total;
+  size_t rows, nmax, nodes, pdfdesc, q, hist, S, pdf, mm_cols, mm_tiles, mm_a, mm_b, total;
 };
 
 // Byte offsets inside the run buffer; host-mode staging only when needed;
 // the matrix-core tables and slices when mm (a plan with mm.nq != 0) is given.
-RunLayout layout(const xs_batch *b, size_t nchunks, unsigned nq, bool host, bool want_S,
+RunLayout layout(const xs_batch *b, unsigned nhist_max, unsigned nq, bool host, bool want_S,
                  bool want_pdf, const MfmaBatchPlan *mm) {
   RunLayout L{};
   size_t off = 0;
@@ -46,7 +47,9 @@ RunLayout layout(const xs_batch *b, size_t nchunks, unsigned nq, bool host, bool
     off += bytes;
     return at;
   };
-  L.chunks = take(std::max<size_t>(nchunks, 1) * sizeof(PairsumChunk));
+  const size_t ntiles = (b->ntypes_total + nodesum::kRows - 1) / nodesum::kRows;
+  L.rows = take(ntiles * nodesum::kRows * sizeof(nodesum::Row));
+  L.nmax = take(ntiles * 4);
   L.pdfdesc = take((size_t)b->nstruct * sizeof(PdfDesc));
   L.q = take(host && want_S ? (size_t)nq * 8 : 0);
   L.hist = take(host ? b->hist_len * 8 : 0);
@@ -56,17 +59,22 @@ RunLayout layout(const xs_batch *b, size_t nchunks, unsigned nq, bool host, bool
   L.mm_tiles = take(mm ? mm->tiles.size() * sizeof(MfmaTile) : 0);
   L.mm_a = take(mm ? mm->a_bytes : 0);
   L.mm_b = take(mm ? mm->b_bytes : 0);
+  // (last: its size depends on the call, and rows and pdfdesc stay where they are)
+  L.nodes = take(want_S && !mm ? nodesum::layout((unsigned)ntiles, nhist_max, nodesum::kBudget).total : 0);
   L.total = align_up(off, 256);
   return L;
 }
 
-std::vector<PairsumChunk> make_chunks(const xs_batch *b) {
-  std::vector<PairsumChunk> c;
+// Pair types, most bins first, padded to whole tiles of 16.
+std::vector<nodesum::Row> make_rows(const xs_batch *b) {
+  std::vector<nodesum::Row> r(b->ntypes_total);
   for (size_t t = 0; t < b->ntypes_total; ++t)
-    for (uint32_t k0 = 0; k0 < b->type_nhist[t]; k0 += kPairsumChunk)
-      c.push_back(PairsumChunk{b->type_hist_off[t] + k0, (uint32_t)t, k0,
-                               std::min<uint32_t>(kPairsumChunk, b->type_nhist[t] - k0), 0u});
-  return c;
+    r[t] = nodesum::Row{b->type_hist_off[t], b->type_nhist[t], (uint32_t)t};
+  std::stable_sort(r.begin(), r.end(), [](const nodesum::Row &x, const nodesum::Row &y) {
+    return x.nhist > y.nhist;
+  });
+  r.resize(align_up(r.size(), nodesum::kRows), nodesum::Row{0ull, 0u, 0u});
+  return r;
 }
 
 std::vector<PdfDesc> make_pdf_desc(const xs_batch *b, const double *rho0, const double *sl,
@@ -114,7 +122,7 @@ std::vector<unsigned long long> pair_counts(const xs_batch *b) {
   return c;
 }
 
-int launch_all(xs_batch *b, const RunPtrs &P, const RunLayout &L, size_t nchunks, unsigned nq,
+int launch_all(xs_batch *b, const RunPtrs &P, const RunLayout &L, unsigned nhist_max, unsigned nq,
                int pdf_type, unsigned pdf_blocks, bool cpu_radius, bool mfma, bool prof) {
   char *buf = static_cast<char *>(b->run.buf);
   XS_TRY(batch_hist_launch(b, P.hist, prof));
@@ -122,9 +130,17 @@ int launch_all(xs_batch *b, const RunPtrs &P, const RunLayout &L, size_t nchunks
     XS_TRY(pairsum_mfma_batch(b->ctx, b->run.mm, P.hist, reinterpret_cast<const MfmaCol *>(buf + L.mm_cols),
                               reinterpret_cast<const MfmaTile *>(buf + L.mm_tiles), buf + L.mm_a,
                               buf + L.mm_b, b->bin, P.q, nq, P.S, prof));
-  else if (P.S)
-    XS_TRY(batch_pairsum_launch(b->ctx, P.hist, reinterpret_cast<const PairsumChunk *>(buf + L.chunks),
-                                nchunks, b->ntypes_total, b->bin, P.q, nq, P.S, prof));
+  else if (P.S) {
+    hipEvent_t ev = nullptr;
+    if (prof) XS_TRY(prof_begin(b->ctx, "batch_pairsum", &ev));
+    const unsigned nrows = (unsigned)b->ntypes_total;
+    const nodesum::Tables T{nodesum::layout((nrows + nodesum::kRows - 1) / nodesum::kRows, nhist_max,
+                                            nodesum::kBudget),
+                            buf + L.nodes, 0, 0, reinterpret_cast<const nodesum::Row *>(buf + L.rows),
+                            reinterpret_cast<const uint32_t *>(buf + L.nmax)};
+    XS_TRY(nodesum::run(b->ctx, T, P.hist, nrows, b->bin, P.q, nq, P.S));
+    if (prof) XS_TRY(prof_end(b->ctx, "batch_pairsum", ev));
+  }
   if (P.pdf)
     XS_TRY(batch_pdf_launch(b->ctx, P.hist, reinterpret_cast<const PdfDesc *>(buf + L.pdfdesc),
                             b->nstruct, pdf_blocks, pdf_type, cpu_radius, b->bin, P.pdf, prof));
@@ -168,11 +184,11 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
                                 "matrix-core path; run without XS_PAIRSUM_MFMA");
     R.mm_uploaded = false;
   }
-  const std::vector<PairsumChunk> chunks = make_chunks(plan);
+  const std::vector<nodesum::Row> rows = make_rows(plan);
   unsigned pdf_blocks = 0;
   const std::vector<PdfDesc> desc = make_pdf_desc(plan, want_pdf ? rho0 : nullptr, want_pdf ? sl : nullptr,
                                                   &pdf_blocks);
-  const RunLayout L = layout(plan, chunks.size(), nq, !device, want_S, want_pdf, mfma ? &R.mm : nullptr);
+  const RunLayout L = layout(plan, rows[0].nhist, nq, !device, want_S, want_pdf, mfma ? &R.mm : nullptr);
 
   // (re)allocate the run buffer and upload the descriptors when they change
   bool fresh = false;
@@ -202,9 +218,11 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
   const bool desc_changed = fresh || key_rho0 != R.key_rho0 || key_sl != R.key_sl;
   if (fresh || desc_changed) {
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    if (!chunks.empty())
-      XS_HIP_CHECK(hipMemcpy(buf + L.chunks, chunks.data(), chunks.size() * sizeof(PairsumChunk),
-                             hipMemcpyHostToDevice));
+    std::vector<uint32_t> nmax;
+    for (size_t i = 0; i < rows.size(); i += nodesum::kRows) nmax.push_back(rows[i].nhist);
+    XS_HIP_CHECK(hipMemcpy(buf + L.rows, rows.data(), rows.size() * sizeof(nodesum::Row),
+                           hipMemcpyHostToDevice));
+    XS_HIP_CHECK(hipMemcpy(buf + L.nmax, nmax.data(), nmax.size() * 4, hipMemcpyHostToDevice));
     XS_HIP_CHECK(hipMemcpy(buf + L.pdfdesc, desc.data(), desc.size() * sizeof(PdfDesc),
                            hipMemcpyHostToDevice));
     R.key_rho0 = key_rho0;
@@ -237,7 +255,7 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
   const bool cpu_radius = flags & XS_PDF_CPU_RADIUS;
 
   if (!graph) {
-    XS_TRY(launch_all(plan, P, L, chunks.size(), nq, pdf_type, pdf_blocks, cpu_radius, mfma, true));
+    XS_TRY(launch_all(plan, P, L, rows[0].nhist, nq, pdf_type, pdf_blocks, cpu_radius, mfma, true));
   } else {
     const unsigned kflags = flags & (XS_DEVICE_PTRS | XS_PDF_CPU_RADIUS | (mfma ? XS_PAIRSUM_MFMA : 0u));
     const bool same = R.exec && R.key_hist == P.hist && R.key_S == P.S && R.key_pdf == P.pdf &&
@@ -251,7 +269,7 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
       R.graph = nullptr;
       XS_HIP_CHECK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
       const int rc =
-          launch_all(plan, P, L, chunks.size(), nq, pdf_type, pdf_blocks, cpu_radius, mfma, false);
+          launch_all(plan, P, L, rows[0].nhist, nq, pdf_type, pdf_blocks, cpu_radius, mfma, false);
       hipGraph_t g = nullptr;
       const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
       if (rc != XS_OK || ec != hipSuccess) {

@@ -234,18 +234,6 @@ struct SortedPoints {
 int grid_sort(xs_ctx *ctx, const double *x, const double *y, const double *z, size_t n,
               double min_cell, SortedPoints &out);
 
-// Pair sums of many histograms: one chunk = up to 2048 bins of one pair type.
-struct PairsumChunk {
-  unsigned long long hist_off;  // first bin of the chunk in the histogram array
-  uint32_t type;                // row of S (S[type * nq + iq])
-  uint32_t k0, kn, pad;         // bin index of the chunk start within its histogram, length
-};
-constexpr unsigned kPairsumChunk = 2048;
-// S[ntypes * nq] is zeroed and accumulated.
-int batch_pairsum_launch(xs_ctx *ctx, const unsigned long long *hist, const PairsumChunk *chunks,
-                         size_t nchunks, size_t ntypes, double bin, const double *q, unsigned nq,
-                         double *S, bool prof);
-
 // H3 as an int8 matrix-core product (device pointers, S[ncols * nq] overwritten).
 int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, unsigned nhist,
                  double bin, const double *q, unsigned nq, double *S);

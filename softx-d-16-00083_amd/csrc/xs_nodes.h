@@ -24,8 +24,8 @@ namespace nodes {
 constexpr double kTol = 5e-13;
 
 // The largest Q h/4 for K moments.
-inline double reach(int K) {
-  double f = 0.5 * kTol;
+inline double reach(int K, double tol = kTol) {
+  double f = 0.5 * tol;
   for (int k = 2; k <= K; ++k) f *= k;
   return std::pow(f, 1.0 / K);
 }

@@ -1,12 +1,12 @@
 // H3 histogram -> pair sums and H4 RDF/PDF/rPDF on gfx950.
 //
 // H3: S_p(q) = sum_k h_p[k] sin(q r_k)/(q r_k), r_k = (k+1/2) bin, through the
-//   Chebyshev nodes of xs_nodesum.hip, in FP64: at low q the intensity is a
+//   Chebyshev nodes of xs_nodesum.hip or bin by bin, in FP64: at low q the intensity is a
 //   difference of the pair sum and the self term that cancels by up to four
 //   orders of magnitude, which FP32 terms (6e-8 relative each) cannot resolve
 //   to 1e-5 (the FP32 form, for comparison, is here).  The reference's
 //   denominator is q r + 1e-8 (CalcFunctions.cpp:861);
-//   1/(x + e) = (1/x)(1 - e/x) + O((e/x)^2) is applied per node, because at the
+//   1/(x + e) = (1/x)(1 - e/x) + O((e/x)^2) is applied per term, because at the
 //   cancelling low-q points that 1e-8 shifts I(q) by ~1e-6 relative.
 //   q = 0 gives S = 0 as the reference does (sin 0 = 0).
 // H4: the reference's PDF formulas (CalcFunctions.cpp:919-957) in FP64, one
@@ -31,6 +31,79 @@ __global__ void fill_f64(double *__restrict__ p, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
     p[i] = 0.0;
+}
+
+// The sums bin by bin, for calls that must not allocate: under stream capture (the
+// graph would keep a pointer to scratch that a later call may move) and where there
+// is no memory for the nodes' tables.  One thread per q and 2,048 bins, chunk sums
+// go to S with atomics: 97,251 bins x 4,096 q 94 us (nodes: 37).
+//
+// Sum over one staged chunk of bins [k0, k0 + kn) for one q (qv != 0).
+// bins[b] = (h y, h y^2) with y = 1/(k0 + b + 1/2), so that the term
+// h y (1 - eps_q y) sin((k + 1/2) q bin) is one FMA for its weight and one
+// to add it.  The sine s_k = sin((k + 1/2) t), t = q bin, is advanced by
+// Reinsch's form of the three-term recurrence (Stoer and Bulirsch,
+// Introduction to Numerical Analysis, sec. 2.3.3): with the difference
+// d_k = s_{k+1} - s_k and lam = -4 sin^2(t/2) = 2 cos t - 2,
+//   s_{k+1} = s_k + d_k,   d_{k+1} = d_k + lam s_{k+1}
+// (one add, one FMA), seeded with d_{k0} = 2 sin(t/2) cos((k0 + 1) t).  The
+// plain recurrence s_{k+1} = 2 cos t s_k - s_{k-1} rounds 2 cos t, whose
+// error shifts the frequency by ~eps cot t: over a 2048-bin chunk its sines
+// drifted by up to 2e-11 at t = 1e-4..1e-3 (an FP64 simulation against
+// extended precision), against 4e-16..2e-15 for this form and 2e-14 for a
+// rotation of (sin, cos) by t (four FMAs).  Two accumulators (even and odd
+// bins) halve the dependent chain of the sums.
+__device__ __forceinline__ double pairsum_chunk(const double2 *bins, unsigned k0, unsigned kn,
+                                                double qv, double bin) {
+  const double turns = qv * bin / (2.0 * kPi);  // phase step per bin, in turns
+  double s, c, h, g;
+  sincos_2pi(((double)k0 + 0.5) * turns, &s, &c);
+  sincos_2pi(0.5 * turns, &h, &g);
+  const double lam = -4.0 * h * h;
+  double d = 2.0 * h * fma(c, g, -(s * h));  // 2 sin(t/2) cos((k0 + 1) t)
+  const double eps_q = 1e-8 / (qv * bin);
+  double acc0 = 0.0, acc1 = 0.0;
+  unsigned b = 0;
+  for (; b + 2 <= kn; b += 2) {
+    const double2 e0 = bins[b], e1 = bins[b + 1];
+    acc0 = fma(fma(-eps_q, e0.y, e0.x), s, acc0);
+    s += d;
+    d = fma(lam, s, d);
+    acc1 = fma(fma(-eps_q, e1.y, e1.x), s, acc1);
+    s += d;
+    d = fma(lam, s, d);
+  }
+  if (b < kn) {
+    const double2 e0 = bins[b];
+    acc0 = fma(fma(-eps_q, e0.y, e0.x), s, acc0);
+  }
+  return acc0 + acc1;
+}
+
+__device__ __forceinline__ void stage_chunk(double2 *bins, const unsigned long long *__restrict__ h,
+                                            unsigned k0, unsigned kn) {
+  for (unsigned b = threadIdx.x; b < kn; b += kQBlock) {
+    const double y = 1.0 / ((double)(k0 + b) + 0.5), hy = (double)h[b] * y;
+    bins[b] = make_double2(hy, hy * y);
+  }
+}
+
+__global__ __launch_bounds__(kQBlock) void pairsum_kernel(const unsigned long long *__restrict__ hist,
+                                                          unsigned nhist, const double *__restrict__ q,
+                                                          unsigned nq, double bin,
+                                                          double *__restrict__ S) {
+  __shared__ double2 bins[kChunk];
+  const unsigned p = blockIdx.z;
+  const unsigned k0 = blockIdx.y * kChunk;
+  const unsigned kn = min((unsigned)kChunk, nhist - k0);
+  stage_chunk(bins, hist + (size_t)p * nhist + k0, k0, kn);
+  __syncthreads();
+  const unsigned iq = blockIdx.x * kQBlock + threadIdx.x;
+  if (iq >= nq) return;
+  const double qv = q[iq];
+  if (qv == 0.0) return;
+  const double acc = pairsum_chunk(bins, k0, kn, qv, bin);
+  if (acc != 0.0) atomicAdd(&S[(size_t)p * nq + iq], acc / (qv * bin));
 }
 
 // The plain FP32 form (XS_PAIRSUM_F32), for comparison: every term
@@ -193,21 +266,35 @@ extern "C" int xs_hist_pairsum(xs_ctx *ctx, const uint64_t *hist, unsigned ntype
   if (flags & XS_PAIRSUM_MFMA) {
     XS_TRY(pairsum_mfma(ctx, hd, ntypes, nhist, bin, qd, nq, Sd));
   } else {
+    const nodesum::Layout L =
+        nodesum::layout((ntypes + nodesum::kRows - 1) / nodesum::kRows, nhist, nodesum::kBudget);
+    bool nodes = !(flags & XS_PAIRSUM_F32);
+    if (nodes) {
+      hipStreamCaptureStatus capture;
+      XS_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));
+      nodes = capture == hipStreamCaptureStatusNone;
+    }
+    if (nodes) {
+      const int e = ensure_matrix(ctx, L.total);
+      if (e != XS_OK && e != XS_ERR_NOMEM) return e;
+      nodes = e == XS_OK;
+    }
     hipEvent_t ev;
-    if (flags & XS_PAIRSUM_F32) {
-      XS_TRY(prof_begin(ctx, "hist_pairsum", &ev));
+    XS_TRY(prof_begin(ctx, "hist_pairsum", &ev));
+    if (nodes) {
+      const nodesum::Tables T{L, static_cast<char *>(ctx->mat), ntypes, nhist, nullptr, nullptr};
+      XS_TRY(nodesum::run(ctx, T, hd, ntypes, bin, qd, nq, Sd));
+    } else {
       const unsigned zb = (unsigned)std::min<size_t>((ssize + 255) / 256, 4096);
       hipLaunchKernelGGL(iq::fill_f64, dim3(zb), dim3(256), 0, ctx->stream, Sd, ssize);
       dim3 grid((nq + iq::kQBlock - 1) / iq::kQBlock, (nhist + iq::kChunk - 1) / iq::kChunk, ntypes);
-      hipLaunchKernelGGL(iq::pairsum_f32_kernel, grid, dim3(iq::kQBlock), 0, ctx->stream, hd, nhist,
-                         qd, nq, bin, Sd);
+      if (flags & XS_PAIRSUM_F32)
+        hipLaunchKernelGGL(iq::pairsum_f32_kernel, grid, dim3(iq::kQBlock), 0, ctx->stream, hd, nhist,
+                           qd, nq, bin, Sd);
+      else
+        hipLaunchKernelGGL(iq::pairsum_kernel, grid, dim3(iq::kQBlock), 0, ctx->stream, hd, nhist, qd,
+                           nq, bin, Sd);
       XS_HIP_CHECK(hipGetLastError());
-    } else {
-      const nodesum::Layout L = nodesum::layout((ntypes + nodesum::kRows - 1) / nodesum::kRows, nhist, nodesum::kBudget);
-      XS_TRY(ensure_matrix(ctx, L.total));
-      XS_TRY(prof_begin(ctx, "hist_pairsum", &ev));
-      const nodesum::Tables T{L, static_cast<char *>(ctx->mat), ntypes, nhist, nullptr, nullptr};
-      XS_TRY(nodesum::run(ctx, T, hd, ntypes, bin, qd, nq, Sd));
     }
     XS_TRY(prof_end(ctx, "hist_pairsum", ev));
   }

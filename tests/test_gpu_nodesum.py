@@ -71,3 +71,35 @@ def test_zero_and_negative_q(ctx, rows):
     check(ctx, rows, 1500, 0.01, [0.0, -3.0, 7.5, -20.0, 0.0, 0.4])
     S = ctx.hist_pairsum(np.ones((rows, 50), np.uint64), 0.1, np.zeros(3))
     assert np.all(S == 0.0)
+
+
+def test_stream_capture(ctx):
+    """A captured call keeps no pointer to the context's scratch: replayed after a
+    larger call has moved it, and between eager calls."""
+    rng = np.random.default_rng(3)
+    q = np.linspace(0.3, 20.0, 300)
+    h = rng.integers(0, 1000, (3, 5000)).astype(np.uint64)
+    ref = O.hist_pairsum(h, 0.01, q)
+    bar = 1e-12 * np.abs(ref).max()
+    with xh.Context(0) as c:
+        hd, qd = torch.from_numpy(h.astype(np.int64)).cuda(), torch.from_numpy(q).cuda()
+        S = torch.empty((3, q.size), dtype=torch.float64, device="cuda")
+        run = lambda: c.hist_pairsum_dev(hd.data_ptr(), 3, 5000, 0.01, qd.data_ptr(), q.size, S.data_ptr())
+        stream = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        c.set_stream(stream.cuda_stream)
+        run()
+        c.synchronize()
+        assert np.abs(S.cpu().numpy() - ref).max() <= bar
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            run()
+        for k in range(3):
+            c.hist_pairsum(np.ones((40 * (k + 1), 9000 * (k + 1)), np.uint64), 0.01, q)
+            S.fill_(7.0)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                g.replay()
+            torch.cuda.synchronize()
+            assert np.abs(S.cpu().numpy() - ref).max() <= bar
+        c.set_stream(0)

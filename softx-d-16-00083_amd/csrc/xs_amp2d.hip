@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "xs_internal.h"
+#include "xs_sincos.h"
 
 namespace xs {
 namespace amp2d {
@@ -76,36 +77,48 @@ __global__ __launch_bounds__(kBlock) void amp2d_kernel(Args A) {
   if (valid) atomicAdd(&A.I[k], Ar * Ar + Ai * Ai);
 }
 
-// Regular q grid: q(iu, iv) = q0 + iu du + iv dv, point k = iv nu + iu.
-// One thread per run of kRun consecutive points of a row and one rotation.
-// For an atom x the phase advances by delta = (R^T du).x per point, so the
-// run's terms are z_m = exp(i ph0) e^{i m delta}: z_0 from one FP32 hardware
-// sine/cosine of the FP64-reduced first phase (as the list kernel), z_1 =
-// z_0 (cos delta + i sin delta), then z_{m+1} = 2 cos(delta) z_m - z_{m-1}
-// (two FP64 FMAs a point).  cos and sin of delta are computed once per atom
-// and work group in FP64 and kept in LDS.  The three-term recurrence scales
-// a rounding error made at step k by |sin((m-k) delta) / sin(delta)| <= m - k,
-// so over a run of 8 it adds < 1e-14 to the seed's error (2^-24 turn).
+// Regular q grid: q(iu, iv) = q0 + iu du + iv dv, point k = iv nu + iu, in runs
+// of 16 consecutive points of a row.  For an atom x the phase advances by
+// delta = (R^T du).x per point.  The run's first phase gives one FP32 hardware
+// sine and cosine (FP64-reduced, as the list kernel), turned by 7.5 delta to the
+// middle of the run in FP64; from there the points lie at +-b delta, b = 1/2 ...
+// 15/2, so with z = C + i S of the middle
+//   sum z e^{+-i b delta} = (sum C cos -+ sum S sin) + i (sum S cos +- sum C sin),
+// two matrix products over the atoms, of 16 runs x (8 cosines, 8 sines) each, and
+// every term serves both signs: 4 atoms x 16 runs x 16 points are two
+// v_mfma_f64_16x16x4.  The cosines and sines of an atom are made once per work
+// group and chunk (FP64, in LDS); a lane forms the seed of one run and atom, the
+// layout that the instruction reads.
+// Bound by the FP64 units: the matrix instructions (128 cycles of a SIMD for 64 runs
+// and atoms) and the seeds (~65), which do not overlap.  50,000 atoms, 512 x 512
+// points, 8 rotations: 9.3 ms; 16 points advanced one from another by a three-term
+// recurrence (four FP64 operations a point, 330 cycles) took 16.1, and 10 times as
+// long on planes of a few thousand runs, which left most of the chip idle.
 constexpr int kRun = 16;
-constexpr int kGridChunk = 512;
+constexpr int kGridChunk = 128;
 
 struct GridArgs {
   const double *x, *y, *z;
   const double *rot;  // nrot x 9
   const double *ff;   // n_el x nqp
   double *I;
+  double *amp;  // nrot x nqp, complex
   double q0[3], du[3], dv[3];
   unsigned nu, nv, runs_per_row, n_el;
   unsigned el_off[17];
 };
 
-__global__ __launch_bounds__(kBlock) void amp2d_grid_kernel(GridArgs A) {
-  __shared__ double sx[kGridChunk], sy[kGridChunk], sz[kGridChunk], sc[kGridChunk],
-      ss[kGridChunk];
-  const unsigned run = blockIdx.x * kBlock + threadIdx.x;
-  const unsigned iv = run / A.runs_per_row;
-  const unsigned iu0 = (run - iv * A.runs_per_row) * kRun;
-  const bool valid = iv < A.nv;
+typedef double double4v __attribute__((ext_vector_type(4)));
+
+// A wave has T tiles of 16 runs.  Grid (tiles, rotations, shares of the atoms'
+// chunks): with more than one share the amplitudes are added up in A.amp.
+template <int T>
+__global__ __launch_bounds__(kBlock, T == 1 ? 4 : 3) void amp2d_grid_kernel(GridArgs A) {
+  constexpr unsigned kStride = 17;  // of an atom's 16 columns: banks
+  __shared__ double sx[kGridChunk], sy[kGridChunk], sz[kGridChunk], sb[kGridChunk * kStride];
+  const unsigned lane = threadIdx.x & 63, col = lane & 15, kc = lane >> 4;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned run0 = (blockIdx.x * (kBlock / 64) + wave) * 16 * T;
   const double *R = A.rot + 9 * (size_t)blockIdx.y;
   // R^T applied to a vector, in turns
   auto turn = [&](double a, double b, double c, double *o) {
@@ -113,73 +126,121 @@ __global__ __launch_bounds__(kBlock) void amp2d_grid_kernel(GridArgs A) {
     o[1] = (a * R[1] + b * R[4] + c * R[7]) * kInvTwoPi;
     o[2] = (a * R[2] + b * R[5] + c * R[8]) * kInvTwoPi;
   };
-  double q[3] = {0, 0, 0}, d[3];
-  if (valid) {
-    const double u = (double)iu0, v = (double)iv;
+  double q[T][3], d[3];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const unsigned run = run0 + 16 * t + col;
+    const unsigned iv = min(run / A.runs_per_row, A.nv - 1);
+    const double u = (double)(run % A.runs_per_row * kRun), v = (double)iv;
     turn(A.q0[0] + u * A.du[0] + v * A.dv[0], A.q0[1] + u * A.du[1] + v * A.dv[1],
-         A.q0[2] + u * A.du[2] + v * A.dv[2], q);
+         A.q0[2] + u * A.du[2] + v * A.dv[2], q[t]);
   }
   turn(A.du[0], A.du[1], A.du[2], d);
-  const size_t k0 = (size_t)iv * A.nu + iu0;
-  double Ar[kRun], Ai[kRun];
+  // the lane's points: run run0 + 16 t + kc + 4 i, place 8 + col or, from column 8
+  // on, 15 - col
+  const bool low = col < 8;
+  const unsigned place = low ? 8 + col : 15 - col;
+  double Ar[T][4], Ai[T][4];
 #pragma unroll
-  for (int m = 0; m < kRun; ++m) Ar[m] = Ai[m] = 0.0;
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) Ar[t][i] = Ai[t][i] = 0.0;
+  auto point = [&](int t, int i, size_t *k) {
+    const unsigned run = run0 + 16 * t + kc + 4 * i, iv = run / A.runs_per_row;
+    const unsigned iu = run % A.runs_per_row * kRun + place;
+    *k = (size_t)iv * A.nu + iu;
+    return iv < A.nv && iu < A.nu;
+  };
+  unsigned chunk = 0;
   for (unsigned e = 0; e < A.n_el; ++e) {
-    double ar[kRun], ai[kRun];
+    double4v ac[T], as[T];
 #pragma unroll
-    for (int m = 0; m < kRun; ++m) ar[m] = ai[m] = 0.0;
+    for (int t = 0; t < T; ++t) ac[t] = as[t] = (double4v){0.0, 0.0, 0.0, 0.0};
     const unsigned e0 = A.el_off[e], e1 = A.el_off[e + 1];
     for (unsigned c0 = e0; c0 < e1; c0 += kGridChunk) {
+      if (chunk++ % gridDim.z != blockIdx.z) continue;
       const unsigned cn = min((unsigned)kGridChunk, e1 - c0);
       __syncthreads();
-      for (unsigned j = threadIdx.x; j < cn; j += kBlock) {
-        const double xj = A.x[c0 + j], yj = A.y[c0 + j], zj = A.z[c0 + j];
-        sx[j] = xj;
-        sy[j] = yj;
-        sz[j] = zj;
+      {  // two threads an atom, four of b each; atoms beyond the last are zeros
+        const unsigned j = threadIdx.x % kGridChunk, half = threadIdx.x / kGridChunk;
+        const bool in = j < cn;
+        const double xj = in ? A.x[c0 + j] : 0.0, yj = in ? A.y[c0 + j] : 0.0,
+                     zj = in ? A.z[c0 + j] : 0.0;
+        if (half == 0) {
+          sx[j] = xj;
+          sy[j] = yj;
+          sz[j] = zj;
+        }
         const double st = fma(d[0], xj, fma(d[1], yj, d[2] * zj));
-        double sn, cs;
-        sincospi(2.0 * (st - floor(st)), &sn, &cs);
-        sc[j] = cs;
-        ss[j] = sn;
+        double sn, cs, s1, c1;
+        sincos_2pi(st, &s1, &c1);
+        sincos_2pi((half ? 4.5 : 0.5) * (st - rint(0.5 * st) * 2.0), &sn, &cs);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          sb[j * kStride + 4 * half + b] = in ? cs : 0.0;
+          sb[j * kStride + 8 + 4 * half + b] = in ? sn : 0.0;
+          const double c = fma(cs, c1, -(sn * s1));
+          sn = fma(cs, s1, sn * c1);
+          cs = c;
+        }
       }
       __syncthreads();
-      for (unsigned j = 0; j < cn; ++j) {
-        const double ph = fma(q[0], sx[j], fma(q[1], sy[j], q[2] * sz[j]));
-        const float f = (float)(ph - floor(ph));
-        const double c = sc[j], sn = ss[j], c2 = 2.0 * c;
-        double rp = (double)__builtin_amdgcn_cosf(f), ip = (double)__builtin_amdgcn_sinf(f);
-        double re = fma(rp, c, -ip * sn), im = fma(rp, sn, ip * c);
-        ar[0] += rp;
-        ai[0] += ip;
+      for (unsigned j0 = 0; j0 < cn; j0 += 4) {
+        const unsigned j = j0 + kc;
+        const double xj = sx[j], yj = sy[j], zj = sz[j];
+        const double b = sb[j * kStride + col], rc = sb[j * kStride + 7], rs = sb[j * kStride + 15];
 #pragma unroll
-        for (int m = 1; m < kRun; ++m) {
-          ar[m] += re;
-          ai[m] += im;
-          if (m + 1 < kRun) {
-            const double rn = fma(c2, re, -rp), in = fma(c2, im, -ip);
-            rp = re;
-            ip = im;
-            re = rn;
-            im = in;
-          }
+        for (int t = 0; t < T; ++t) {
+          const double ph = fma(q[t][0], xj, fma(q[t][1], yj, q[t][2] * zj));
+          const float f = (float)__builtin_amdgcn_fract(ph);
+          const double c = (double)__builtin_amdgcn_cosf(f), s = (double)__builtin_amdgcn_sinf(f);
+          ac[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(fma(c, rc, -(s * rs)), b, ac[t], 0, 0, 0);
+          as[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(fma(s, rc, c * rs), b, as[t], 0, 0, 0);
         }
       }
     }
-    if (valid) {
 #pragma unroll
-      for (int m = 0; m < kRun; ++m)
-        if (iu0 + m < A.nu) {
-          const double w = A.ff[(size_t)e * A.nu * A.nv + k0 + m];
-          Ar[m] = fma(w, ar[m], Ar[m]);
-          Ai[m] = fma(w, ai[m], Ai[m]);
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // columns 0-7: sum C cos, sum S cos; 8-15: sum C sin, sum S sin
+        const double pc = __shfl_xor(ac[t][i], 8, 64), ps = __shfl_xor(as[t][i], 8, 64);
+        const double re = low ? ac[t][i] - ps : pc + as[t][i];
+        const double im = low ? as[t][i] + pc : ps - ac[t][i];
+        size_t k;
+        if (point(t, i, &k)) {
+          const double w = A.ff[(size_t)e * A.nu * A.nv + k];
+          Ar[t][i] = fma(w, re, Ar[t][i]);
+          Ai[t][i] = fma(w, im, Ai[t][i]);
         }
-    }
+      }
   }
-  if (valid) {
 #pragma unroll
-    for (int m = 0; m < kRun; ++m)
-      if (iu0 + m < A.nu) atomicAdd(&A.I[k0 + m], Ar[m] * Ar[m] + Ai[m] * Ai[m]);
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      size_t k;
+      if (!point(t, i, &k)) continue;
+      if (gridDim.z > 1) {
+        double *o = A.amp + 2 * ((size_t)blockIdx.y * A.nu * A.nv + k);
+        atomicAdd(o, Ar[t][i]);
+        atomicAdd(o + 1, Ai[t][i]);
+      } else {
+        atomicAdd(&A.I[k], Ar[t][i] * Ar[t][i] + Ai[t][i] * Ai[t][i]);
+      }
+    }
+}
+
+__global__ void sum_squares(const double *__restrict__ amp, size_t nqp, unsigned nrot,
+                            double *__restrict__ I) {
+  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < nqp;
+       k += (size_t)gridDim.x * blockDim.x) {
+    double v = 0.0;
+    for (unsigned r = 0; r < nrot; ++r) {
+      const double *a = amp + 2 * (r * nqp + k);
+      v += a[0] * a[0] + a[1] * a[1];
+    }
+    I[k] = v;
   }
 }
 
@@ -307,14 +368,43 @@ extern "C" int xs_amp2d_grid(xs_ctx *ctx, const double *xyz, size_t n_atoms,
   A.rot = rd;
   A.ff = fd;
   A.I = Id;
-  const unsigned zb = (unsigned)std::min<size_t>((nqp + 255) / 256, 4096);
-  hipLaunchKernelGGL(amp2d::zero_f64, dim3(zb), dim3(256), 0, ctx->stream, Id, nqp);
-  const size_t runs = (size_t)A.runs_per_row * nv;
+  const size_t tiles = ((size_t)A.runs_per_row * nv + 15) / 16, groups = (tiles + 3) / 4 * nrot;
+  // Few tiles leave CUs idle or a last round of work groups nearly empty: the atoms
+  // are shared out, until there are 12 work groups a CU (not under stream capture,
+  // where a graph would keep the scratch's address, nor without memory for it).
+  // 31,170 atoms, 304 x 240 points, 8 rotations: 2.0 ms (one share 2.5); 32,397
+  // atoms, 363 x 375, 8 rotations: 3.7 ms (one share, tiles in pairs: 4.6).  Above that
+  // two tiles a wave share the loads of an atom: 50,000 atoms, 512 x 512, 8 rotations
+  // 9.3 ms against 9.8 with one.
+  const unsigned chunks = (unsigned)((n_atoms + amp2d::kGridChunk - 1) / amp2d::kGridChunk);
+  unsigned shares = 1;
+  if (groups < 8 * (size_t)ctx->cu_count) {
+    shares = std::max(1u, std::min((unsigned)(12 * (size_t)ctx->cu_count / groups), chunks / 2));
+    hipStreamCaptureStatus capture;
+    XS_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) shares = 1;
+  }
+  if (shares > 1) {
+    const int e = ensure_matrix(ctx, nrot * nqp * 16);
+    if (e != XS_OK && e != XS_ERR_NOMEM) return e;
+    if (e != XS_OK) shares = 1;
+    A.amp = static_cast<double *>(ctx->mat);
+  }
+  double *const sum = shares > 1 ? A.amp : Id;
+  const size_t nsum = shares > 1 ? 2 * nrot * nqp : nqp;
+  hipLaunchKernelGGL(amp2d::zero_f64, dim3((unsigned)std::min<size_t>((nsum + 255) / 256, 4096)),
+                     dim3(256), 0, ctx->stream, sum, nsum);
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "amp2d", &ev));
-  hipLaunchKernelGGL(amp2d::amp2d_grid_kernel,
-                     dim3((unsigned)((runs + amp2d::kBlock - 1) / amp2d::kBlock), nrot),
-                     dim3(amp2d::kBlock), 0, ctx->stream, A);
+  if (groups >= 8 * (size_t)ctx->cu_count)
+    hipLaunchKernelGGL(amp2d::amp2d_grid_kernel<2>, dim3((unsigned)((tiles + 7) / 8), nrot),
+                       dim3(amp2d::kBlock), 0, ctx->stream, A);
+  else
+    hipLaunchKernelGGL(amp2d::amp2d_grid_kernel<1>, dim3((unsigned)((tiles + 3) / 4), nrot, shares),
+                       dim3(amp2d::kBlock), 0, ctx->stream, A);
+  if (shares > 1)
+    hipLaunchKernelGGL(amp2d::sum_squares, dim3((unsigned)std::min<size_t>((nqp + 255) / 256, 4096)),
+                       dim3(256), 0, ctx->stream, A.amp, nqp, nrot, Id);
   XS_HIP_CHECK(hipGetLastError());
   XS_TRY(prof_end(ctx, "amp2d", ev));
   if (!device) {

@@ -5,12 +5,17 @@
 // atoms, 1020-1022 and 1033).
 //
 // One thread per (q point, rotation); the atoms stream through LDS in chunks
-// of 1024 (FP64 SoA), read by every lane at the same address (broadcast).
+// of 256 (FP64 SoA), read by every lane at the same address (broadcast).
 // The phase q'.x is formed in FP64 (in turns) and reduced to [0, 1), so the
 // FP32 hardware sine and cosine (v_sin_f32 / v_cos_f32 take turns) see an
 // argument accurate to 2^-24 turn even where q'.x reaches 10^2 turns; the
 // element amplitudes are accumulated in FP64 and |A|^2 is added into the
-// FP64 result with atomics (one per rotation and q point).
+// FP64 result with atomics (one per rotation and q point), or, where the atoms
+// are given out in shares, the amplitudes are.  Bound by the issue of one term:
+// three FMAs, v_fract_f64 (a floor and a subtraction took 5 cycles more), a
+// conversion to FP32, two hardware sines, two conversions back and two adds,
+// ~55 cycles of a SIMD for 64 points; 20,000 atoms x 92,160 points x 4 rotations
+// 2.87 ms (3.11 with floor and one share).
 #include <algorithm>
 #include <cmath>
 
@@ -21,7 +26,7 @@ namespace xs {
 namespace amp2d {
 
 constexpr int kBlock = 256;
-constexpr int kChunk = 1024;
+constexpr int kChunk = 256;
 constexpr double kInvTwoPi = 0.15915494309189533576888376337251;
 
 struct Args {
@@ -30,6 +35,7 @@ struct Args {
   const double *rot;   // nrot x 9, row-major R
   const double *ff;    // n_el x nqp
   double *I;
+  double *amp;  // nrot x nqp, complex
   unsigned nqp, n_el;
   unsigned el_off[17];
 };
@@ -48,10 +54,12 @@ __global__ __launch_bounds__(kBlock) void amp2d_kernel(Args A) {
     qz = (a * R[2] + b * R[5] + c * R[8]) * kInvTwoPi;
   }
   double Ar = 0.0, Ai = 0.0;
+  unsigned chunk = 0;
   for (unsigned e = 0; e < A.n_el; ++e) {
     double ar = 0.0, ai = 0.0;
     const unsigned e0 = A.el_off[e], e1 = A.el_off[e + 1];
     for (unsigned c0 = e0; c0 < e1; c0 += kChunk) {
+      if (chunk++ % gridDim.z != blockIdx.z) continue;
       const unsigned cn = min((unsigned)kChunk, e1 - c0);
       __syncthreads();
       for (unsigned j = threadIdx.x; j < cn; j += kBlock) {
@@ -63,7 +71,7 @@ __global__ __launch_bounds__(kBlock) void amp2d_kernel(Args A) {
 #pragma unroll 4
       for (unsigned j = 0; j < cn; ++j) {
         const double ph = fma(qx, sx[j], fma(qy, sy[j], qz * sz[j]));
-        const float f = (float)(ph - floor(ph));
+        const float f = (float)__builtin_amdgcn_fract(ph);
         ar += (double)__builtin_amdgcn_cosf(f);
         ai += (double)__builtin_amdgcn_sinf(f);
       }
@@ -74,7 +82,14 @@ __global__ __launch_bounds__(kBlock) void amp2d_kernel(Args A) {
       Ai = fma(w, ai, Ai);
     }
   }
-  if (valid) atomicAdd(&A.I[k], Ar * Ar + Ai * Ai);
+  if (!valid) return;
+  if (gridDim.z > 1) {
+    double *o = A.amp + 2 * ((size_t)blockIdx.y * A.nqp + k);
+    atomicAdd(o, Ar);
+    atomicAdd(o + 1, Ai);
+  } else {
+    atomicAdd(&A.I[k], Ar * Ar + Ai * Ai);
+  }
 }
 
 // Regular q grid: q(iu, iv) = q0 + iu du + iv dv, point k = iv nu + iu, in runs
@@ -250,6 +265,29 @@ __global__ void zero_f64(double *__restrict__ p, size_t n) {
     p[i] = 0.0;
 }
 
+// How many shares the atoms are given out in.  Few work groups leave CUs idle or a
+// last round of them nearly empty: below 8 a CU the atoms are shared out until there
+// are 12, two chunks a share at least.  Not under stream capture, where a graph would
+// keep the scratch's address, nor without memory for the amplitudes.
+// Grid, 31,170 atoms, 304 x 240 points, 8 rotations: 2.0 ms (one share 2.5); 32,397
+// atoms, 363 x 375, 8 rotations: 3.7 ms (one share, tiles in pairs: 4.6).  List, 20,000
+// atoms, 92,160 points, 4 rotations: 2.87 ms; 10,106 atoms, 6,319 points, 2 rotations:
+// 65 us (one share 387).
+static int atom_shares(xs_ctx *ctx, size_t groups, size_t n_atoms, unsigned chunk, size_t amplitudes,
+                       unsigned *shares) {
+  *shares = 1;
+  const size_t most = (n_atoms + chunk - 1) / chunk / 2, cus = (size_t)ctx->cu_count;
+  if (groups >= 8 * cus || most < 2) return XS_OK;
+  hipStreamCaptureStatus capture;
+  XS_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));
+  if (capture != hipStreamCaptureStatusNone) return XS_OK;
+  const size_t want = std::min<size_t>(std::min(12 * cus / groups, most), 65535);
+  if (want < 2) return XS_OK;
+  const int e = ensure_matrix(ctx, amplitudes * 16);
+  if (e == XS_OK) *shares = (unsigned)want;
+  return e == XS_ERR_NOMEM ? XS_OK : e;
+}
+
 }  // namespace amp2d
 }  // namespace xs
 
@@ -300,12 +338,21 @@ extern "C" int xs_amp2d(xs_ctx *ctx, const double *xyz, size_t n_atoms, const un
   A.rot = rd;
   A.ff = fd;
   A.I = Id;
-  const unsigned zb = (unsigned)std::min<size_t>((nqp + 255) / 256, 4096);
-  hipLaunchKernelGGL(amp2d::zero_f64, dim3(zb), dim3(256), 0, ctx->stream, Id, nqp);
+  const size_t groups = (nqp + amp2d::kBlock - 1) / amp2d::kBlock;
+  unsigned shares = 1;
+  XS_TRY(amp2d::atom_shares(ctx, groups * nrot, n_atoms, amp2d::kChunk, (size_t)nrot * nqp, &shares));
+  A.amp = static_cast<double *>(ctx->mat);
+  double *const sum = shares > 1 ? A.amp : Id;
+  const size_t nsum = shares > 1 ? 2 * (size_t)nrot * nqp : nqp;
+  hipLaunchKernelGGL(amp2d::zero_f64, dim3((unsigned)std::min<size_t>((nsum + 255) / 256, 4096)),
+                     dim3(256), 0, ctx->stream, sum, nsum);
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "amp2d", &ev));
-  hipLaunchKernelGGL(amp2d::amp2d_kernel, dim3((unsigned)((nqp + amp2d::kBlock - 1) / amp2d::kBlock), nrot),
-                     dim3(amp2d::kBlock), 0, ctx->stream, A);
+  hipLaunchKernelGGL(amp2d::amp2d_kernel, dim3((unsigned)groups, nrot, shares), dim3(amp2d::kBlock), 0,
+                     ctx->stream, A);
+  if (shares > 1)
+    hipLaunchKernelGGL(amp2d::sum_squares, dim3((unsigned)std::min<size_t>((nqp + 255) / 256, 4096)),
+                       dim3(256), 0, ctx->stream, A.amp, nqp, nrot, Id);
   XS_HIP_CHECK(hipGetLastError());
   XS_TRY(prof_end(ctx, "amp2d", ev));
   if (!device) {
@@ -369,29 +416,13 @@ extern "C" int xs_amp2d_grid(xs_ctx *ctx, const double *xyz, size_t n_atoms,
   A.ff = fd;
   A.I = Id;
   const size_t tiles = ((size_t)A.runs_per_row * nv + 15) / 16, groups = (tiles + 3) / 4 * nrot;
-  // Few tiles leave CUs idle or a last round of work groups nearly empty: the atoms
-  // are shared out, until there are 12 work groups a CU (not under stream capture,
-  // where a graph would keep the scratch's address, nor without memory for it).
-  // 31,170 atoms, 304 x 240 points, 8 rotations: 2.0 ms (one share 2.5); 32,397
-  // atoms, 363 x 375, 8 rotations: 3.7 ms (one share, tiles in pairs: 4.6).  Above that
-  // two tiles a wave share the loads of an atom: 50,000 atoms, 512 x 512, 8 rotations
-  // 9.3 ms against 9.8 with one.
-  const unsigned chunks = (unsigned)((n_atoms + amp2d::kGridChunk - 1) / amp2d::kGridChunk);
+  // (two tiles a wave share the loads of an atom: 9.3 ms for 50,000 atoms, 512 x 512
+  // points and 8 rotations, 9.8 with one; more than that loses to shares below it)
   unsigned shares = 1;
-  if (groups < 8 * (size_t)ctx->cu_count) {
-    shares = std::max(1u, std::min((unsigned)(12 * (size_t)ctx->cu_count / groups), chunks / 2));
-    hipStreamCaptureStatus capture;
-    XS_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));
-    if (capture != hipStreamCaptureStatusNone) shares = 1;
-  }
-  if (shares > 1) {
-    const int e = ensure_matrix(ctx, nrot * nqp * 16);
-    if (e != XS_OK && e != XS_ERR_NOMEM) return e;
-    if (e != XS_OK) shares = 1;
-    A.amp = static_cast<double *>(ctx->mat);
-  }
+  XS_TRY(amp2d::atom_shares(ctx, groups, n_atoms, amp2d::kGridChunk, (size_t)nrot * nqp, &shares));
+  A.amp = static_cast<double *>(ctx->mat);
   double *const sum = shares > 1 ? A.amp : Id;
-  const size_t nsum = shares > 1 ? 2 * nrot * nqp : nqp;
+  const size_t nsum = shares > 1 ? 2 * (size_t)nrot * nqp : nqp;
   hipLaunchKernelGGL(amp2d::zero_f64, dim3((unsigned)std::min<size_t>((nsum + 255) / 256, 4096)),
                      dim3(256), 0, ctx->stream, sum, nsum);
   hipEvent_t ev;

@@ -175,6 +175,7 @@ int xs_free(xs_ctx *ctx) {
     (void)hipEventDestroy(r.stop);
   }
   for (auto e : ctx->event_pool) (void)hipEventDestroy(e);
+  if (ctx->read_back) (void)hipEventDestroy(ctx->read_back);
   if (ctx->ws) (void)hipFree(ctx->ws);
   if (ctx->aux) (void)hipFree(ctx->aux);
   if (ctx->mat) (void)hipFree(ctx->mat);

@@ -140,6 +140,7 @@ struct xs_ctx {
   std::vector<xs::ProfRecord> prof_pending;
   std::map<std::string, std::pair<double, unsigned long long>> prof_done;
   std::vector<hipEvent_t> event_pool;
+  hipEvent_t read_back = nullptr;  // after a copy that the host waits for
 };
 
 namespace xs {

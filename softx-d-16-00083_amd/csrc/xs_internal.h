@@ -96,6 +96,7 @@ struct xs_atoms {
   std::vector<unsigned> block_el_count;  // [nblocks * n_el]
   size_t n = 0;
   double *xyz = nullptr;  // x[n], y[n], z[n]
+  size_t cap = 0;         // its bytes
 };
 
 struct xs_ctx {
@@ -126,6 +127,8 @@ struct xs_ctx {
   std::set<xs_batch *> plans;
   // Built ensembles on this context (freed by xs_free if still alive).
   std::set<xs_atoms *> atom_sets;
+  double *spare = nullptr;  // an atom set's memory for the next build (xs_atoms.hip)
+  size_t spare_size = 0;
 
   // FP32 binning: bins (float bits) checked for the FP32 quotient form; the
   // outcome of the exhaustive check of the FP32 square root (-1 not run yet,

@@ -3,7 +3,7 @@
 // Tiling.  Each element's atoms are split into equal-count tiles of kTile
 // atoms (all full but one), compact in space and no wider than two tile
 // diagonals fit the LDS window: k-d splits on the host (kd_tiles), x-slab /
-// y-column / z-run radix sorts on the device (eq_tiles_device), or, when
+// y-column / z-run counts on the device (xs_order.hip), or, when
 // those tiles are too wide for the window, the cells of a uniform grid.  A
 // tile carries its bounding box.  Counts do not depend on atom order, so the
 // permutation leaves the histogram unchanged.
@@ -29,7 +29,7 @@
 //
 // Pipelines.
 //   xs_hist, device input: the bbox is computed on the GPU and read back; the
-//     equal-count sorts run on the GPU and the tiles follow from the counts
+//     atoms are put in tile order on the GPU and the tiles follow from the counts
 //     (one more read-back of the tile boxes when the window caps their width;
 //     the cell-grid fallback reads back per-cell counts).
 //   xs_hist, host input, and xs_batch_plan: the sort, tiles, boxes and work
@@ -48,11 +48,10 @@
 #include <type_traits>
 #include <vector>
 
-#include <hipcub/hipcub.hpp>
-
 #include "xs_fixbin.h"
 #include "xs_hist_plan.h"
 #include "xs_internal.h"
+#include "xs_order.h"
 
 namespace xs {
 namespace hist {
@@ -187,7 +186,8 @@ __global__ void hist_scatter(const T *__restrict__ x, const T *__restrict__ y,
 template <class T>
 __global__ void hist_tile_boxes(const T *__restrict__ x, const T *__restrict__ y,
                                 const T *__restrict__ z, const Tile *__restrict__ tiles,
-                                double *__restrict__ boxes) {
+                                double *__restrict__ boxes, double cap,
+                                unsigned long long *__restrict__ wide) {
   const Tile t = tiles[blockIdx.x];
   double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (uint32_t i = threadIdx.x; i < t.cnt; i += blockDim.x) {
@@ -213,60 +213,13 @@ __global__ void hist_tile_boxes(const T *__restrict__ x, const T *__restrict__ y
     __syncthreads();
   }
   if (threadIdx.x < 6) boxes[(size_t)blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
+  if (wide && threadIdx.x < 3 && s[3 + threadIdx.x][0] - s[threadIdx.x][0] > cap) *wide = 1ull;
 }
 
 __global__ void fill_u64(unsigned long long *__restrict__ p, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
     p[i] = 0ull;
-}
-
-// ---- equal-count tiles on the device (see eq_tiles_device) ----
-
-__global__ void iota_u32(uint32_t *p, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = i;
-}
-
-// Part of rank r when n ranks are split into g equal-count parts, part s
-// starting at floor(s n / g).
-__device__ inline uint32_t equal_part(uint64_t r, uint64_t n, uint64_t g) {
-  uint64_t s = r * g / n;
-  while (s + 1 < g && (s + 1) * n / g <= r) ++s;
-  while (s > 0 && s * n / g > r) --s;
-  return (uint32_t)s;
-}
-
-// slab[ord[r]] = equal part of rank r (ord: atoms in x order)
-__global__ void eq_slabs(const uint32_t *ord, uint32_t n, uint32_t gx, uint32_t *slab) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n) slab[ord[r]] = equal_part(r, n, gx);
-}
-
-__global__ void gather_u32(const uint32_t *src, const uint32_t *ord, uint32_t n, uint32_t *dst) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n) dst[r] = src[ord[r]];
-}
-
-// col[ord[r]] = s gy + equal part of r within slab s (ord: slab-major, y order)
-__global__ void eq_columns(const uint32_t *sslab, const uint32_t *ord, uint32_t n, uint32_t gx,
-                           uint32_t gy, uint32_t *col) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const uint64_t s = sslab[r];
-  const uint64_t st = s * n / gx, en = (s + 1) * n / gx;
-  col[ord[r]] = (uint32_t)s * gy + equal_part(r - st, en - st, gy);
-}
-
-template <class T>
-__global__ void gather_xyz(const T *x, const T *y, const T *z, const uint32_t *ord, uint32_t n,
-                           T *sx, T *sy, T *sz) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const uint32_t i = ord[r];
-  sx[r] = x[i];
-  sy[r] = y[i];
-  sz[r] = z[i];
 }
 
 // ---------------------------------------------------------------- histogram kernel
@@ -1394,76 +1347,6 @@ static int quot_f32_exact(xs_ctx *ctx, double bin_d, bool *ok) {
 
 // ---------------------------------------------------------------- xs_hist
 
-// Scratch of eq_tiles_device for elements of up to maxne atoms.
-template <class T>
-static size_t eq_scratch_bytes(uint32_t maxne, size_t *sort_bytes) {
-  size_t b1 = 0, b2 = 0;
-  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, b1, (const T *)nullptr, (T *)nullptr,
-                                           (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                           (int)maxne);
-  (void)hipcub::DeviceRadixSort::SortPairs(nullptr, b2, (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                           (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                           (int)maxne);
-  *sort_bytes = align_up(std::max(b1, b2), 256);
-  return Carver::need({maxne * sizeof(T), 6 * (size_t)maxne * sizeof(uint32_t), *sort_bytes});
-}
-
-// Equal-count tiles of every element on the device: stable radix sorts by
-// x (slabs), by y then slab (columns), by z then column (tiles); the sorted
-// coordinates go to sxp, syp, szp (element-major, as the input).
-template <class T>
-static int eq_tiles_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_count,
-                           unsigned n_el, const uint32_t *eoff, const double bbox[6], double cap,
-                           void *scratch, uint32_t maxne, T *sxp, T *syp, T *szp,
-                           std::vector<Tile> &tiles, uint32_t *ebase, uint32_t *en) {
-  size_t sb = 0;
-  (void)eq_scratch_bytes<T>(maxne, &sb);
-  Carver cv(scratch);
-  T *kout = cv.take<T>(maxne);
-  uint32_t *iota = cv.take<uint32_t>(maxne), *ordA = cv.take<uint32_t>(maxne),
-           *ordB = cv.take<uint32_t>(maxne), *lab = cv.take<uint32_t>(maxne),
-           *k32a = cv.take<uint32_t>(maxne), *k32b = cv.take<uint32_t>(maxne);
-  void *tmp = cv.take<char>(sb);
-  hipStream_t st = ctx->stream;
-  for (unsigned e = 0; e < n_el; ++e) {
-    const uint32_t ne = el_count[e];
-    ebase[e] = (uint32_t)tiles.size();
-    en[e] = 0;
-    if (!ne) continue;
-    const T *ex = xyz + eoff[e], *ey = xyz + n + eoff[e], *ez = xyz + 2 * n + eoff[e];
-    uint32_t gx, gy, nz;
-    choose_equal_count(ne, bbox, cap, sizeof(T) == 8, gx, gy, nz);
-    const unsigned nb = (ne + 255) / 256;
-    size_t b = sb;
-    hipLaunchKernelGGL(iota_u32, dim3(nb), dim3(256), 0, st, iota, ne);
-    XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, ex, kout, iota, ordA, (int)ne, 0,
-                                                    (int)(sizeof(T) * 8), st));
-    hipLaunchKernelGGL(eq_slabs, dim3(nb), dim3(256), 0, st, ordA, ne, gx, lab);
-    b = sb;
-    XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, ey, kout, iota, ordA, (int)ne, 0,
-                                                    (int)(sizeof(T) * 8), st));
-    hipLaunchKernelGGL(gather_u32, dim3(nb), dim3(256), 0, st, lab, ordA, ne, k32a);
-    b = sb;
-    XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, k32a, k32b, ordA, ordB, (int)ne, 0,
-                                                    bits_for(gx), st));
-    hipLaunchKernelGGL(eq_columns, dim3(nb), dim3(256), 0, st, k32b, ordB, ne, gx, gy, lab);
-    b = sb;
-    XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, ez, kout, iota, ordA, (int)ne, 0,
-                                                    (int)(sizeof(T) * 8), st));
-    hipLaunchKernelGGL(gather_u32, dim3(nb), dim3(256), 0, st, lab, ordA, ne, k32a);
-    b = sb;
-    XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, k32a, k32b, ordA, ordB, (int)ne, 0,
-                                                    bits_for((uint64_t)gx * gy), st));
-    hipLaunchKernelGGL((gather_xyz<T>), dim3(nb), dim3(256), 0, st, ex, ey, ez, ordB, ne,
-                       sxp + eoff[e], syp + eoff[e], szp + eoff[e]);
-    XS_HIP_CHECK(hipGetLastError());
-    equal_count_tiles(eoff[e], ne, gx, gy, nz, sizeof(T) == 8, tiles);
-    en[e] = (uint32_t)tiles.size() - ebase[e];
-  }
-  return XS_OK;
-}
-
-
 template <class T>
 static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_count,
                       unsigned n_el, double bin, unsigned nhist, unsigned long long *hist_d,
@@ -1496,39 +1379,52 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
   }
   XS_TRY(check_span(bbox, bin));
 
-  // 2. workspace: sorted coordinates, cell keys, overflow counter, scratch
-  //    of the equal-count sorts
-  uint32_t maxne = 0;
-  for (unsigned e = 0; e < n_el; ++e) maxne = std::max<uint32_t>(maxne, el_count[e]);
-  size_t sortb = 0;
-  const size_t eqb = equal_count ? eq_scratch_bytes<T>(std::max(maxne, 1u), &sortb) : 0;
+  // 2. the equal-count partition, and the workspace: sorted coordinates, cell keys,
+  //    overflow counter, scratch of the ordering
+  const double cap = cell_cap(bin, nhist, wcap);
+  order::Tables ord;
+  std::vector<Tile> tiles;
+  uint32_t ebase[kMaxEl], en[kMaxEl];
+  for (unsigned e = 0; e < n_el && equal_count; ++e) {
+    ebase[e] = (uint32_t)tiles.size();
+    en[e] = 0;
+    if (!el_count[e]) continue;
+    uint32_t gx, gy, nz;
+    choose_equal_count(el_count[e], bbox, cap, sizeof(T) == 8, gx, gy, nz);
+    ord.add(eoff[e], el_count[e], gx, gy, bbox);
+    equal_count_tiles(eoff[e], el_count[e], gx, gy, nz, sizeof(T) == 8, tiles);
+    en[e] = (uint32_t)tiles.size() - ebase[e];
+  }
   const size_t nrec = sizeof(T) == 8 ? 4 * n : 0;  // FP64 J records
   XS_TRY(ensure_workspace(ctx, Carver::need({3 * n * sizeof(T), n * sizeof(uint32_t),
-                                             sizeof(unsigned long long), eqb,
-                                             nrec * sizeof(double)})));
+                                             2 * sizeof(unsigned long long), ord.table_bytes(),
+                                             ord.scratch_bytes(), nrec * sizeof(double)})));
   Carver cv(ctx->ws);
   T *sorted = cv.take<T>(3 * n);
   uint32_t *keys = cv.take<uint32_t>(n);
-  unsigned long long *ovf_own = cv.take<unsigned long long>(1);
-  void *eq_scratch = cv.take<char>(eqb);
+  unsigned long long *ovf_own = cv.take<unsigned long long>(2);  // (and the flag of wide tiles)
+  char *ord_tables = cv.take<char>(ord.table_bytes());
+  char *ord_scratch = cv.take<char>(ord.scratch_bytes());
   double *rec = cv.take<double>(nrec);
   unsigned long long *ovf_d = ovf_user ? ovf_user : ovf_own;
   T *sxp = sorted, *syp = sorted + n, *szp = sorted + 2 * n;
 
-  // 3. tiles.  Equal-count tiles (stable sorts on the device; the tiles
+  // 3. tiles.  Equal-count tiles (the atoms ordered on the device; the tiles
   //    follow from the counts alone) or, as the fallback, a cell grid per
   //    element sized for full tiles (counts read back, tiles on the host;
   //    the counts go through the table buffer, which holds nothing else yet).
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "hist_prep", &ev));
-  const double cap = cell_cap(bin, nhist, wcap);
   std::vector<Grid> grids(n_el);
   std::vector<uint32_t> m_of(n_el), soff(n_el + 1, 0u), start_h;
-  std::vector<Tile> tiles;
-  uint32_t ebase[kMaxEl], en[kMaxEl];
-  if (equal_count)
-    XS_TRY(eq_tiles_device<T>(ctx, xyz, n, el_count, n_el, eoff, bbox, cap, eq_scratch,
-                              std::max(maxne, 1u), sxp, syp, szp, tiles, ebase, en));
+  size_t staged = 0;  // of the pinned memory, by copies that may be under way
+  if (equal_count) {
+    staged = align_up(ord.table_bytes(), 256);
+    XS_TRY(ensure_pinned(ctx, staged));
+    ord.write_tables(static_cast<char *>(ctx->pin));
+    XS_HIP_CHECK(hipMemcpyAsync(ord_tables, ctx->pin, ord.table_bytes(), hipMemcpyHostToDevice, ctx->stream));
+    XS_TRY((order::run<T, T>(ctx, ord, ord_tables, ord_scratch, xyz, xyz + n, xyz + 2 * n, sxp, syp, szp)));
+  }
   for (unsigned e = 0; e < n_el && !equal_count; ++e) {
     const uint32_t ne = el_count[e];
     double cell = first_cell(bbox, ne, cap);
@@ -1581,24 +1477,34 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
   }
   order_items(items, types, tiles, sizeof(T) == 8);
 
-  // 4. tables (exact sizes) in the table buffer; the stream is idle here
-  const size_t sb = start_h.size() * sizeof(uint32_t), tb = tiles.size() * sizeof(Tile),
-               yb = types.size() * sizeof(TypeDesc), ib = items.size() * sizeof(Item),
-               bb = tiles.size() * 6 * sizeof(double);
-  XS_TRY(ensure_aux(ctx, Carver::need({sb, tb, yb, ib, bb})));
-  Carver ca(ctx->aux);
-  uint32_t *start_d = ca.take<uint32_t>(start_h.size());
-  Tile *tiles_d = ca.take<Tile>(tiles.size());
-  TypeDesc *types_d = ca.take<TypeDesc>(types.size());
-  Item *items_d = ca.take<Item>(items.size());
-  double *boxes = ca.take<double>(tiles.size() * 6);
-  if (sb) XS_HIP_CHECK(hipMemcpy(start_d, start_h.data(), sb, hipMemcpyHostToDevice));
-  if (tb) XS_HIP_CHECK(hipMemcpy(tiles_d, tiles.data(), tb, hipMemcpyHostToDevice));
-  XS_HIP_CHECK(hipMemcpy(types_d, types.data(), yb, hipMemcpyHostToDevice));
-  if (ib) XS_HIP_CHECK(hipMemcpy(items_d, items.data(), ib, hipMemcpyHostToDevice));
+  // 4. tables (exact sizes) in the table buffer, in one copy
+  const size_t nbox = tiles.size() * 6;
+  const size_t up = Carver::need({start_h.size() * sizeof(uint32_t), tiles.size() * sizeof(Tile),
+                                  types.size() * sizeof(TypeDesc), items.size() * sizeof(Item)});
+  XS_TRY(ensure_aux(ctx, up + nbox * sizeof(double)));
+  XS_TRY(ensure_pinned(ctx, staged + up + 256));
+  Carver ca(ctx->aux), cp(static_cast<char *>(ctx->pin) + staged);
+  auto table = [&](const auto &v) {
+    using E = typename std::decay_t<decltype(v)>::value_type;
+    E *h = cp.take<E>(v.size());
+    if (!v.empty()) std::memcpy(h, v.data(), v.size() * sizeof(E));
+    return ca.take<E>(v.size());
+  };
+  uint32_t *start_d = table(start_h);
+  Tile *tiles_d = table(tiles);
+  TypeDesc *types_d = table(types);
+  Item *items_d = table(items);
+  XS_HIP_CHECK(hipMemcpyAsync(ctx->aux, static_cast<char *>(ctx->pin) + staged, cp.used,
+                              hipMemcpyHostToDevice, ctx->stream));
+  double *boxes = reinterpret_cast<double *>(static_cast<char *>(ctx->aux) + up);
   const unsigned zb = (unsigned)std::min<size_t>((hsize + 255) / 256, 4096);
   hipLaunchKernelGGL(fill_u64, dim3(std::max(zb, 1u)), dim3(256), 0, ctx->stream, hist_d, hsize);
   hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, ctx->stream, ovf_d, (size_t)1);
+  unsigned long long *wide_d = nullptr;
+  if (equal_count && std::isfinite(cap)) {
+    wide_d = ovf_own + 1;
+    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, ctx->stream, wide_d, (size_t)1);
+  }
   for (unsigned e = 0; e < n_el && !equal_count; ++e)
     if (el_count[e])
       hipLaunchKernelGGL((hist_scatter<T>), dim3((el_count[e] + 255) / 256), dim3(256), 0, ctx->stream,
@@ -1606,19 +1512,17 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
                          keys + eoff[e], start_d + soff[e], sxp, syp, szp);
   if (!tiles.empty())
     hipLaunchKernelGGL((hist_tile_boxes<T>), dim3((unsigned)tiles.size()), dim3(256), 0, ctx->stream,
-                       sxp, syp, szp, tiles_d, boxes);
+                       sxp, syp, szp, tiles_d, boxes, cap, wide_d);
   launch_records<T>(ctx->stream, sxp, syp, szp, tiles_d, boxes, tiles.size(), bin, rec);
   XS_HIP_CHECK(hipGetLastError());
-  if (equal_count && std::isfinite(cap) && !tiles.empty()) {
+  if (wide_d && !tiles.empty()) {
     // equal-count tiles of a structure far from uniform density can be wider
     // than the window allows: then the cell grid instead
-    std::vector<double> bx(tiles.size() * 6);
-    XS_HIP_CHECK(hipMemcpyAsync(bx.data(), boxes, bb, hipMemcpyDeviceToHost, ctx->stream));
+    unsigned long long *wide_h = reinterpret_cast<unsigned long long *>(static_cast<char *>(ctx->pin) + staged +
+                                                                        align_up(cp.used, 256));
+    XS_HIP_CHECK(hipMemcpyAsync(wide_h, wide_d, 8, hipMemcpyDeviceToHost, ctx->stream));
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    bool wide = false;
-    for (size_t t = 0; t < tiles.size() && !wide; ++t)
-      for (int a = 0; a < 3; ++a)
-        if (bx[6 * t + 3 + a] - bx[6 * t + a] > cap) wide = true;
+    const bool wide = *wide_h != 0ull;
     if (wide) {
       XS_TRY(prof_end(ctx, "hist_prep", ev));
       return run_device<T>(ctx, xyz, n, el_count, n_el, bin, nhist, hist_d, ovf_user, quot, false);
@@ -1902,11 +1806,8 @@ static int plan_build(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el, const
 // ---- batch plans from coordinates already on the device ----
 //
 // The same plan as plan_build, tiled on the GPU: every structure's
-// coordinates are gathered into one SoA array, and three stable radix sorts
-// over all atoms of all structures at once order them by (element segment,
-// x), then (slab, y), then (column, z), with 64-bit keys whose high word is
-// the segment / slab / column number and whose low word the order-keeping
-// bits of the coordinate as float.  Slabs and columns hold equal counts, so
+// coordinates are gathered into one SoA array, whose elements (segments) are put
+// in tile order at once (xs_order.hip).  Slabs and columns hold equal counts, so
 // the tiles follow from the counts alone (equal_count_tiles, on the host).
 // A structure whose equal-count tiles come out wider than its window allows
 // (an element that forms a hollow shell) is re-tiled on the host with the
@@ -1914,18 +1815,7 @@ static int plan_build(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el, const
 
 struct SegDev {
   uint32_t start, n;  // atoms [start, start + n) of the concatenated arrays
-  uint32_t gx, slab0;  // its slabs: global numbers slab0 .. slab0 + gx - 1
 };
-struct SlabDev {
-  uint32_t start, n;  // positions of the slab after the x sort
-  uint32_t gy, col0;  // its columns: global numbers col0 .. col0 + gy - 1
-};
-
-// Bits of (float)v whose unsigned order is the order of v.
-__device__ __forceinline__ uint32_t ord_bits(double v) {
-  const uint32_t u = __float_as_uint((float)v);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
 
 // raw[a], raw[N + a], raw[2N + a] = atom a of the concatenation of the
 // structures' own SoA arrays (structure s holds atoms abase[s] .. abase[s+1]).
@@ -1980,75 +1870,8 @@ __global__ void seg_boxes(const double *__restrict__ x, const double *__restrict
   if (threadIdx.x < 6) box[(size_t)blockIdx.x * 6 + threadIdx.x] = any_nan ? NAN : sh[threadIdx.x][0];
 }
 
-// Keys of the first sort: (segment, x), values the atom numbers.
-__global__ void seg_keys(const double *__restrict__ x, const SegDev *__restrict__ segs,
-                         unsigned long long *__restrict__ keys, uint32_t *__restrict__ vals) {
-  const SegDev sg = segs[blockIdx.x];
-  for (uint32_t i = sg.start + threadIdx.x; i < sg.start + sg.n; i += blockDim.x) {
-    keys[i] = ((unsigned long long)blockIdx.x << 32) | ord_bits(x[i]);
-    vals[i] = i;
-  }
-}
-
-// After the (segment, x) sort: the slab of each atom.
-__global__ void slab_labels(const unsigned long long *__restrict__ keys,
-                            const uint32_t *__restrict__ vals, const SegDev *__restrict__ segs,
-                            size_t ntot, uint32_t *__restrict__ lab) {
-  for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < ntot;
-       p += (size_t)gridDim.x * blockDim.x) {
-    const SegDev sg = segs[keys[p] >> 32];
-    lab[vals[p]] = sg.slab0 + equal_part(p - sg.start, sg.n, sg.gx);
-  }
-}
-
-// After the (slab, y) sort: the column of each atom.
-__global__ void col_labels(const unsigned long long *__restrict__ keys,
-                           const uint32_t *__restrict__ vals, const SlabDev *__restrict__ slabs,
-                           size_t ntot, uint32_t *__restrict__ lab) {
-  for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < ntot;
-       p += (size_t)gridDim.x * blockDim.x) {
-    const SlabDev sb = slabs[keys[p] >> 32];
-    lab[vals[p]] = sb.col0 + equal_part(p - sb.start, sb.n, sb.gy);
-  }
-}
-
-// Keys (label, coordinate) of the second and third sorts.
-__global__ void label_keys(const double *__restrict__ c, const uint32_t *__restrict__ lab,
-                           size_t ntot, unsigned long long *__restrict__ keys,
-                           uint32_t *__restrict__ vals) {
-  for (size_t a = blockIdx.x * (size_t)blockDim.x + threadIdx.x; a < ntot;
-       a += (size_t)gridDim.x * blockDim.x) {
-    keys[a] = ((unsigned long long)lab[a] << 32) | ord_bits(c[a]);
-    vals[a] = (uint32_t)a;
-  }
-}
-
-// The plan's coordinates in the final order (as T).
-template <class T>
-__global__ void gather_sorted(const double *__restrict__ raw, const uint32_t *__restrict__ ord,
-                              size_t ntot, size_t nc, T *__restrict__ out) {
-  for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < ntot;
-       p += (size_t)gridDim.x * blockDim.x) {
-    const uint32_t a = ord[p];
-    out[p] = (T)raw[a];
-    out[nc + p] = (T)raw[ntot + a];
-    out[2 * nc + p] = (T)raw[2 * ntot + a];
-  }
-}
-
 static unsigned grid_for(size_t n) {
   return (unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 16384));
-}
-
-// One stable sort of (key, value) pairs over all atoms on the low `bits`
-// key bits (scratch from tmp, sized by the caller).
-static int sort_u64(xs_ctx *ctx, void *tmp, size_t tmp_bytes, const unsigned long long *kin,
-                    unsigned long long *kout, const uint32_t *vin, uint32_t *vout, size_t n,
-                    int bits) {
-  size_t b = tmp_bytes;
-  XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, b, kin, kout, vin, vout, (int)n, 0, bits,
-                                                  ctx->stream));
-  return XS_OK;
 }
 
 template <class T>
@@ -2080,7 +1903,7 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
   for (unsigned s = 0, g = 0; s < nstruct; ++s) {
     uint32_t o = (uint32_t)abase[s];
     for (unsigned e = 0; e < n_el[s]; ++e, ++g) {
-      segs[g] = SegDev{o, el_count[ecf[s] + e], 1u, 0u};
+      segs[g] = SegDev{o, el_count[ecf[s] + e]};
       o += el_count[ecf[s] + e];
     }
   }
@@ -2111,9 +1934,8 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
   // 3. bin counts, window caps, slabs and columns (host)
   std::vector<uint32_t> nh_of(nstruct);
   std::vector<double> cap_of(nstruct);
-  std::vector<SlabDev> slabs;
-  std::vector<uint32_t> seg_gy(nseg), seg_nz(nseg);
-  uint32_t ncols = 0;
+  order::Tables ord;
+  std::vector<uint32_t> seg_gx(nseg), seg_gy(nseg), seg_nz(nseg);
   for (unsigned s = 0, g = 0; s < nstruct; ++s) {
     double bb[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
     bool nan = false;
@@ -2145,45 +1967,21 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
     for (unsigned e = 0; e < n_el[s]; ++e, ++g) {
       uint32_t gx, gy, nz;
       choose_equal_count(segs[g].n, &sbox[g * 6], cap_of[s], sizeof(T) == 8, gx, gy, nz);
-      segs[g].gx = gx;
-      segs[g].slab0 = (uint32_t)slabs.size();
+      seg_gx[g] = gx;
       seg_gy[g] = gy;
       seg_nz[g] = nz;
-      for (uint64_t sl = 0; sl < gx; ++sl) {
-        const uint32_t a0 = (uint32_t)(sl * segs[g].n / gx), a1 = (uint32_t)((sl + 1) * segs[g].n / gx);
-        slabs.push_back(SlabDev{segs[g].start + a0, a1 - a0, gy, ncols});
-        ncols += gy;
-      }
+      if (segs[g].n) ord.add(segs[g].start, segs[g].n, gx, gy, &sbox[g * 6]);
     }
   }
 
-  // 4. the three sorts (device)
-  DevMem slabd, keys, vals, lab, tmp;
-  size_t tb = 0;
-  XS_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (const unsigned long long *)nullptr,
-                                                  (unsigned long long *)nullptr,
-                                                  (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                                  (int)ntot, 0, 64, st));
-  XS_TRY(slabd.alloc(std::max<size_t>(slabs.size(), 1) * sizeof(SlabDev), "batch slabs"));
-  XS_TRY(keys.alloc(2 * ntot * 8, "batch sort keys"));
-  XS_TRY(vals.alloc(2 * ntot * 4, "batch sort values"));
-  XS_TRY(lab.alloc(ntot * 4, "batch labels"));
-  XS_TRY(tmp.alloc(tb, "batch sort scratch"));
-  XS_HIP_CHECK(hipMemcpy(segd.p, segs.data(), nseg * sizeof(SegDev), hipMemcpyHostToDevice));
-  XS_HIP_CHECK(hipMemcpy(slabd.p, slabs.data(), slabs.size() * sizeof(SlabDev), hipMemcpyHostToDevice));
-  unsigned long long *k0 = keys.at<unsigned long long>(), *k1 = k0 + ntot;
-  uint32_t *v0 = vals.at<uint32_t>(), *v1 = v0 + ntot, *lb = lab.at<uint32_t>();
-  hipLaunchKernelGGL(seg_keys, dim3((unsigned)nseg), dim3(256), 0, st, rx, segd.at<SegDev>(), k0, v0);
-  XS_TRY(sort_u64(ctx, tmp.p, tb, k0, k1, v0, v1, ntot, 32 + bits_for(nseg)));
-  hipLaunchKernelGGL(slab_labels, dim3(grid_for(ntot)), dim3(256), 0, st, k1, v1, segd.at<SegDev>(),
-                     ntot, lb);
-  hipLaunchKernelGGL(label_keys, dim3(grid_for(ntot)), dim3(256), 0, st, ry, lb, ntot, k0, v0);
-  XS_TRY(sort_u64(ctx, tmp.p, tb, k0, k1, v0, v1, ntot, 32 + bits_for(slabs.size())));
-  hipLaunchKernelGGL(col_labels, dim3(grid_for(ntot)), dim3(256), 0, st, k1, v1, slabd.at<SlabDev>(),
-                     ntot, lb);
-  hipLaunchKernelGGL(label_keys, dim3(grid_for(ntot)), dim3(256), 0, st, rz, lb, ntot, k0, v0);
-  XS_TRY(sort_u64(ctx, tmp.p, tb, k0, k1, v0, v1, ntot, 32 + bits_for(std::max(ncols, 1u))));
-  XS_HIP_CHECK(hipGetLastError());
+  // 4. scratch and tables of the ordering
+  DevMem ordd;
+  XS_TRY(ordd.alloc(align_up(ord.table_bytes(), 256) + ord.scratch_bytes(), "batch ordering"));
+  {
+    std::vector<char> t(ord.table_bytes());
+    ord.write_tables(t.data());
+    XS_HIP_CHECK(hipMemcpy(ordd.p, t.data(), t.size(), hipMemcpyHostToDevice));
+  }
 
   // 5. the plan: sorted coordinates, equal-count tiles and their boxes
   auto *b = new xs_batch();
@@ -2200,7 +1998,7 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
     tile0[s] = (uint32_t)tiles.size();
     for (unsigned e = 0; e < n_el[s]; ++e, ++g) {
       ebase_all[g] = (uint32_t)tiles.size();
-      equal_count_tiles(segs[g].start, segs[g].n, segs[g].gx, seg_gy[g], seg_nz[g], sizeof(T) == 8,
+      equal_count_tiles(segs[g].start, segs[g].n, seg_gx[g], seg_gy[g], seg_nz[g], sizeof(T) == 8,
                         tiles);
       en_all[g] = (uint32_t)tiles.size() - ebase_all[g];
     }
@@ -2213,8 +2011,9 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
     return fail(XS_ERR_NOMEM, "xs_batch_plan: device allocation failed");
   }
   T *c = static_cast<T *>(b->coords);
-  hipLaunchKernelGGL((gather_sorted<T>), dim3(grid_for(ntot)), dim3(256), 0, st, rx, v1, ntot, nc, c);
-  int rc = tiled.alloc(std::max<size_t>(tiles.size(), 1) * sizeof(Tile), "batch tiles");
+  int rc = order::run<double, T>(ctx, ord, ordd.at<char>(), ordd.at<char>(align_up(ord.table_bytes(), 256)), rx,
+                                 ry, rz, c, c + nc, c + 2 * nc);
+  if (rc == XS_OK) rc = tiled.alloc(std::max<size_t>(tiles.size(), 1) * sizeof(Tile), "batch tiles");
   if (rc == XS_OK) rc = boxes_d.alloc(std::max<size_t>(tiles.size(), 1) * 48, "batch tile boxes");
   if (rc != XS_OK) {
     free_plan(b);
@@ -2224,7 +2023,7 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
   hipError_t e = hipMemcpy(tiled.p, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL((hist_tile_boxes<T>), dim3((unsigned)tiles.size()), dim3(256), 0, st, c, c + nc,
-                       c + 2 * nc, tiled.at<Tile>(), boxes_d.at<double>());
+                       c + 2 * nc, tiled.at<Tile>(), boxes_d.at<double>(), INFINITY, nullptr);
     e = hipMemcpyAsync(boxes.data(), boxes_d.p, boxes.size() * 8, hipMemcpyDeviceToHost, st);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -335,6 +335,28 @@ __device__ __forceinline__ float sqrt_rn_f32(float s) {
   return r;
 }
 
+// The same root by one Newton step from v_rsq_f32 (Markstein's form: g = s y, g +
+// (s - g^2) y / 2): a hardware operation and four FP32 ones, where sqrt_rn_f32 takes
+// eight after its own.  Not proven to round correctly for every s, so taken only where
+// sqrt_f32_check_kernel has found no s that it gets wrong.  150,000 atoms in 3 elements:
+// 5.20 ms (with sqrt_rn_f32 5.94); the kernel is bound by VALU issue, ~60 cycles of a
+// SIMD for 64 pairs, of which the LDS atomic takes 25 beside it.  s = 0 and denormal s give
+// NaN, which bin_f32 puts into bin 0 where they belong.
+__device__ __forceinline__ float sqrt_newton_f32(float s) {
+#pragma clang fp contract(off)
+  const float y = __builtin_amdgcn_rsqf(s);
+  const float g = s * y;
+  return fmaf(fmaf(-g, g, s), 0.5f * y, g);
+}
+
+// floor(t) for t >= 0, 0 for NaN, the largest integer beyond the range: what the
+// instruction does, where the language leaves a NaN open.
+__device__ __forceinline__ uint32_t bin_f32(float t) {
+  uint32_t k;
+  __asm__("v_cvt_u32_f32 %0, %1" : "=v"(k) : "v"(t));
+  return k;
+}
+
 // sqrtf(s) / bin in IEEE single precision (before the conversion to a bin).
 __device__ __forceinline__ float dist_over_bin_f32(float s, double inv_bin) {
   return (float)((double)sqrt_rn_f32(s) * inv_bin);
@@ -381,11 +403,12 @@ __global__ void quot_f32_check_kernel(float bin, double inv_bin, unsigned long l
 // have 25 significant bits and y >= 2^-75, so m+-^2 is exact in double and
 // the test is exact.  bad[0] counts wrong roots for s >= 2^-96; bad[1] counts
 // s < 2^-96 whose result is not in [0, 2^-47); bad[2] wrong roots for
-// s < 2^-96.  The FP32 binning relies on bad[0] = bad[1] = 0 and, unless
+// s < 2^-96; bad[3] counts s where sqrt_newton_f32 differs from the IEEE root (from
+// 2^-96 up) or is neither in [0, 2^-47) nor NaN (below).  The FP32 binning relies on bad[0] = bad[1] = 0 and, unless
 // bad[2] = 0 too, on bins of at least 2^-40 (then every s < 2^-96 bins to 0
 // with the IEEE root and with sqrt_rn_f32 alike).
 __global__ void sqrt_f32_check_kernel(unsigned long long *bad) {
-  unsigned long long b0 = 0, b1 = 0, b2 = 0;
+  unsigned long long b0 = 0, b1 = 0, b2 = 0, b3 = 0;
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t u = 1u + blockIdx.x * blockDim.x + threadIdx.x; u < 0x7f800000u; u += stride) {
     const float s = __uint_as_float(u);
@@ -398,9 +421,12 @@ __global__ void sqrt_f32_check_kernel(unsigned long long *bad) {
       const double hi = 0.5 * (yd + (double)__uint_as_float(yb + 1u));
       ok = lo * lo < (double)s && (double)s < hi * hi;
     }
+    const float w = sqrt_newton_f32(s);
     if (u >= 0x0f800000u) {  // s >= 2^-96
       b0 += !ok;
+      b3 += !ok || w != y;
     } else {
+      b3 += w < 0.0f || w >= 0x1p-47f;
       b1 += !(y >= 0.0f && y < 0x1p-47f);
       b2 += !ok;
     }
@@ -408,6 +434,7 @@ __global__ void sqrt_f32_check_kernel(unsigned long long *bad) {
   if (b0) atomicAdd(&bad[0], b0);
   if (b1) atomicAdd(&bad[1], b1);
   if (b2) atomicAdd(&bad[2], b2);
+  if (b3) atomicAdd(&bad[3], b3);
 }
 
 __device__ __forceinline__ uint32_t bin_index_f32(float s, double inv_bin, uint32_t nhist) {
@@ -471,8 +498,8 @@ __device__ __forceinline__ double tile_band(const double *bi, double band0, doub
 
 // FP32 groups of 8 J atoms (not the like-element diagonal tile): the
 // reference GPU expression for 8 independent pairs, no per-pair branch.
-// FQ: the quotient by bin as quot_f32 (yb = recip_f32(bin)), else as the
-// rounded double product.
+// FQ: the root as sqrt_newton_f32 and the quotient by bin as quot_f32 (yb =
+// recip_f32(bin)), else as sqrt_rn_f32 and the rounded double product.
 // SAFE: the J tile's bin range lies inside the window and below nhist
 // (kl >= B, ku < B + WCAP, ku < nhist from the tile boxes) and maps to slots
 // without a wrap, so every pair goes to slot k + off unchecked; otherwise
@@ -497,7 +524,7 @@ __device__ __forceinline__ void pair_group8_f32(float xi, float yi, float zi, co
       // no clamp: a bin at or past nhist (t >= nhist, converted with
       // saturation) goes to the overflow counter below either way
       if constexpr (FQ)
-        k[p] = (uint32_t)quot_f32(sqrt_rn_f32(s), bin, yb);
+        k[p] = bin_f32(quot_f32(sqrt_newton_f32(s), bin, yb));
       else
         k[p] = (uint32_t)dist_over_bin_f32(s, inv_bin);
     }
@@ -1307,10 +1334,11 @@ static int sqrt_f32_checked(xs_ctx *ctx, double bin) {
     hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, ctx->stream, ctx->quot_check, (size_t)4);
     hipLaunchKernelGGL(sqrt_f32_check_kernel, dim3(8192), dim3(256), 0, ctx->stream, ctx->quot_check);
     XS_HIP_CHECK(hipGetLastError());
-    XS_HIP_CHECK(hipMemcpyAsync(ctx->pin, ctx->quot_check, 24, hipMemcpyDeviceToHost, ctx->stream));
+    XS_HIP_CHECK(hipMemcpyAsync(ctx->pin, ctx->quot_check, 32, hipMemcpyDeviceToHost, ctx->stream));
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     const auto *bad = static_cast<const unsigned long long *>(ctx->pin);
     ctx->sqrt_f32_state = (bad[0] || bad[1]) ? 0 : (bad[2] ? 2 : 1);
+    ctx->newton_f32_ok = bad[3] == 0;
   }
   if (ctx->sqrt_f32_state == 0)
     return fail(XS_ERR_DEVICE, "FP32 binning: this device's v_sqrt_f32 fails the exhaustive check "
@@ -1320,12 +1348,13 @@ static int sqrt_f32_checked(xs_ctx *ctx, double bin) {
   return XS_OK;
 }
 
-// Whether FP32 binning may take quot_f32 for this bin: quot_f32_check_kernel
+// Whether FP32 binning may take quot_f32 (and sqrt_newton_f32) for this bin: quot_f32_check_kernel
 // over all 2^23 significands, once per bin and context (synchronises).
 static int quot_f32_exact(xs_ctx *ctx, double bin_d, bool *ok) {
   *ok = false;
   const float bin = (float)bin_d;
-  if (!(bin >= 0x1p-60f && bin <= 0x1p60f)) return XS_OK;
+  // (sqrt_newton_f32 comes with it, whose roots below 2^-48 must be bin 0)
+  if (!ctx->newton_f32_ok || !(bin >= 0x1p-40f && bin <= 0x1p60f)) return XS_OK;
   uint32_t key;
   std::memcpy(&key, &bin, sizeof key);
   const auto it = ctx->quot_f32_ok.find(key);

@@ -137,6 +137,7 @@ struct xs_ctx {
   // allocated on first use).
   std::map<uint32_t, bool> quot_f32_ok;
   int sqrt_f32_state = -1;
+  bool newton_f32_ok = false;
   unsigned long long *quot_check = nullptr;
 
   bool profiling = false;

@@ -26,18 +26,20 @@
 // 8i + 4 (l / 32) + jj, column l % 32.
 //
 // Work groups: 4 waves stacked along q (128 q) x 1 or 2 side by side of NT tiles
-// of 32 columns; tiles are ordered so that the work groups that share a q block
-// run on the same XCD (consecutive work-group ids go to different XCDs).  Few work
-// groups, or a last round of them half empty, share out the k range.
+// of 32 columns, in equal shares of all k tiles; work groups with consecutive
+// shares run on the same XCD (consecutive work-group ids go to different XCDs).
 //
-// Ensembles (pairsum_mfma_batch): the columns are the pair types of many
-// structures, each with its own bin count.  They come sorted and grouped by
-// xs_mfma_plan.h; each group of NT column tiles has its own k range and
-// count slices, one launch covers the groups of one slice count, and the
-// columns' results go to their pair types' rows of S.  The slice count of a
-// type comes from its pair count, so nothing is read back.
+// The columns (the histograms of a call, or in pairsum_mfma_batch the pair types of
+// many structures) come sorted and grouped by xs_mfma_plan.h; each group has its own
+// k range and count slices, one launch covers the groups of one slice count, and the
+// columns' results go to their rows of S.  In an ensemble a column's extent is its
+// structure's bin count and its slices come from its pair count, so nothing is read
+// back; in a call of its own both are read off the counts, while the slices of the
+// sine are made.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <vector>
 
 #include "xs_internal.h"
 #include "xs_sincos.h"
@@ -49,31 +51,50 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kNA = kMfmaSlicesA;        // sinc slices
-constexpr int kMaxNB = kMfmaMaxSlicesB;  // count slices (counts < 2^35)
 constexpr unsigned kFlush = 1024;  // k tiles (of 32 bins) per int32 accumulation
 constexpr double kPi = 3.14159265358979323846;
 
-// All counts or-ed together: as many 7-bit slices as the largest.  A work group adds
-// its word only where that brings a new bit (an atomic per wave, 8,192 on one address,
-// was 97 us for 12.6 M counts, whose 100 MB of loads take 20; now 21).
-__global__ __launch_bounds__(256) void or_u64(const unsigned long long *__restrict__ h, size_t n,
-                                              unsigned long long *__restrict__ out) {
-  unsigned long long m = 0;
-  const size_t step = (size_t)gridDim.x * blockDim.x;
-  size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  for (; i + 3 * step < n; i += 4 * step)
-    m |= (h[i] | h[i + step]) | (h[i + 2 * step] | h[i + 3 * step]);
-  for (; i < n; i += step) m |= h[i];
-  for (int o = 32; o > 0; o >>= 1) m |= (unsigned long long)__shfl_xor(m, o);
-  __shared__ unsigned long long part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x) return;
-  m = (part[0] | part[1]) | (part[2] | part[3]);
-  if (m & ~__hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(out, m);
+__global__ __launch_bounds__(256) void clear_u32(uint32_t *__restrict__ p, size_t n) {
+  const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
 }
 
-__global__ void zero_u64(unsigned long long *p) { *p = 0ull; }
+// Every column's counts or-ed together (as many 7-bit slices as the largest) and one
+// past its last bin that is not empty.  Grid (columns, parts of the bins).  One atomic
+// each per work group: a single word for all columns, an atomic per wave, was 97 us
+// for 12.6 M counts, whose 100 MB of loads take 20; this takes 20.
+__global__ __launch_bounds__(256) void column_stats(const unsigned long long *__restrict__ hist,
+                                                    unsigned nhist,
+                                                    unsigned long long *__restrict__ bits,
+                                                    uint32_t *__restrict__ last) {
+  const unsigned k0 = (unsigned)((unsigned long long)nhist * blockIdx.y / gridDim.y);
+  const unsigned k1 = (unsigned)((unsigned long long)nhist * (blockIdx.y + 1) / gridDim.y);
+  const unsigned long long *h = hist + (size_t)blockIdx.x * nhist;
+  unsigned long long m = 0;
+  uint32_t l = 0;
+#pragma unroll 4
+  for (unsigned k = k0 + threadIdx.x; k < k1; k += 256) {
+    const unsigned long long v = h[k];
+    m |= v;
+    l = v ? k + 1 : l;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    m |= (unsigned long long)__shfl_xor(m, o);
+    l = max(l, (uint32_t)__shfl_xor(l, o));
+  }
+  __shared__ unsigned long long pm[4];
+  __shared__ uint32_t pl[4];
+  if ((threadIdx.x & 63) == 0) {
+    pm[threadIdx.x >> 6] = m;
+    pl[threadIdx.x >> 6] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  l = max(max(pl[0], pl[1]), max(pl[2], pl[3]));
+  if (!l) return;
+  atomicOr(&bits[blockIdx.x], (pm[0] | pm[1]) | (pm[2] | pm[3]));
+  atomicMax(&last[blockIdx.x], l);
+}
 
 // Slices of the sine table: one thread per (q tile, kSincTiles k tiles, lane), 16
 // values a k tile, NA slices of 16 bytes.
@@ -164,46 +185,18 @@ static void launch_slice_sinc(xs_ctx *ctx, const double *q, unsigned nq, unsigne
                      nq, nhist, bin, MT, KT, As);
 }
 
-// One thread per (column tile, k tile, lane): 16 counts, NB 7-bit slices.  S, if
-// given, is cleared.
-__global__ void slice_counts(const unsigned long long *__restrict__ hist, unsigned ncols,
-                             unsigned nhist, unsigned NTn, unsigned KT, int nb,
-                             v4i *__restrict__ Bs, double *__restrict__ S, size_t ssize) {
-  const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (S)
-    for (size_t i = tid; i < ssize; i += (size_t)gridDim.x * blockDim.x) S[i] = 0.0;
-  const size_t total = (size_t)NTn * KT * 64;
-  if (tid >= total) return;
-  const unsigned lane = tid & 63;
-  const size_t tile = tid >> 6;
-  const unsigned kt = tile % KT;
-  const unsigned nt = tile / KT;
-  const unsigned col = nt * 32 + (lane & 31);
-  const unsigned k0 = kt * 32 + 16 * (lane >> 5);
-  unsigned long long cnt[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j)
-    cnt[j] = (col < ncols && k0 + j < nhist) ? hist[(size_t)col * nhist + k0 + j] : 0ull;
-  for (int s = 0; s < nb; ++s) {
-    int8_t b[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) b[j] = (int8_t)((cnt[j] >> (7 * s)) & 127ull);
-    v4i w;
-    __builtin_memcpy(&w, b, 16);
-    Bs[(size_t)s * total + tid] = w;
-  }
-}
-
-// Counts of an ensemble's pair types: one thread per (group, column tile t
-// of the group, k tile below kt_max, lane); threads past their group's k
-// range return.  Group g's slices go to b_off in the layout [nb][NT][kt][64];
-// columns past ncols and bins past a column's nhist are zero.
-__global__ void slice_counts_batch(const unsigned long long *__restrict__ hist,
+// Counts in slices: one thread per (group, column tile t of the group's NT, k tile
+// below kt_max, lane); threads past their group's k range return.  Group g's slices
+// go to b_off in the layout [nb][NT][kt][64]; columns past ncols and bins past a
+// column's nhist are zero.  S, if given, is cleared.
+__global__ void slice_counts(const unsigned long long *__restrict__ hist,
                                    const MfmaCol *__restrict__ cols, unsigned ncols,
                                    const MfmaTile *__restrict__ tiles, unsigned tile0,
                                    unsigned ntiles, unsigned kt_max, int nb, int NT,
-                                   v4i *__restrict__ Bs) {
+                                   v4i *__restrict__ Bs, double *__restrict__ S, size_t ssize) {
   const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (S)
+    for (size_t i = tid; i < ssize; i += (size_t)gridDim.x * blockDim.x) S[i] = 0.0;
   const size_t per_t = (size_t)kt_max * 64, per_group = per_t * NT;
   if (tid >= per_group * ntiles) return;
   const unsigned g = (unsigned)(tid / per_group);
@@ -230,20 +223,28 @@ __global__ void slice_counts_batch(const unsigned long long *__restrict__ hist,
   }
 }
 
+// The same value in every lane, in scalar registers (a 64-bit division leaves it in
+// vector registers, of which the products have none to spare).
+__device__ __forceinline__ unsigned uniform(unsigned v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
+  return (unsigned long long)uniform((unsigned)(v >> 32)) << 32 | uniform((unsigned)v);
+}
+
 // The product.  A work group is 4 waves stacked along q (4 x 32 q) by WN side by
 // side, of NT column tiles each.  Per k tile it needs 4 NA A tiles and NB NT WN B
 // tiles, 1 KiB each in the pre-tiled layout, so a global_load_lds_dwordx4 of one
 // wave writes exactly one tile (lane l's 16 bytes at 16 l).  The tiles go through
-// three LDS stages: those of k tile kt + 2 are fetched while the products of kt
+// NS LDS stages: those of k tile kt + NS - 1 are fetched while the products of kt
 // run, and the products read their operands from LDS (ds_read_b128 at 16 l, no
 // bank conflicts).  Each tile is fetched once per work group, tile b by wave
 // b mod (4 WN), which costs one barrier per k tile: before it, each wave waits
 // for its own loads of stage kt (vmcnt) and for its own reads of stage
 // kt - 1 (lgkmcnt); after it, stage kt is complete in LDS and stage kt - 1,
-// which is refilled next with k tile kt + 2, is read by no wave.
-// The int32 accumulators go to S (FP64) every kFlush k tiles; a wave owns
-// its output elements, so the first flush stores and later ones add, or, with
-// the k range in shares (grid y), all add to the cleared S.
+// which is refilled next with k tile kt + NS - 1, is read by no wave.
+// The int32 accumulators go to S (FP64) every kFlush k tiles.  There are as many
+// work groups as run at a time, and each takes an equal share of all k tiles: a
+// wave owns the output of a group that lies in its share as a whole (the first
+// flush stores, later ones add); those that are cut are added to the cleared S.
 //
 // Measured on the 768-histogram workload (768 x 16,384 bins x 8,192 q):
 // operands loaded straight into registers kept the MFMA pipe busy 35% of
@@ -251,23 +252,26 @@ __global__ void slice_counts_batch(const unsigned long long *__restrict__ hist,
 // registers for a prefetch); per-wave LDS stages one k tile ahead, with
 // every wave fetching its own copy of the B tiles (9 KiB per wave per k
 // tile), 50%.  Two waves side by side (WN = 2) load 14 KiB instead of 24 for the
-// products of four waves: whole call with counts of one, two and three slices
-// 916, 1,272 and 1,607 us (1,033, 1,397, 1,743 with WN = 1).
+// products of four waves.  A work group per group and 128 q left CUs idle 40% of the
+// time with two slices (a round and a quarter of work groups of unequal length): 530
+// us for the products, 400 in equal shares.  Particles of 500 to 8,000 atoms leave a
+// third of the bins empty past each column's last, and half of the columns take one
+// slice: as columns of one k range and slice count the products took 790.
 //
-// BATCH: the column tiles come in groups of NT with their own k range and
-// slices (tiles[tile0 + group]: the count slices at b_off, laid out
-// [NB][NT][kt][64]), A is laid out with KT = the largest k range, and the
-// columns go to the rows of S that cols[] names.  Otherwise all columns
-// share KT and B is laid out [NB][NTn][KT][64].
-template <int NA, int NB, int NT, int WN, bool BATCH>
+// The column tiles come in groups of NT WN with their own k range and slices
+// (tiles[tile0 + group]: the count slices at b_off, laid out [NB][NT WN][kt][64]);
+// A is laid out with KT, at least the largest k range, and the columns go to the
+// rows of S that cols[] names.
+template <int NA, int NB, int NT, int WN>
 __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i *__restrict__ As,
                                                                 const v4i *__restrict__ Bs,
-                                                                unsigned MT, unsigned NTn, unsigned KT,
+                                                                unsigned MT, unsigned ngrp, unsigned KT,
                                                                 unsigned nq, unsigned ncols,
                                                                 double *__restrict__ S,
                                                                 const MfmaTile *__restrict__ tiles,
                                                                 const MfmaCol *__restrict__ cols,
-                                                                unsigned tile0) {
+                                                                unsigned tile0, const double *__restrict__ q,
+                                                                double bin) {
   constexpr int DMIN = -(NA - 1);
   constexpr int DMAX = NB - 1;
   constexpr int NG = DMAX - DMIN + 1;
@@ -275,53 +279,18 @@ __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i
   constexpr int TPS = 4 * NA + NBT;    // tiles per stage
   constexpr int NW = 4 * WN;           // waves
   constexpr int NL = (TPS + NW - 1) / NW;  // of which a wave fetches at most NL
-  constexpr int NS = 3;                // stages
-  // loads per stage that every wave issues at least (the first waves issue one
-  // more; waiting for this count still covers their older stage)
-  constexpr int VM = TPS / NW;
-  static_assert(VM <= 15, "vmcnt field");
+  constexpr int NS = WN == 2 ? 5 : 3;  // stages (one work group a CU, or two)
+  // loads per stage that every wave issues at least (without the top slices; some
+  // waves issue one or two more: waiting for this count still covers their older stage)
+  constexpr int VM = (TPS - 4) / NW;
+  constexpr int WAIT = VM * (NS - 2);
+  static_assert(WAIT <= 15, "vmcnt field");
   __shared__ v4i stage[NS][TPS][64];
   const unsigned lane = threadIdx.x & 63;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned wm = wave % 4, wn = wave / 4;
-  const unsigned ngrp = NTn / (NT * WN);
-  unsigned tile = blockIdx.x;
-  if ((gridDim.x & 7u) == 0) tile = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const unsigned mg = tile / ngrp, ng = tile % ngrp;
-  const unsigned mt = mg * 4 + wm;
-  // this group's k tiles, B slice stride, B column-tile stride, B base
-  unsigned KTg = KT;
-  size_t sB = (size_t)NTn * KT * 64, tB = (size_t)KT * 64;
-  const v4i *bp = Bs + (size_t)ng * NT * WN * KT * 64;
-  unsigned col0 = (ng * WN + wn) * NT * 32, colend = ncols;
-  if constexpr (BATCH) {
-    static_assert(!BATCH || WN == 1, "a batch's groups are NT column tiles");
-    const MfmaTile d = tiles[tile0 + ng];
-    KTg = d.kt;
-    sB = (size_t)NT * d.kt * 64;
-    tB = (size_t)d.kt * 64;
-    bp = Bs + d.b_off;
-    col0 = d.col0;
-    colend = min(ncols, d.col0 + d.ncol);
-  }
   typedef __attribute__((address_space(3))) void lds_t;
 
-  // the tiles of a stage go round the waves: the A tiles (q tile m, slice i) as
-  // m NA + i, then the B tiles (slice j, column tile t) as 4 NA + j NT WN + t
-  const v4i *src[NL];
-#pragma unroll
-  for (int l = 0; l < NL; ++l) {
-    const int b = l * NW + (int)wave, c = b - 4 * NA;
-    src[l] = c < 0 ? As + ((size_t)(b % NA) * MT + mg * 4 + b / NA) * KT * 64
-                   : bp + (size_t)(c / (NT * WN)) * sB + (size_t)(c % (NT * WN)) * tB;
-  }
-  auto fetch = [&](unsigned kt, int st) {
-#pragma unroll
-    for (int l = 0; l < NL; ++l)
-      if (l < TPS / NW || l * NW + (int)wave < TPS)
-        __builtin_amdgcn_global_load_lds((const void *)(src[l] + (size_t)kt * 64 + lane),
-                                         (lds_t *)&stage[st][l * NW + wave][0], 16, 0, 0);
-  };
   // all waves: own LDS reads done, then the barrier; the empty asm keeps the
   // compiler from moving LDS accesses across it
   auto sync_lds = [&]() {
@@ -331,145 +300,224 @@ __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i
     __asm__ volatile("" ::: "memory");
   };
 
-  // this share's k tiles
-  const unsigned kfirst = (unsigned)((unsigned long long)KTg * blockIdx.y / gridDim.y);
-  const unsigned klast = (unsigned)((unsigned long long)KTg * (blockIdx.y + 1) / gridDim.y);
-  for (unsigned kb = kfirst; kb < klast; kb += kFlush) {
-    const unsigned ke = min(klast, kb + kFlush);
-    v16i acc[NG][NT];
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[g][t] = v16i{0};
-    // no wave still reads a stage of the previous block
-    sync_lds();
-    fetch(kb, 0);
-    if (kb + 1 < ke) fetch(kb + 1, 1);
-    int st = 0;
-    for (unsigned kt = kb; kt < ke; ++kt) {
-      if (kt + 1 < ke)
-        __builtin_amdgcn_s_waitcnt(0x0f70 | VM);  // vmcnt(VM): own loads of stage kt landed
+  // This work group's share of all k tiles, in the order (128 q, group, k tile).  A
+  // group's first k tile in that order follows from where its slices begin.
+  constexpr unsigned long long kUnit = (unsigned long long)NB * NT * WN * 64;
+  const unsigned long long b0 = tiles[tile0].b_off;
+  const unsigned long long K =
+      uniform((tiles[tile0 + ngrp - 1].b_off - b0) / kUnit + tiles[tile0 + ngrp - 1].kt);
+  const unsigned long long total = K * (MT / 4);
+  unsigned share = blockIdx.x;
+  if ((gridDim.x & 7u) == 0) share = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  unsigned long long w = uniform(total * share / gridDim.x);
+  const unsigned long long wend = uniform(total * (share + 1) / gridDim.x);
+  unsigned mg = uniform((unsigned)(w / K)), ng = 0;
+  {
+    const unsigned long long r = w - mg * K;
+    unsigned hi = ngrp - 1;
+    while (ng < hi) {
+      const unsigned mid = (ng + hi + 1) / 2;
+      if ((tiles[tile0 + mid].b_off - b0) / kUnit <= r)
+        ng = mid;
       else
-        __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0)
+        hi = mid - 1;
+    }
+  }
+  ng = uniform(ng);
+  unsigned kfirst = uniform((unsigned)(w - mg * K - (tiles[tile0 + ng].b_off - b0) / kUnit));
+  while (w < wend) {
+    const unsigned mt = mg * 4 + wm;
+    // this group's k tiles, B slice stride, B column-tile stride, B base
+    const MfmaTile d = tiles[tile0 + ng];
+    const unsigned klast = (unsigned)min((unsigned long long)d.kt, kfirst + (wend - w));
+    const bool whole = kfirst == 0 && klast == d.kt;
+    const size_t sB = (size_t)NT * WN * d.kt * 64, tB = (size_t)d.kt * 64;
+    const v4i *bp = Bs + d.b_off;
+    const unsigned col0 = d.col0 + wn * NT * 32, colend = min(ncols, d.col0 + d.ncol);
+
+    // Where |q| r > 129 for all of a q tile, every value is below 1/128 and its top slice
+    // is 0: no products with it from k tile ktop on, no loads from the largest ktop of the
+    // work group's q tiles on (kfetch).
+    unsigned ktop = 0, kfetch = 0;
+#pragma unroll
+    for (unsigned m = 0; m < 4; ++m) {
+      const unsigned row = (mg * 4 + m) * 32 + (lane & 31);
+      double a = row < nq ? fabs(q[row]) : 0.0;
+      a = a > 0.0 ? a : INFINITY;  // (q = 0: a row of zeros; NaN: as it comes)
+      for (int o = 16; o > 0; o >>= 1) a = fmin(a, __shfl_xor(a, o, 64));
+      const double k = 129.0 / (a * bin) * (1.0 / 32.0) + 1.0;
+      const unsigned kk = __builtin_amdgcn_readfirstlane(k < 4294967295.0 ? (unsigned)k : ~0u);
+      kfetch = max(kfetch, kk);
+      if (m == wm) ktop = kk;
+    }
+    // The tiles of a stage go round the waves: the A tiles (q tile m, slice i > 0) as
+    // m (NA - 1) + i - 1, the B tiles (slice j, column tile t) as kB0 + j NT WN + t, and
+    // last the top slices, kTop0 + m, which are fetched where a wave needs its own.
+    constexpr int kB0 = 4 * (NA - 1), kTop0 = kB0 + NBT;
+    const v4i *src[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const int b = l * NW + (int)wave, c = b - kB0, m = b - kTop0;
+      src[l] = c < 0   ? As + ((size_t)(b % (NA - 1) + 1) * MT + mg * 4 + b / (NA - 1)) * KT * 64
+               : m < 0 ? bp + (size_t)(c / (NT * WN)) * sB + (size_t)(c % (NT * WN)) * tB
+                       : As + ((size_t)mg * 4 + min(m, 3)) * KT * 64;
+    }
+    auto fetch = [&](unsigned kt, int st) {
+      const int tiles_now = kt < kfetch ? TPS : kTop0;
+#pragma unroll
+      for (int l = 0; l < NL; ++l)
+        if (l < VM || l * NW + (int)wave < tiles_now)
+          __builtin_amdgcn_global_load_lds((const void *)(src[l] + (size_t)kt * 64 + lane),
+                                           (lds_t *)&stage[st][l * NW + wave][0], 16, 0, 0);
+    };
+    for (unsigned kb = kfirst; kb < klast; kb += kFlush) {
+      const unsigned ke = min(klast, kb + kFlush);
+      v16i acc[NG][NT];
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[g][t] = v16i{0};
+      // no wave still reads a stage of the previous block
       sync_lds();
-      if (kt + 2 < ke) fetch(kt + 2, st == 0 ? 2 : st - 1);
-      v4i a[NA], b[NB][NT];
 #pragma unroll
-      for (int i = 0; i < NA; ++i) a[i] = stage[st][wm * NA + i][lane];
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) b[j][t] = stage[st][4 * NA + (j * WN + wn) * NT + t][lane];
-#pragma unroll
-      for (int i = 0; i < NA; ++i)
+      for (int i = 0; i < NS - 1; ++i)
+        if (kb + i < ke) fetch(kb + i, i);
+      int st = 0;
+      for (unsigned kt = kb; kt < ke; ++kt) {
+        if (kt + NS - 2 < ke)
+          __builtin_amdgcn_s_waitcnt(0x0f70 | WAIT);  // vmcnt(WAIT): own loads of stage kt landed
+        else
+          __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0)
+        sync_lds();
+        if (kt + NS - 1 < ke) fetch(kt + NS - 1, st == 0 ? NS - 1 : st - 1);
+        // the counts first, then the sine's slices one by one, whose products start as
+        // they arrive
+        v4i a[NA], b[NB][NT];
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
-            acc[j - i - DMIN][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                BATCH ? a[i] : b[j][t], BATCH ? b[j][t] : a[i], acc[j - i - DMIN][t], 0, 0, 0);
-      st = st == 2 ? 0 : st + 1;
-    }
-    auto value = [&](int t, int e) {
-      double v = 0.0;
+          for (int t = 0; t < NT; ++t) b[j][t] = stage[st][kB0 + (j * WN + wn) * NT + t][lane];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int g = 0; g < NG; ++g) v = fma((double)acc[g][t][e], ldexp(1.0, 7 * (g + DMIN) - 6), v);
-      return v;
-    };
-    // opaque, or the addresses would be formed before the loop over kb and kept
-    unsigned stride = nq;
-    __asm__ volatile("" : "+s"(stride));
-    if constexpr (BATCH) {
-      // lane % 32 is a column (one look at its row of S)
+        for (int i = 1; i < NA; ++i) {
+          a[i] = stage[st][wm * (NA - 1) + i - 1][lane];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        auto multiply = [&](int i) {
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[j - i - DMIN][t] =
+                  __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j][t], a[i], acc[j - i - DMIN][t], 0, 0, 0);
+        };
+#pragma unroll
+        for (int i = 1; i < NA; ++i) multiply(i);
+        if (kt < ktop) {
+          a[0] = stage[st][kTop0 + wm][lane];
+          multiply(0);
+        }
+        st = st == NS - 1 ? 0 : st + 1;
+      }
+      // lane % 32 is a q, so that 32 lanes write 32 consecutive ones of a row.  (Stride
+      // and lane are opaque, or addresses would be formed before the loops and kept;
+      // the rows' numbers go round by shuffles, as 32 loads a lane would spill.)
+      unsigned stride = nq, l = lane;
+      __asm__ volatile("" : "+s"(stride), "+v"(l));
+      const unsigned row = mt * 32 + (l & 31), half = 4 * (l >> 5);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const unsigned col = col0 + t * 32 + (lane & 31);
-        if (col >= colend) continue;
-        const unsigned row0 = mt * 32 + 4 * (lane >> 5);
-        double *const o0 = S + (size_t)cols[col].type * stride + row0;
+        const unsigned mine = min(col0 + t * 32 + (l & 31), ncols - 1);
+        uint32_t type = cols[mine].type;
+        __asm__ volatile("" : "+v"(type));
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const unsigned r = 8 * (e >> 2) + (e & 3);
-          if (row0 + r < nq) {
-            const double v = value(t, e);
-            o0[r] = kb == 0 ? v : o0[r] + v;
+          const unsigned c = 8 * (e >> 2) + (e & 3) + half;
+          const size_t srow = (uint32_t)__shfl((int)type, (int)c, 64);
+          double v = 0.0;
+#pragma unroll
+          for (int g = 0; g < NG; ++g) v = fma((double)acc[g][t][e], ldexp(1.0, 7 * (g + DMIN) - 6), v);
+          if (row < nq && col0 + t * 32 + c < colend) {
+            double *o = S + srow * stride + row;
+            if (whole)
+              *o = kb == 0 ? v : *o + v;
+            else
+              atomicAdd(o, v);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-    } else {
-      // lane % 32 is a q, so that 32 lanes write 32 consecutive ones
-      const unsigned row = mt * 32 + (lane & 31), cl = col0 + 4 * (lane >> 5);
-      if (row >= nq) continue;
-      double *const o0 = S + (size_t)cl * stride + row;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const unsigned c = t * 32 + 8 * (e >> 2) + (e & 3);
-          if (cl + c < colend) {
-            const double v = value(t, e);
-            double *o = o0 + (size_t)c * stride;
-            if (gridDim.y > 1)
-              atomicAdd(o, v);
-            else
-              *o = kb == 0 ? v : *o + v;
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
+    }
+    w += klast - kfirst;
+    kfirst = klast;
+    if (klast == d.kt) {
+      kfirst = 0;
+      if (++ng == ngrp) {
+        ng = 0;
+        ++mg;
+      }
     }
   }
 }
 
-template <int NT, int WN, bool BATCH>
-static void launch_gemm(int nb, dim3 grid, hipStream_t st, const v4i *As, const v4i *Bs, unsigned MT,
-                        unsigned NTn, unsigned KT, unsigned nq, unsigned ncols, double *S,
-                        const MfmaTile *tiles = nullptr, const MfmaCol *cols = nullptr,
-                        unsigned tile0 = 0) {
-#define XS_MM_LAUNCH(NBV, NTV)                                                                       \
-  hipLaunchKernelGGL((pairsum_mfma_lds_kernel<kNA, NBV, NTV, WN, BATCH>), grid, dim3(256 * WN), 0, st, \
-                     As, Bs, MT, NTn, KT, nq, ncols, S, tiles, cols, tile0)
-  switch (nb) {
-    case 1:
-      XS_MM_LAUNCH(1, NT);
-      break;
-    case 2:
-      XS_MM_LAUNCH(2, NT);
-      break;
-    case 3:
-      if constexpr (NT == 1) XS_MM_LAUNCH(3, 1);  // three count slices with two column tiles would spill
-      break;
-    default:
-      if constexpr (NT == 1) {
-        if (nb == 4)
-          XS_MM_LAUNCH(4, 1);
-        else
-          XS_MM_LAUNCH(5, 1);
-      }
-      break;
+// The products of one slice count's groups.
+template <int NT, int WN>
+static void launch_gemm(unsigned nb, dim3 grid, hipStream_t st, const v4i *As, const v4i *Bs, unsigned MT,
+                        unsigned ngrp, unsigned KT, unsigned nq, unsigned ncols, double *S,
+                        const MfmaTile *tiles, const MfmaCol *cols, unsigned tile0, const double *q,
+                        double bin) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256 * WN), 0, st, As, Bs, MT, ngrp, KT, nq, ncols, S, tiles, cols,
+                       tile0, q, bin);
+  };
+  if constexpr (NT == 2) {  // three count slices with two column tiles would spill
+    launch(nb == 1 ? pairsum_mfma_lds_kernel<kNA, 1, NT, WN> : pairsum_mfma_lds_kernel<kNA, 2, NT, WN>);
+  } else {
+    launch(nb == 3   ? pairsum_mfma_lds_kernel<kNA, 3, NT, WN>
+           : nb == 4 ? pairsum_mfma_lds_kernel<kNA, 4, NT, WN>
+                     : pairsum_mfma_lds_kernel<kNA, 5, NT, WN>);
   }
-#undef XS_MM_LAUNCH
 }
+
+// Count slices and products of a plan's groups (S is cleared first).
+static int products(xs_ctx *ctx, const MfmaBatchPlan &plan, const unsigned long long *hist,
+                    const MfmaCol *cols, const MfmaTile *tiles, const v4i *As, v4i *Bs, unsigned KT,
+                    double bin, const double *q, unsigned nq, double *S);
 
 }  // namespace mm
 
-// Shares of the k range for `groups` work groups, `slots` of which run at a time: the
-// rounds of work groups that a share takes, and the sums that every share adds to S
-// (3% of the products of 512 k tiles).  Counts of two slices, 16,384 bins x 8,192 q,
-// whole call: 768 histograms, a round and a half, 1,272 us in one share, 1,204 in two,
-// 1,247 in three; 400, one round, 863 in one and 857 in two; 94, a quarter of one, 405
-// in four and 462 in two.
-static unsigned k_shares(unsigned groups, unsigned KT, unsigned slots) {
-  unsigned best = 1;
-  double cost = std::ceil((double)groups / slots);
-  for (unsigned z = 2; z <= 16 && KT / z >= 32; ++z) {
-    const double c = std::ceil((double)groups * z / slots) / z + 15.0 * z * groups / ((double)slots * KT);
-    if (c < cost) {
-      cost = c;
-      best = z;
-    }
+static int mm::products(xs_ctx *ctx, const MfmaBatchPlan &plan, const unsigned long long *hist,
+                        const MfmaCol *cols, const MfmaTile *tiles, const v4i *As, v4i *Bs, unsigned KT,
+                        double bin, const double *q, unsigned nq, double *S) {
+  const unsigned MT = (nq + 127) / 128 * 4, ncols = (unsigned)plan.cols.size();
+  for (const MfmaLaunch &L : plan.launches) {
+    const unsigned NTg = L.nt * L.wn;
+    const size_t tb = (size_t)L.ntiles * NTg * plan.kt_max * 64;
+    hipLaunchKernelGGL(slice_counts, dim3((unsigned)((tb + 255) / 256)), dim3(256), 0, ctx->stream, hist, cols,
+                       ncols, tiles, L.tile0, L.ntiles, plan.kt_max, (int)L.nb, (int)NTg, Bs,
+                       &L == &plan.launches[0] ? S : nullptr, (size_t)ncols * nq);
   }
-  return best;
+  for (const MfmaLaunch &L : plan.launches) {
+    // as many work groups as run at a time, of 16 k tiles at least
+    unsigned long long work = 0;
+    for (uint32_t g = 0; g < L.ntiles; ++g) work += plan.tiles[L.tile0 + g].kt;
+    work *= MT / 4;
+    const unsigned slots = 2 / L.wn * (unsigned)ctx->cu_count;
+    const dim3 grid((unsigned)std::min<unsigned long long>(slots, std::max(1ull, work / 16)));
+    auto gemm = [&](auto launch) {
+      launch(L.nb, grid, ctx->stream, As, Bs, MT, L.ntiles, KT, nq, ncols, S, tiles, cols, L.tile0, q, bin);
+    };
+    if (L.nt == 2 && L.wn == 2)
+      gemm(launch_gemm<2, 2>);
+    else if (L.nt == 2)
+      gemm(launch_gemm<2, 1>);
+    else if (L.wn == 2)
+      gemm(launch_gemm<1, 2>);
+    else
+      gemm(launch_gemm<1, 1>);
+  }
+  XS_HIP_CHECK(hipGetLastError());
+  return XS_OK;
 }
 
 int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, unsigned nhist,
@@ -477,63 +525,54 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   using namespace mm;
   const unsigned MT = (nq + 127) / 128 * 4;
   const unsigned KT = (nhist + 31) / 32;
-  const unsigned NTmax = (ncols + 127) / 128 * 4;  // column tiles for any form
-  const size_t aBytes = (size_t)kNA * MT * KT * 1024, bBytes = (size_t)kMaxNB * NTmax * KT * 1024;
-  XS_TRY(ensure_matrix(ctx, Carver::need({aBytes, bBytes, 8})));
-  XS_TRY(ensure_pinned(ctx, 64));
+  const size_t aBytes = (size_t)kNA * MT * KT * 1024;
+  XS_TRY(ensure_matrix(ctx, Carver::need({aBytes, (size_t)ncols * 8, (size_t)ncols * 4})));
+  XS_TRY(ensure_pinned(ctx, (size_t)ncols * 12));
   Carver cv(ctx->mat);
   v4i *As = cv.take<v4i>(aBytes / 16);
-  v4i *Bs = cv.take<v4i>(bBytes / 16);
-  unsigned long long *mx = cv.take<unsigned long long>(1);
-  // bits of the largest count -> number of count slices (one read back, while the
-  // sine's slices are made)
-  const size_t hn = (size_t)ncols * nhist;
-  hipLaunchKernelGGL(zero_u64, dim3(1), dim3(1), 0, ctx->stream, mx);
-  hipLaunchKernelGGL(or_u64, dim3((unsigned)std::min<size_t>((hn + 1023) / 1024, 1024)), dim3(256), 0,
-                     ctx->stream, hist, hn, mx);
-  XS_HIP_CHECK(hipGetLastError());
-  XS_HIP_CHECK(hipMemcpyAsync(ctx->pin, mx, 8, hipMemcpyDeviceToHost, ctx->stream));
-  if (!ctx->read_back) XS_HIP_CHECK(hipEventCreateWithFlags(&ctx->read_back, hipEventDisableTiming));
-  XS_HIP_CHECK(hipEventRecord(ctx->read_back, ctx->stream));
+  unsigned long long *bits = cv.take<unsigned long long>(ncols);
+  uint32_t *last = cv.take<uint32_t>(ncols);
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "pairsum_slices", &ev));
+  // every column's slices and extent, read back while the sine's slices are made
+  const size_t nclear = (size_t)(last + ncols - reinterpret_cast<uint32_t *>(bits));
+  hipLaunchKernelGGL(clear_u32, dim3((unsigned)((nclear + 255) / 256)), dim3(256), 0, ctx->stream,
+                     reinterpret_cast<uint32_t *>(bits), nclear);
+  hipLaunchKernelGGL(column_stats, dim3(ncols, std::min(64u, (nhist + 4095) / 4096)), dim3(256), 0, ctx->stream,
+                     hist, nhist, bits, last);
+  XS_HIP_CHECK(hipGetLastError());
+  char *const pin = static_cast<char *>(ctx->pin);
+  XS_HIP_CHECK(hipMemcpyAsync(pin, bits, (size_t)ncols * 8, hipMemcpyDeviceToHost, ctx->stream));
+  XS_HIP_CHECK(hipMemcpyAsync(pin + (size_t)ncols * 8, last, (size_t)ncols * 4, hipMemcpyDeviceToHost,
+                              ctx->stream));
+  if (!ctx->read_back) XS_HIP_CHECK(hipEventCreateWithFlags(&ctx->read_back, hipEventDisableTiming));
+  XS_HIP_CHECK(hipEventRecord(ctx->read_back, ctx->stream));
   launch_slice_sinc(ctx, q, nq, nhist, bin, MT, KT, As);
   XS_HIP_CHECK(hipGetLastError());
   XS_HIP_CHECK(hipEventSynchronize(ctx->read_back));
-  const unsigned long long cmax = *static_cast<unsigned long long *>(ctx->pin);
-  int nb = 1;
-  while (nb < kMaxNB && (cmax >> (7 * nb)) != 0ull) ++nb;
-  if ((cmax >> (7 * nb)) != 0ull) {
+  std::vector<unsigned long long> off(ncols), bound(ncols);
+  std::vector<uint32_t> extent(ncols);
+  std::memcpy(bound.data(), pin, (size_t)ncols * 8);
+  std::memcpy(extent.data(), pin + (size_t)ncols * 8, (size_t)ncols * 4);
+  for (unsigned c = 0; c < ncols; ++c) off[c] = (unsigned long long)c * nhist;
+  MfmaBatchPlan plan;
+  if (!mfma_batch_plan(off, extent, bound, nq, &plan, true)) {
     XS_TRY(prof_end(ctx, "pairsum_slices", ev));
     return fail(XS_ERR_RANGE, "xs_hist_pairsum: a bin count exceeds 2^35 (matrix-core path)");
   }
-  // two column tiles per wave unless the accumulators would not fit
-  const int NT = (ncols > 32 && nb <= 2) ? 2 : 1;  // nb = 3 with NT = 2 would spill
-  // two waves side by side where there are columns for both
-  const int WN = ncols > 32u * NT ? 2 : 1;
-  const unsigned NTn = (ncols + 32 * NT * WN - 1) / (32 * NT * WN) * (NT * WN);
-
-  const size_t tb = (size_t)NTn * KT * 64;
-  const unsigned groups = (MT / 4) * (NTn / (NT * WN));
-  const unsigned shares = k_shares(groups, KT, 2 / WN * (unsigned)ctx->cu_count);
-  hipLaunchKernelGGL(slice_counts, dim3((unsigned)((tb + 255) / 256)), dim3(256), 0, ctx->stream, hist,
-                     ncols, nhist, NTn, KT, nb, Bs, shares > 1 ? S : nullptr, (size_t)ncols * nq);
-  XS_HIP_CHECK(hipGetLastError());
+  const size_t colsb = plan.cols.size() * sizeof(MfmaCol), tilesb = plan.tiles.size() * sizeof(MfmaTile);
+  XS_TRY(ensure_aux(ctx, Carver::need({colsb, tilesb, plan.b_bytes})));
+  XS_TRY(ensure_pinned(ctx, align_up(colsb, 256) + tilesb));
+  Carver ca(ctx->aux);
+  MfmaCol *cols = ca.take<MfmaCol>(plan.cols.size());
+  MfmaTile *tiles = ca.take<MfmaTile>(plan.tiles.size());
+  v4i *Bs = ca.take<v4i>(plan.b_bytes / 16);
+  std::memcpy(ctx->pin, plan.cols.data(), colsb);
+  std::memcpy(static_cast<char *>(ctx->pin) + align_up(colsb, 256), plan.tiles.data(), tilesb);
+  XS_HIP_CHECK(hipMemcpyAsync(cols, ctx->pin, align_up(colsb, 256) + tilesb, hipMemcpyHostToDevice, ctx->stream));
   XS_TRY(prof_end(ctx, "pairsum_slices", ev));
   XS_TRY(prof_begin(ctx, "pairsum_mfma", &ev));
-  const dim3 grid(groups, shares);
-  auto gemm = [&](auto launch) {
-    launch(nb, grid, ctx->stream, As, Bs, MT, NTn, KT, nq, ncols, S, nullptr, nullptr, 0u);
-  };
-  if (WN == 2 && NT == 2)
-    gemm(launch_gemm<2, 2, false>);
-  else if (WN == 2)
-    gemm(launch_gemm<1, 2, false>);
-  else if (NT == 2)
-    gemm(launch_gemm<2, 1, false>);
-  else
-    gemm(launch_gemm<1, 1, false>);
-  XS_HIP_CHECK(hipGetLastError());
+  XS_TRY(products(ctx, plan, hist, cols, tiles, As, Bs, KT, bin, q, nq, S));
   XS_TRY(prof_end(ctx, "pairsum_mfma", ev));
   return XS_OK;
 }
@@ -544,26 +583,11 @@ int pairsum_mfma_batch(xs_ctx *ctx, const MfmaBatchPlan &plan, const unsigned lo
   using namespace mm;
   if (nq != plan.nq) return fail(XS_ERR_ARG, "pairsum_mfma_batch: plan made for another nq");
   const unsigned MT = (nq + 127) / 128 * 4;
-  const unsigned KT = plan.kt_max;
-  const unsigned ncols = (unsigned)plan.cols.size();
-  v4i *As = static_cast<v4i *>(a_buf), *Bs = static_cast<v4i *>(b_buf);
   hipEvent_t ev{};
   if (prof) XS_TRY(prof_begin(ctx, "batch_pairsum", &ev));
-  launch_slice_sinc(ctx, q, nq, KT * 32, bin, MT, KT, As);
-  for (const MfmaLaunch &L : plan.launches) {
-    const size_t tb = (size_t)L.ntiles * L.nt * KT * 64;
-    hipLaunchKernelGGL(slice_counts_batch, dim3((unsigned)((tb + 255) / 256)), dim3(256), 0,
-                       ctx->stream, hist, cols_d, ncols, tiles_d, L.tile0, L.ntiles, KT, (int)L.nb,
-                       (int)L.nt, Bs);
-    const dim3 grid((MT / 4) * L.ntiles);
-    if (L.nt == 2)
-      launch_gemm<2, 1, true>((int)L.nb, grid, ctx->stream, As, Bs, MT, L.ntiles * 2, KT, nq, ncols, S,
-                           tiles_d, cols_d, L.tile0);
-    else
-      launch_gemm<1, 1, true>((int)L.nb, grid, ctx->stream, As, Bs, MT, L.ntiles, KT, nq, ncols, S,
-                           tiles_d, cols_d, L.tile0);
-  }
-  XS_HIP_CHECK(hipGetLastError());
+  v4i *As = static_cast<v4i *>(a_buf);
+  launch_slice_sinc(ctx, q, nq, plan.kt_max * 32, bin, MT, plan.kt_max, As);
+  XS_TRY(products(ctx, plan, hist, cols_d, tiles_d, As, static_cast<v4i *>(b_buf), plan.kt_max, bin, q, nq, S));
   if (prof) XS_TRY(prof_end(ctx, "batch_pairsum", ev));
   return XS_OK;
 }

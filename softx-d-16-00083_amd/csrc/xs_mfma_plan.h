@@ -27,7 +27,8 @@ struct MfmaTile {
   uint32_t pad;
 };
 struct MfmaLaunch {
-  uint32_t tile0, ntiles, nb, nt;  // groups [tile0, tile0 + ntiles), slices, tiles per group
+  uint32_t tile0, ntiles, nb, nt;  // groups [tile0, tile0 + ntiles), slices, tiles a wave
+  uint32_t wn;                     // waves side by side: a group has 32 nt wn columns
 };
 struct MfmaBatchPlan {
   std::vector<MfmaCol> cols;
@@ -45,10 +46,13 @@ struct MfmaBatchPlan {
 // would not fit), never columns of the next.  Its slices are laid out
 // [nb][NT][kt][64] (16-byte units) at b_off; the sinc slices take
 // kMfmaSlicesA x MT x kt_max KiB, MT = 4 ceil(nq / 128).
+// wide: a group may be two waves' tiles side by side (where there are columns for
+// both), and columns of fewer slices join those of more while together they fit one
+// such group, which saves a pass over the sinc slices.
 inline bool mfma_batch_plan(const std::vector<unsigned long long> &hist_off,
                             const std::vector<uint32_t> &nhist,
                             const std::vector<unsigned long long> &count_bound, unsigned nq,
-                            MfmaBatchPlan *plan) {
+                            MfmaBatchPlan *plan, bool wide = false) {
   MfmaBatchPlan p;
   const size_t n = nhist.size();
   std::vector<uint32_t> nb(n);
@@ -63,26 +67,46 @@ inline bool mfma_batch_plan(const std::vector<unsigned long long> &hist_off,
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
     return nb[a] != nb[b] ? nb[a] > nb[b] : nhist[a] > nhist[b];
   });
+  struct Class {
+    size_t c0, c1;
+    uint32_t nb;
+  };
+  std::vector<Class> classes;
+  for (size_t c = 0; c < n; ++c) {
+    const uint32_t k = nb[order[c]];
+    if (classes.empty() || classes.back().nb != k) {
+      if (wide && !classes.empty() && c - classes.back().c0 < 64 * (classes.back().nb <= 2 ? 2u : 1u)) {
+        size_t e = c;
+        while (e < n && nb[order[e]] == k) ++e;
+        if (e - classes.back().c0 <= 64 * (classes.back().nb <= 2 ? 2u : 1u)) {
+          classes.back().c1 = e;
+          std::stable_sort(order.begin() + classes.back().c0, order.begin() + e,
+                           [&](uint32_t a, uint32_t b) { return nhist[a] > nhist[b]; });
+          c = e - 1;
+          continue;
+        }
+      }
+      classes.push_back(Class{c, c, k});
+    }
+    classes.back().c1 = c + 1;
+  }
   p.cols.resize(n);
   for (size_t c = 0; c < n; ++c) p.cols[c] = MfmaCol{hist_off[order[c]], nhist[order[c]], order[c]};
   unsigned long long b_off = 0;
   uint32_t max_nh = 0;
-  for (size_t c0 = 0; c0 < n;) {
-    const uint32_t k = nb[order[c0]];
-    size_t c1 = c0;
-    while (c1 < n && nb[order[c1]] == k) ++c1;
-    const uint32_t NT = k <= 2 ? 2 : 1;
-    MfmaLaunch L{(uint32_t)p.tiles.size(), 0u, k, NT};
-    for (size_t g = c0; g < c1; g += 32 * NT) {
+  for (const Class &cl : classes) {
+    const uint32_t NT = cl.nb <= 2 ? 2 : 1;
+    const uint32_t WN = wide && cl.c1 - cl.c0 > 32 * NT ? 2 : 1;
+    MfmaLaunch L{(uint32_t)p.tiles.size(), 0u, cl.nb, NT, WN};
+    for (size_t g = cl.c0; g < cl.c1; g += 32 * NT * WN) {
       const uint32_t kt = std::max<uint32_t>(1u, (nhist[order[g]] + 31) / 32);
-      const uint32_t ncol = (uint32_t)std::min<size_t>(32 * NT, c1 - g);
+      const uint32_t ncol = (uint32_t)std::min<size_t>(32 * NT * WN, cl.c1 - g);
       p.tiles.push_back(MfmaTile{b_off, kt, (uint32_t)g, ncol, 0u});
-      b_off += (unsigned long long)k * NT * kt * 64;
+      b_off += (unsigned long long)cl.nb * NT * WN * kt * 64;
       max_nh = std::max(max_nh, nhist[order[g]]);
       ++L.ntiles;
     }
     p.launches.push_back(L);
-    c0 = c1;
   }
   const unsigned MT = (nq + 127) / 128 * 4;
   p.kt_max = std::max<uint32_t>(1u, (max_nh + 31) / 32);

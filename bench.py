@@ -62,12 +62,15 @@ CU_ISSUE_PER_S = 256 * 2.4e9
 # instruction type (2 for this one, 1 for the FP64 kernel).
 F32_ACTIVE_PER_64_PAIRS = 23.89
 FP32_PEAK_TFLOPS = 157.3
-# Direct Debye and 2D units (one op per sin, cos, add, multiply): 4 ops per
-# pair-q term (sin, q r, x 1/(q r), accumulate) and 7 per complex-exponential
-# term (sin, cos, 3 for q.r, 2 accumulations).  Both kernels compute in FP64,
-# so the peak is the FP64 vector one.
+# Direct Debye: the direct form's unit is 4 ops per pair-q term (sin, q r, x 1/(q r),
+# accumulate).  The kernels go through moments of the pair distances and execute far
+# fewer, so the rate in that unit is reported without a fraction of a peak.
 DEBYE_OPS_PER_PAIR_Q = 4
-AMP2D_OPS_PER_TERM = 7
+# 2D patterns on a q grid: FP64 operations the kernel executes per
+# complex-exponential term: two FMAs of the matrix instruction, and one sixteenth of a
+# run's seed (3 FMAs for q.r, reduction, sine and cosine, a rotation of 4, conversions:
+# 14).  The peak is the FP64 one, the same for matrix and vector instructions.
+AMP2D_OPS_PER_TERM = 2 * 2 + 14 / 16
 # HBM bytes per launch of hist_kernel_f64<32768, true> on this workload, from
 # rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (KiB per dispatch), scaled by
 # the counters' reading for a 1 GiB device-to-device copy (FETCH_SIZE reads
@@ -570,7 +573,7 @@ def pairsum_matrix_leg(ctx, steps):
                            "per q (the arithmetic of the reference GPU kernels)",
         "fp64_equiv_tflops_mfma": round(flop / tm / 1e12, 2),
         "roofline_mfma": {"bound": "mfma", "achieved": round(int8_ops / (mm_ms * 1e-3) / 1e12, 1),
-                          "peak": 5000.0, "unit": "TOP/s (int8)",
+                          "peak": 5000.0, "unit": "TOP/s (int8, of products over all bins and slices; empty ones are skipped)",
                           "frac": round(int8_ops / (mm_ms * 1e-3) / 1e12 / 5000.0, 4),
                           "int8_products": 5 * nb},
         "max_rel_err_S_vs_fp64": {"fp64_vector": s_err(Svh), "mfma": s_err(Smh),
@@ -721,9 +724,8 @@ def debye_leg(ctx):
         achieved = DEBYE_OPS_PER_PAIR_Q * pairs * q.size / (kms * 1e-3) / 1e12
         rec = {"atoms": ens.n, "nq": int(q.size), "pair_q": pairs * int(q.size), "ms": round(t * 1e3, 3),
                "kernel_ms": round(kms, 3), "gpair_q_per_s": round(pairs * q.size / (kms * 1e-3) / 1e9, 1),
-               "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS,
-                            "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                            "ops_per_pair_q": DEBYE_OPS_PER_PAIR_Q, "kernel": "debye_kernel<true>"}}
+               "direct_equivalent": {"tflops": round(achieved, 3), "ops_per_pair_q": DEBYE_OPS_PER_PAIR_Q,
+                                     "kernel": "moments_kernel (LDS atomics), eval_kernel"}}
         if ens.n <= 2000:
             d = np.sqrt(((x64[:, :, None] - x64[:, None, :]) ** 2).sum(axis=0))
             iu = np.triu_indices(ens.n, 1)

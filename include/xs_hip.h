@@ -126,8 +126,11 @@ int xs_hist(xs_ctx *ctx, const void *xyz, size_t n_atoms,
  * int8 matrix cores: A (the sinc table) split into five int8 slices, the
  * counts into exact 7-bit slices, int32 accumulation; the result differs
  * from the FP64 sum by about 2^-35 sum_k h[k] (needs counts < 2^35 and a
- * workspace of ~5 nq nhist bytes).  It pays off for many histograms (pair
- * types of many structures) on one bin grid.
+ * workspace of ~5 nq nhist bytes, and reads the counts' extents back).  The
+ * FP64 form is faster where 64 nodes stand for more than ~300 bins.
+ * On device arrays and without XS_PAIRSUM_MFMA the call may be captured: it
+ * then sums bin by bin, without scratch (as it does where the node tables'
+ * memory, at most ~260 MiB + 16 bytes a bin, cannot be had).
  * XS_PAIRSUM_F32 evaluates the terms and the sums over 2048-bin chunks in
  * FP32 (IEEE sinf), the arithmetic of the reference GPU kernels; its error
  * against FP64 reaches ~1e-4 of I(q) at low q, where I(q) is a cancelling
@@ -147,9 +150,11 @@ int xs_pdf(xs_ctx *ctx, const uint64_t *hist, unsigned n_el,
            double rho0, const double *sl, double *pdf, unsigned flags);
 
 /* H5: direct Debye pair sums S[p*nq+iq] = sum_{pairs in p} sin(q r)/(q r + 1e-8)
- * with FP64 pair terms (xyz double).  On a uniform q mesh (the reference's,
- * ReadXML.cpp:220-222) sin(q r) advances from q to q by a rotation; other
- * meshes evaluate the series per q.  Replaces the pair loop of calcIntDebye
+ * with FP64 pair terms (xyz double).  Where that is cheaper the sums go
+ * through Chebyshev moments of the pair distances (5e-13 a pair); else, on a
+ * uniform q mesh (the reference's, ReadXML.cpp:220-222) sin(q r) advances
+ * from q to q by a rotation, and other meshes evaluate the series per q.
+ * Replaces the pair loop of calcIntDebye
  * (CalcFunctions.cpp:561-591) and calcIntDebyeKernel (CalcFunctionsCUDA.cu:1163-1273). */
 int xs_debye_pairsum(xs_ctx *ctx, const double *xyz, size_t n_atoms,
                      const unsigned *el_count, unsigned n_el, const double *q,
@@ -241,8 +246,8 @@ int xs_pairlist_pairsum(xs_ctx *ctx, const double *r, const unsigned *type, size
  * nhist[s] = 0 (or nhist == NULL) takes GetHistSize's bin count
  * (CalcFunctions.cpp:224-243).  Each structure needs at least one atom.
  * With XS_DEVICE_PTRS the xyz[s] are device pointers (the array xyz itself
- * is host memory) and the structures are tiled on the GPU (radix sorts over
- * all atoms at once; fewer than 2^31 atoms in all); otherwise they are
+ * is host memory) and the structures are tiled on the GPU (all atoms at
+ * once; fewer than 2^31 atoms in all); otherwise they are
  * tiled on the host's cores and uploaded.  Either way the call returns
  * when the plan is ready, and the coordinates are not needed afterwards.
  * The plan holds on the device the sorted coordinates (24 or 12 bytes per

@@ -42,17 +42,17 @@ NQ = 4096
 FP64_PEAK_TFLOPS = 78.6           # MI355X published FP64 vector peak (binning is FP64)
 VALU_ISSUE_TOPS = 256 * 4 * 16 * 2.4e9 / 1e12   # non-packed lane-ops/s (39.3 T)
 OPS_PER_PAIR = 11                 # 3 sub, 3 mul, 2 add, sqrt, div, cvt
-# VALU issue cycles per 64 pairs of the histogram kernel, from rocprofv3 SQ
-# counters on this workload: 11.68 VALU wave-instructions per 64 pairs, 1.04
-# of them v_rsq_f64, which occupies the issue port four times as long as
-# v_fma_f64 (3 extra cycles); SQ_ACTIVE_INST_VALU reads 14.79.  A CU
-# issues one 64-lane VALU instruction per cycle (4 SIMDs x 16 lanes), so the
-# fraction of the CUs' issue cycles at the 2.4 GHz peak clock the kernel
-# spends issuing VALU work is SLOTS_PER_PAIR * pairs / 64 / (256 * 2.4e9 * t).
-SLOTS_PER_PAIR = 14.79
+# Issue cycles per 64 pairs of the histogram kernel, from rocprofv3 SQ counters on
+# this workload: vector instructions 10.00 (SQ_ACTIVE_INST_VALU: 6.93 of them, 1.02
+# v_rsq_f64, which holds the port four times as long as v_fma_f64) and the FP64 matrix
+# instruction 4.08 (SQ_VALU_MFMA_BUSY_CYCLES, 16.3 cycles of one of the four SIMDs);
+# the two do not overlap.  A CU issues one 64-lane instruction per cycle (4 SIMDs x 16
+# lanes), so the fraction of the CUs' issue cycles at the 2.4 GHz peak clock the kernel
+# spends issuing is SLOTS_PER_PAIR * pairs / 64 / (256 * 2.4e9 * t).
+SLOTS_PER_PAIR = 14.08
 CU_ISSUE_PER_S = 256 * 2.4e9
 # FP32 binning kernel (hist_kernel_f32<32768, true>) on the same workload:
-# SQ_ACTIVE_INST_VALU reads 23.89 wave-instructions per 64 pairs.  Its
+# SQ_ACTIVE_INST_VALU reads 20.06 wave-instructions per 64 pairs.  Its
 # roofline fraction is the algorithmic one of the FP64 line: 11 ops per pair
 # x pairs / t against MI355X's FP32 vector peak (157.3 TFLOP/s).  Beside it,
 # the issue rate it reaches in wave-instructions per CU-cycle at 2.4 GHz:
@@ -60,7 +60,7 @@ CU_ISSUE_PER_S = 256 * 2.4e9
 # (measured), i.e. up to two FP32 wave-instructions per CU-cycle against one
 # for FP64, so each kernel's issue rate is read against the peak of its own
 # instruction type (2 for this one, 1 for the FP64 kernel).
-F32_ACTIVE_PER_64_PAIRS = 23.89
+F32_ACTIVE_PER_64_PAIRS = 20.06
 FP32_PEAK_TFLOPS = 157.3
 # Direct Debye: the direct form's unit is 4 ops per pair-q term (sin, q r, x 1/(q r),
 # accumulate).  The kernels go through moments of the pair distances and execute far
@@ -71,11 +71,11 @@ DEBYE_OPS_PER_PAIR_Q = 4
 # run's seed (3 FMAs for q.r, reduction, sine and cosine, a rotation of 4, conversions:
 # 14).  The peak is the FP64 one, the same for matrix and vector instructions.
 AMP2D_OPS_PER_TERM = 2 * 2 + 14 / 16
-# HBM bytes per launch of hist_kernel_f64<32768, true> on this workload, from
+# HBM bytes per launch of hist_kernel_f64<32768> on this workload, from
 # rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (KiB per dispatch), scaled by
 # the counters' reading for a 1 GiB device-to-device copy (FETCH_SIZE reads
 # 524,308 KiB for the 1,048,576 KiB copied, WRITE_SIZE 1,048,576 KiB).
-HIST_FETCH_KIB, HIST_WRITE_KIB = 7746906, 9982160
+HIST_FETCH_KIB, HIST_WRITE_KIB = 7096870, 9979720
 FETCH_SCALE, WRITE_SCALE = 1048576 / 524308, 1.0
 HIST_TRAFFIC_BYTES = int((HIST_FETCH_KIB * FETCH_SCALE + HIST_WRITE_KIB * WRITE_SCALE) * 1024)
 
@@ -1051,15 +1051,15 @@ def main():
                    "parallelism": "single GPU"},
         "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                     "traffic": HIST_TRAFFIC_BYTES, "kernel": "hist_kernel_f64<32768, true>",
+                     "traffic": HIST_TRAFFIC_BYTES, "kernel": "hist_kernel_f64<32768>",
                      "ops_per_pair": OPS_PER_PAIR, "kernel_ms": round(hist_ms, 3),
                      "valu_issue_frac": round(achieved / VALU_ISSUE_TOPS, 4),
                      "valu_issue_cycles_per_64_pairs": SLOTS_PER_PAIR,
                      "valu_issue_cycle_frac": round(
                          SLOTS_PER_PAIR * pairs / 64 / (CU_ISSUE_PER_S * hist_ms * 1e-3), 4),
                      "traffic_note": "HBM bytes per launch (FETCH_SIZE x 2.0 + WRITE_SIZE, copy-calibrated); "
-                                     "J records read per work item through the scalar cache, their "
-                                     "L2 misses served from MALL/HBM, and histogram window flushes "
+                                     "J records read per work item, their L2 misses served "
+                                     "from MALL/HBM, and histogram window flushes "
                                      "(device-scope atomics, 64 B each): ~26 GB at ~120 GB/s, 1.5% "
                                      "of HBM bandwidth"},
         "kernels_ms_per_step": {k: round(v[0] / max(v[1], 1), 4) for k, v in kern.items()},

@@ -183,11 +183,44 @@ __global__ void hist_scatter(const T *__restrict__ x, const T *__restrict__ y,
   sz[pos] = z[i];
 }
 
+// Records of the FP64 kernel's J atoms: each atom relative to the centre c
+// of its tile's box lo, hi (the centre tile_band takes) in units of 2 bins
+// (scale = 1/(2 bin)), (x', y', z', |r'|^2), four doubles per atom in the
+// sorted order.
+__device__ __forceinline__ void tile_records(const double *__restrict__ x, const double *__restrict__ y,
+                                             const double *__restrict__ z, const Tile &t,
+                                             const double (&lo)[3], const double (&hi)[3],
+                                             double scale, double *__restrict__ rec) {
+  double c[3];
+  for (int a = 0; a < 3; ++a) c[a] = 0.5 * (lo[a] + hi[a]);
+  for (uint32_t i = threadIdx.x; i < t.cnt; i += blockDim.x) {
+    const size_t g = (size_t)t.off + i;
+    const double u = (x[g] - c[0]) * scale, v = (y[g] - c[1]) * scale, w = (z[g] - c[2]) * scale;
+    double *r = rec + 4 * g;
+    r[0] = u;
+    r[1] = v;
+    r[2] = w;
+    r[3] = fma(w, w, fma(v, v, u * u));
+  }
+}
+
+__global__ void hist_tile_records(const double *__restrict__ x, const double *__restrict__ y,
+                                  const double *__restrict__ z, const Tile *__restrict__ tiles,
+                                  const double *__restrict__ boxes, double scale,
+                                  double *__restrict__ rec) {
+  const double *b = boxes + 6 * (size_t)blockIdx.x;
+  const double lo[3] = {b[0], b[1], b[2]}, hi[3] = {b[3], b[4], b[5]};
+  tile_records(x, y, z, tiles[blockIdx.x], lo, hi, scale, rec);
+}
+
+// Boxes of the tiles, the flag of one wider than cap, and, where rec is given, the FP64
+// kernel's records.
 template <class T>
 __global__ void hist_tile_boxes(const T *__restrict__ x, const T *__restrict__ y,
                                 const T *__restrict__ z, const Tile *__restrict__ tiles,
                                 double *__restrict__ boxes, double cap,
-                                unsigned long long *__restrict__ wide) {
+                                unsigned long long *__restrict__ wide, double scale,
+                                double *__restrict__ rec) {
   const Tile t = tiles[blockIdx.x];
   double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (uint32_t i = threadIdx.x; i < t.cnt; i += blockDim.x) {
@@ -214,6 +247,27 @@ __global__ void hist_tile_boxes(const T *__restrict__ x, const T *__restrict__ y
   }
   if (threadIdx.x < 6) boxes[(size_t)blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
   if (wide && threadIdx.x < 3 && s[3 + threadIdx.x][0] - s[threadIdx.x][0] > cap) *wide = 1ull;
+  if constexpr (sizeof(T) == 8) {
+    if (rec) {
+      for (int a = 0; a < 3; ++a) {
+        lo[a] = s[a][0];
+        hi[a] = s[3 + a][0];
+      }
+      tile_records(x, y, z, t, lo, hi, scale, rec);
+    }
+  }
+}
+
+// Zeros for a call's counts and its two single words (b may be null).
+__global__ void fill_counts(unsigned long long *__restrict__ p, size_t n, unsigned long long *__restrict__ a,
+                            unsigned long long *__restrict__ b) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *a = 0ull;
+    if (b) *b = 0ull;
+  }
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+       i += (size_t)gridDim.x * blockDim.x)
+    p[i] = 0ull;
 }
 
 __global__ void fill_u64(unsigned long long *__restrict__ p, size_t n) {
@@ -697,29 +751,6 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
     }
   }
   flush_window<WCAP>(win, B, min(B + (uint32_t)WCAP, nhist), D, hp);
-}
-
-// Records of the FP64 kernel's J atoms: each atom relative to the centre c
-// of its tile's box (the centre tile_band takes) in units of 2 bins
-// (scale = 1/(2 bin)), (x', y', z', |r'|^2), four doubles per atom in the
-// sorted order.
-__global__ void hist_tile_records(const double *__restrict__ x, const double *__restrict__ y,
-                                  const double *__restrict__ z, const Tile *__restrict__ tiles,
-                                  const double *__restrict__ boxes, double scale,
-                                  double *__restrict__ rec) {
-  const Tile t = tiles[blockIdx.x];
-  const double *b = boxes + 6 * (size_t)blockIdx.x;
-  double c[3];
-  for (int a = 0; a < 3; ++a) c[a] = 0.5 * (b[a] + b[3 + a]);
-  for (uint32_t i = threadIdx.x; i < t.cnt; i += blockDim.x) {
-    const size_t g = (size_t)t.off + i;
-    const double u = (x[g] - c[0]) * scale, v = (y[g] - c[1]) * scale, w = (z[g] - c[2]) * scale;
-    double *r = rec + 4 * g;
-    r[0] = u;
-    r[1] = v;
-    r[2] = w;
-    r[3] = fma(w, w, fma(v, v, u * u));
-  }
 }
 
 // FP64 binning: one work item = (pair type, I tile pair {2 ti, 2 ti + 1},
@@ -1396,10 +1427,11 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
     Carver cb(ctx->ws);
     double *part = cb.take<double>(kBoxBlocks * 6);
     double *bbox_d = cb.take<double>(8);
-    const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, kBoxBlocks);
+    const unsigned nb = n <= 1024 ? 1 : (unsigned)std::min<size_t>((n + 255) / 256, kBoxBlocks);
     hipLaunchKernelGGL((hist_bbox_partial<T>), dim3(nb), dim3(256), 0, ctx->stream, xyz, xyz + n,
-                       xyz + 2 * n, n, part);
-    hipLaunchKernelGGL(hist_bbox_reduce, dim3(1), dim3(256), 0, ctx->stream, part, (int)nb, bbox_d);
+                       xyz + 2 * n, n, nb == 1 ? bbox_d : part);
+    if (nb > 1)
+      hipLaunchKernelGGL(hist_bbox_reduce, dim3(1), dim3(256), 0, ctx->stream, part, (int)nb, bbox_d);
     XS_HIP_CHECK(hipGetLastError());
     XS_HIP_CHECK(hipMemcpyAsync(ctx->pin, bbox_d, 6 * sizeof(double), hipMemcpyDeviceToHost,
                                 ctx->stream));
@@ -1527,13 +1559,9 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
                               hipMemcpyHostToDevice, ctx->stream));
   double *boxes = reinterpret_cast<double *>(static_cast<char *>(ctx->aux) + up);
   const unsigned zb = (unsigned)std::min<size_t>((hsize + 255) / 256, 4096);
-  hipLaunchKernelGGL(fill_u64, dim3(std::max(zb, 1u)), dim3(256), 0, ctx->stream, hist_d, hsize);
-  hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, ctx->stream, ovf_d, (size_t)1);
-  unsigned long long *wide_d = nullptr;
-  if (equal_count && std::isfinite(cap)) {
-    wide_d = ovf_own + 1;
-    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, ctx->stream, wide_d, (size_t)1);
-  }
+  unsigned long long *wide_d = equal_count && std::isfinite(cap) ? ovf_own + 1 : nullptr;
+  hipLaunchKernelGGL(fill_counts, dim3(std::max(zb, 1u)), dim3(256), 0, ctx->stream, hist_d, hsize, ovf_d,
+                     wide_d);
   for (unsigned e = 0; e < n_el && !equal_count; ++e)
     if (el_count[e])
       hipLaunchKernelGGL((hist_scatter<T>), dim3((el_count[e] + 255) / 256), dim3(256), 0, ctx->stream,
@@ -1541,8 +1569,8 @@ static int run_device(xs_ctx *ctx, const T *xyz, size_t n, const unsigned *el_co
                          keys + eoff[e], start_d + soff[e], sxp, syp, szp);
   if (!tiles.empty())
     hipLaunchKernelGGL((hist_tile_boxes<T>), dim3((unsigned)tiles.size()), dim3(256), 0, ctx->stream,
-                       sxp, syp, szp, tiles_d, boxes, cap, wide_d);
-  launch_records<T>(ctx->stream, sxp, syp, szp, tiles_d, boxes, tiles.size(), bin, rec);
+                       sxp, syp, szp, tiles_d, boxes, cap, wide_d, 0.5 / bin,
+                       sizeof(T) == 8 ? rec : nullptr);
   XS_HIP_CHECK(hipGetLastError());
   if (wide_d && !tiles.empty()) {
     // equal-count tiles of a structure far from uniform density can be wider
@@ -2052,7 +2080,7 @@ static int plan_build_device(xs_ctx *ctx, unsigned nstruct, const unsigned *n_el
   hipError_t e = hipMemcpy(tiled.p, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL((hist_tile_boxes<T>), dim3((unsigned)tiles.size()), dim3(256), 0, st, c, c + nc,
-                       c + 2 * nc, tiled.at<Tile>(), boxes_d.at<double>(), INFINITY, nullptr);
+                       c + 2 * nc, tiled.at<Tile>(), boxes_d.at<double>(), INFINITY, nullptr, 0.0, nullptr);
     e = hipMemcpyAsync(boxes.data(), boxes_d.p, boxes.size() * 8, hipMemcpyDeviceToHost, st);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -11,7 +11,8 @@
 //
 // Bound by launches (eight, about 3 us each) and the latency of the atomics.  110,592
 // atoms, FP64 (two elements): 47 us; the radix and merge sorts of three 64-bit
-// and two 32-bit keys per element took 480 in 110 launches.
+// and two 32-bit keys per element took 480 in 110 launches.  Few atoms go through one
+// work group in one launch (small).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -252,6 +253,90 @@ __global__ __launch_bounds__(kThreads) void put(Work W, const S *__restrict__ x,
   sz[p] = (T)z[a];
 }
 
+// The same by one work group, for up to kSmallAtoms atoms and kSmallCounters counters:
+// counters in LDS, an atom's coordinates, counter and place in registers.  Parts follow
+// one another in the counters as their atoms do in the ranks, so one sum over all
+// counters of an axis gives every atom its rank.  Bound by latency (tables, LDS atomics,
+// 15 barriers): 2,000 atoms 14 us, where the eight launches take 27 and their gaps.
+// Whole FP64 histograms of 500, 2,000 and 3,000 atoms 134, 149 and 140 -> 118, 138 and 133 us
+// (with one launch less each for records and clearing); at 4,096 atoms both ways take 143.5.
+constexpr int kSmallThreads = 1024, kSmallPer = 4;
+constexpr uint32_t kSmallAtoms = kSmallThreads * kSmallPer, kSmallCounters = 8192;
+
+template <class S, class T>
+__global__ __launch_bounds__(kSmallThreads) void small(Work W, const S *__restrict__ x,
+                                                       const S *__restrict__ y, const S *__restrict__ z,
+                                                       T *__restrict__ sx, T *__restrict__ sy,
+                                                       T *__restrict__ sz) {
+  __shared__ uint32_t count[kSmallCounters], part[kSmallThreads / 64];
+  constexpr uint32_t kOwn = kSmallCounters / kSmallThreads;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  S v[3][kSmallPer] = {};
+  uint32_t seg[kSmallPer] = {}, slab[kSmallPer] = {}, rank[kSmallPer] = {}, key[kSmallPer] = {};
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j) {
+    const uint32_t a = tid + j * kSmallThreads;
+    if (a < W.natoms) {
+      v[0][j] = x[a];
+      v[1][j] = y[a];
+      v[2][j] = z[a];
+      seg[j] = seg_of(W, a);
+    }
+  }
+#pragma unroll
+  for (int axis = 0; axis < 3; ++axis) {
+    for (uint32_t i = tid; i < kSmallCounters; i += kSmallThreads) count[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSmallPer; ++j) {
+      const bool in = tid + j * kSmallThreads < W.natoms;
+      if (in) {
+        const Seg s = W.segs[seg[j]];
+        if (axis == 0) {
+          key[j] = s.count0 + bucket((double)v[0][j], s.lo[0], s.scale[0], s.nb);
+        } else if (axis == 1) {
+          slab[j] = s.slab0 + equal_part(rank[j] - s.start, s.n, s.gx);
+          const Slab l = W.slabs[slab[j]];
+          key[j] = l.count0 + bucket((double)v[1][j], s.lo[1], s.scale[1], l.nb);
+        } else {
+          const Slab l = W.slabs[slab[j]];
+          const uint32_t c = equal_part(rank[j] - l.start, l.n, l.gy);
+          key[j] = l.zcount0 + c * l.znb + bucket((double)v[2][j], s.lo[2], s.scale[2], l.znb);
+        }
+      }
+      rank[j] = take_place(count, key[j], in);
+    }
+    __syncthreads();
+    uint32_t before[kOwn], sum = 0;
+    for (uint32_t i = 0; i < kOwn; ++i) {
+      before[i] = sum;
+      sum += count[kOwn * tid + i];
+    }
+    uint32_t incl = sum;
+    for (int d = 1; d < 64; d *= 2) {
+      const uint32_t o = __shfl_up(incl, d, 64);
+      if ((int)lane >= d) incl += o;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    uint32_t first = incl - sum;
+    for (uint32_t w = 0; w < wave; ++w) first += part[w];
+    for (uint32_t i = 0; i < kOwn; ++i) count[kOwn * tid + i] = first + before[i];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSmallPer; ++j)
+      if (tid + j * kSmallThreads < W.natoms) rank[j] += count[key[j]];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kSmallPer; ++j)
+    if (tid + j * kSmallThreads < W.natoms) {
+      sx[rank[j]] = (T)v[0][j];
+      sy[rank[j]] = (T)v[1][j];
+      sz[rank[j]] = (T)v[2][j];
+    }
+}
+
 template <class S, class T>
 int run(xs_ctx *ctx, const Tables &t, const char *tables, char *scratch, const S *x, const S *y,
         const S *z, T *sx, T *sy, T *sz) {
@@ -268,6 +353,11 @@ int run(xs_ctx *ctx, const Tables &t, const char *tables, char *scratch, const S
   W.slab = cv.take<uint32_t>(t.natoms);
   W.natoms = (uint32_t)t.natoms;
   const hipStream_t st = ctx->stream;
+  if (t.natoms <= kSmallAtoms && t.counters <= kSmallCounters) {
+    hipLaunchKernelGGL((small<S, T>), dim3(1), dim3(kSmallThreads), 0, st, W, x, y, z, sx, sy, sz);
+    XS_HIP_CHECK(hipGetLastError());
+    return XS_OK;
+  }
   const dim3 block(kThreads), atoms((unsigned)((t.natoms + kThreads - 1) / kThreads));
   hipLaunchKernelGGL(clear, dim3((unsigned)((t.counters + kThreads - 1) / kThreads)), block, 0, st, W.count,
                      t.counters);

@@ -627,8 +627,8 @@ __device__ __forceinline__ void pair_block_f32(float xi, float yi, float zi, uin
   }
 }
 
-// FP32 binning: one work item = (pair type, I tile, run of J tiles), one I
-// atom per thread.
+// FP32 binning: one work item = (pair type, I tile, run of J tiles), of each J
+// tile the share blockIdx.y of gridDim.y, one I atom per thread.
 template <int WCAP, bool FQ>
 __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
   using T = float;
@@ -722,8 +722,10 @@ __global__ __launch_bounds__(kTile) void hist_kernel_f32(Args<float> A) {
     }
     const Tile J = A.tiles[tjg];
     const bool diag = td.same && tj == it.ti;
-    for (uint32_t s0 = 0; s0 < J.cnt; s0 += kStage) {
-      const uint32_t cn = min((uint32_t)kStage, J.cnt - s0);
+    const uint32_t g8 = (J.cnt + 7) / 8;  // this work group's share, by groups of 8
+    const uint32_t jend = min(g8 * (blockIdx.y + 1) / gridDim.y * 8, J.cnt);
+    for (uint32_t s0 = g8 * blockIdx.y / gridDim.y * 8; s0 < jend; s0 += kStage) {
+      const uint32_t cn = min((uint32_t)kStage, jend - s0);
       if (tid < cn) {
         const size_t g = (size_t)J.off + s0 + tid;
         sx[tid] = A.x[g];
@@ -1291,8 +1293,7 @@ static void launch_records(hipStream_t st, const T *x, const T *y, const T *z, c
   }
 }
 
-// Shares that the J tiles of every FP64 item are cut into (hist_kernel_f64's
-// grid.y), so that a small structure's few items fill the chip: an item of
+// Shares that the J tiles of every item are cut into (the kernels' grid.y), so that a small structure's few items fill the chip: an item of
 // 2,048 x 1,024 pairs keeps one CU busy for 0.2 ms (16.6 cycles per 64 pairs),
 // while a work group costs some 4 or 20 us more than its pairs (window cleared
 // and flushed, J tiles sorted).  The estimate is rounds x work group time, half
@@ -1300,12 +1301,18 @@ static void launch_records(hipStream_t st, const T *x, const T *y, const T *z, c
 // 2,000 atoms (2 items) 205, 130, 85, 59, 47, 40 us; 8,000 atoms (20 items)
 // 248, 143, 91, 59, 76, 92; 22,000 atoms (156 items) 235, 231, 217, 237, 319,
 // 584; 60,000 atoms (930 items) 880, 913, 944, 1,069, 1,343, 1,883.
-static unsigned item_shares(size_t nitems, double pairs, uint32_t wcap, int cus) {
+// FP32 items fill a CU at nearly the same rate and go by the same estimate; where they
+// fill the chip once, a share is no less than a stage of J atoms, whose barriers it
+// would pay for fewer pairs.  Calls from the host with 1,000, 4,096, 8,000, 15,000 and
+// 60,000 atoms took 314, 317, 312, 332 and 1,185 us in one share, 125, 149, 177, 226 and
+// 1,108 so; 16 structures of 3,000 atoms 332 -> 118, 48 of 10,000 1,328 -> 1,314.
+static unsigned item_shares(size_t nitems, double pairs, uint32_t wcap, bool f64, int cus) {
   const double w = pairs / (double)nitems / 64.0 * 16.6 / 2400.0;  // us
   const double fixed = wcap > 8192 ? 20.0 : 4.0;
+  const unsigned most = !f64 && nitems >= (size_t)cus ? kTile / kStage : 32;
   unsigned best = 1;
   double bt = INFINITY;
-  for (unsigned s = 1; s <= 32; s *= 2) {
+  for (unsigned s = 1; s <= most; s *= 2) {
     const double rounds = std::ceil((double)nitems * s / cus);
     const double t = (rounds + 0.5) * (w / s + fixed);
     if (t < bt) {
@@ -1324,8 +1331,8 @@ static int launch_hist(xs_ctx *ctx, const Args<T> &A, size_t nitems, double pair
   if (prof) XS_TRY(prof_begin(ctx, "hist", &ev));
   dim3 grid((unsigned)nitems);
   const dim3 block(kTile);
+  grid.y = item_shares(nitems, pairs, wcap, sizeof(T) == 8, ctx->cu_count);
   if constexpr (sizeof(T) == 8) {
-    grid.y = item_shares(nitems, pairs, wcap, ctx->cu_count);
     if (wcap == 8192)
       hipLaunchKernelGGL((hist_kernel_f64<8192>), grid, block, 0, ctx->stream, A);
     else

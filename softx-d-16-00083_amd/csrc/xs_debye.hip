@@ -380,10 +380,14 @@ static int run(xs_ctx *ctx, const double *xyz_in, size_t n, const unsigned *el_c
   const MeshBox in = mesh_box(*static_cast<const BoxOut *>(ctx->pin));
 
   MomentPlan mp;
+  bool moments = false;
   if (plan_moments(in, seg_cnt, n_el, nblocks, nq, ctx->cu_count, &mp)) {
-    XS_TRY(ensure_aux(ctx, moments_table_bytes(seg_cnt, n_el, nblocks, ctx->cu_count)));
-    XS_TRY(run_moments(ctx, mp, xyz, n, seg_cnt, n_el, nblocks, in, qd, nq, Sd, ctx->aux));
-  } else {
+    int e = ensure_aux(ctx, moments_table_bytes(seg_cnt, n_el, nblocks, ctx->cu_count));
+    if (e == XS_OK) e = run_moments(ctx, mp, xyz, n, seg_cnt, n_el, nblocks, in, qd, nq, Sd, ctx->aux);
+    if (e != XS_OK && e != XS_ERR_NOMEM) return e;
+    moments = e == XS_OK;  // without memory for the moments (nothing launched): pair by pair
+  }
+  if (!moments) {
     std::vector<Tile> tiles;
     std::vector<Item> items;
     tile_tables(seg_cnt, n_el, nblocks, &tiles, &items);

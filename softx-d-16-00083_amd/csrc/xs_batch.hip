@@ -17,6 +17,7 @@
 #include <cstring>
 #include <vector>
 
+#include "xs_batch_layout.h"
 #include "xs_internal.h"
 #include "xs_nodesum.h"
 
@@ -31,38 +32,31 @@ void release_batch_run(BatchRunState &r) {
 
 namespace {
 
-struct RunLayout {
-  size_t rows, nmax, nodes, pdfdesc, q, hist, S, pdf, mm_cols, mm_tiles, mm_a, mm_b, total;
-};
-
-// Byte offsets inside the run buffer; host-mode staging only when needed;
-// the matrix-core tables and slices when mm (a plan with mm.nq != 0) is given.
+// The run buffer of one call; host-mode staging only when needed, the
+// matrix-core slices when mm (a plan with mm.nq != 0) is given.
 RunLayout layout(const xs_batch *b, unsigned nhist_max, unsigned nq, bool host, bool want_S,
                  bool want_pdf, const MfmaBatchPlan *mm) {
-  RunLayout L{};
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    off = align_up(off, 256);
-    const size_t at = off;
-    off += bytes;
-    return at;
-  };
   const size_t ntiles = (b->ntypes_total + nodesum::kRows - 1) / nodesum::kRows;
-  L.rows = take(ntiles * nodesum::kRows * sizeof(nodesum::Row));
-  L.nmax = take(ntiles * 4);
-  L.pdfdesc = take((size_t)b->nstruct * sizeof(PdfDesc));
-  L.q = take(host && want_S ? (size_t)nq * 8 : 0);
-  L.hist = take(host ? b->hist_len * 8 : 0);
-  L.S = take(host && want_S ? b->ntypes_total * nq * 8 : 0);
-  L.pdf = take(host && want_pdf ? b->pdf_len * 8 : 0);
-  L.mm_cols = take(mm ? mm->cols.size() * sizeof(MfmaCol) : 0);
-  L.mm_tiles = take(mm ? mm->tiles.size() * sizeof(MfmaTile) : 0);
-  L.mm_a = take(mm ? mm->a_bytes : 0);
-  L.mm_b = take(mm ? mm->b_bytes : 0);
-  // (last: its size depends on the call, and rows and pdfdesc stay where they are)
-  L.nodes = take(want_S && !mm ? nodesum::layout((unsigned)ntiles, nhist_max, nodesum::kBudget).total : 0);
-  L.total = align_up(off, 256);
-  return L;
+  RunSizes n;
+  n.rows = ntiles * nodesum::kRows * sizeof(nodesum::Row);
+  n.nmax = ntiles * 4;
+  n.pdfdesc = (size_t)b->nstruct * sizeof(PdfDesc);
+  // (a column for every pair type, and no group without a column)
+  n.mm_cols = b->ntypes_total * sizeof(MfmaCol);
+  n.mm_tiles = b->ntypes_total * sizeof(MfmaTile);
+  if (host) {
+    n.q = want_S ? (size_t)nq * 8 : 0;
+    n.hist = b->hist_len * 8;
+    n.S = want_S ? b->ntypes_total * nq * 8 : 0;
+    n.pdf = want_pdf ? b->pdf_len * 8 : 0;
+  }
+  if (mm) {
+    n.mm_a = mm->a_bytes;
+    n.mm_b = mm->b_bytes;
+  } else if (want_S) {
+    n.nodes = nodesum::layout((unsigned)ntiles, nhist_max, nodesum::kBudget).total;
+  }
+  return run_layout(n);
 }
 
 // Pair types, most bins first, padded to whole tiles of 16.
@@ -191,7 +185,6 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
   const RunLayout L = layout(plan, rows[0].nhist, nq, !device, want_S, want_pdf, mfma ? &R.mm : nullptr);
 
   // (re)allocate the run buffer and upload the descriptors when they change
-  bool fresh = false;
   if (L.total > R.buf_cap) {
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     if (R.exec) (void)hipGraphExecDestroy(R.exec);
@@ -207,7 +200,7 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
       return fail(XS_ERR_NOMEM, "xs_batch_run: device allocation failed");
     }
     R.buf_cap = L.total;
-    fresh = true;
+    R.uploaded = R.mm_uploaded = false;
   }
   char *buf = static_cast<char *>(R.buf);
   std::vector<double> key_rho0, key_sl;
@@ -215,8 +208,8 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
     key_rho0.assign(rho0 ? rho0 : nullptr, rho0 ? rho0 + plan->nstruct : nullptr);
     key_sl.assign(sl, sl + plan->el_count.size());
   }
-  const bool desc_changed = fresh || key_rho0 != R.key_rho0 || key_sl != R.key_sl;
-  if (fresh || desc_changed) {
+  if (!R.uploaded || key_rho0 != R.key_rho0 || key_sl != R.key_sl) {
+    R.uploaded = false;
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     std::vector<uint32_t> nmax;
     for (size_t i = 0; i < rows.size(); i += nodesum::kRows) nmax.push_back(rows[i].nhist);
@@ -227,15 +220,15 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
                            hipMemcpyHostToDevice));
     R.key_rho0 = key_rho0;
     R.key_sl = key_sl;
+    R.uploaded = true;
   }
-  if (mfma && (fresh || !R.mm_uploaded || R.mm_at != L.mm_cols)) {
+  if (mfma && !R.mm_uploaded) {
     XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     XS_HIP_CHECK(hipMemcpy(buf + L.mm_cols, R.mm.cols.data(), R.mm.cols.size() * sizeof(MfmaCol),
                            hipMemcpyHostToDevice));
     XS_HIP_CHECK(hipMemcpy(buf + L.mm_tiles, R.mm.tiles.data(), R.mm.tiles.size() * sizeof(MfmaTile),
                            hipMemcpyHostToDevice));
     R.mm_uploaded = true;
-    R.mm_at = L.mm_cols;
   }
 
   RunPtrs P{};

@@ -55,9 +55,9 @@ struct BatchRunState {
   std::vector<double> key_rho0, key_sl;
   void *buf = nullptr;   // pair-sum and PDF descriptors, host-mode staging
   size_t buf_cap = 0;
+  bool uploaded = false;     // buf holds the rows and descriptors of key_rho0, key_sl
   MfmaBatchPlan mm;      // XS_PAIRSUM_MFMA: columns, groups, buffer sizes (mm.nq = 0: none)
-  bool mm_uploaded = false;
-  size_t mm_at = 0;      // offset in buf of the uploaded matrix-core tables
+  bool mm_uploaded = false;  // its tables are in buf
 };
 
 }  // namespace xs

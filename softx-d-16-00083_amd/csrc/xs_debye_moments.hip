@@ -35,22 +35,10 @@
 namespace xs {
 namespace debye {
 
-constexpr int kMTile = 64;          // atoms per tile: one per lane
 constexpr int kMBlock = 1024;
-constexpr size_t kMLds = 160000;    // of the CU's 163,840 bytes
 constexpr double kMagic = 6755399441055744.0;            // 1.5 * 2^52
 constexpr unsigned long long kMagicBits = 0x4338000000000000ull;
 constexpr double kTwoPi = 6.283185307179586476925286766559;
-
-// A run of tile pairs of segments A and B: items first .. first + count,
-// an item being a tile pair's share of jr J atoms.
-struct Run {
-  uint32_t first, count, offA, cntA, offB, cntB, diag, pad;
-};
-
-static size_t lds_bytes(unsigned nb, int K) {
-  return (size_t)nb * (K - 1) * 8 + align_up((size_t)nb * 4, 8) + (size_t)K * 8;
-}
 
 __device__ __forceinline__ double lane_value(double v, int lane) {
   const unsigned long long u = __double_as_longlong(v);
@@ -88,24 +76,10 @@ __global__ __launch_bounds__(kMBlock) void moments_kernel(
   const unsigned TA = (run.cntA + kMTile - 1) / kMTile, TB = (run.cntB + kMTile - 1) / kMTile;
   const unsigned jr = kMTile >> sub_shift;
   __syncthreads();
-  for (unsigned m = run.first + wave; m < run.first + run.count; m += kMBlock / 64) {
-    const unsigned sub = m & ((1u << sub_shift) - 1), tp = m >> sub_shift;
-    unsigned ti, tj;
-    if (run.diag) {
-      // row ti holds the J tiles ti..TB-1; rows before it c(ti) pairs
-      const double T2 = 2.0 * (double)TB + 1.0;
-      const double g = floor(0.5 * (T2 - sqrt(fmax(T2 * T2 - 8.0 * (double)tp, 0.0))));
-      uint64_t i = g < 0.0 ? 0 : (uint64_t)g;
-      if (i >= TB) i = TB - 1;
-      auto c = [TB](uint64_t v) { return v * TB - v * (v - 1) / 2; };
-      while (i > 0 && c(i) > tp) --i;
-      while (i + 1 < TB && c(i + 1) <= tp) ++i;
-      ti = __builtin_amdgcn_readfirstlane((unsigned)i);
-      tj = __builtin_amdgcn_readfirstlane((unsigned)(i + (tp - c(i))));
-    } else {
-      ti = tp / TB;
-      tj = tp % TB;
-    }
+  for (uint64_t m = run.first + wave; m < run.first + run.count; m += kMBlock / 64) {
+    const unsigned sub = (unsigned)m & ((1u << sub_shift) - 1);
+    const TilePair tp = tile_pair(m >> sub_shift, TB, run.diag);
+    const unsigned ti = __builtin_amdgcn_readfirstlane(tp.ti), tj = __builtin_amdgcn_readfirstlane(tp.tj);
     // a tile is every TA-th (TB-th) atom: the lanes' distances to a J atom then
     // spread over the bins
     const unsigned ia = ti + lane * TA, ja = tj + lane * TB;
@@ -269,30 +243,6 @@ __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M,
 // ---------------------------------------------------------------- host side
 namespace {
 
-struct SegPair {
-  uint32_t row, a, b;
-};
-
-constexpr int kMoments[] = {6, 8, 10, 12, 14, 18, 24};
-
-// Cycles of the CUs for one call, to choose K and to leave small inputs to
-// debye_kernel.  Measured: 143 cycles a wave of 64 pairs for K = 8 on the
-// 8,000-atom rock-salt cube (1,560 bins) and 250 for K = 12 on 5,000 atoms
-// (290 bins), about 20 a moment; the evaluation's sines at half the issue
-// rate; 25 us for the launches and the copy of the tables.
-double moments_cycles(double pairs, double rows, double rgroups, unsigned nq, const nodes::Bins &b,
-                      double cus) {
-  const double per_pair = 20.0 * b.K / 64.0;
-  const double node_q = (double)b.entries() * nq * 2.0 * (26.0 * rgroups + 1.5 * rows) / 64.0;
-  return pairs * per_pair / cus + node_q / cus + (double)b.entries() * 1.5 + 60000.0;
-}
-// 3.28 VALU instructions per pair and q at 67% issue, for q in blocks of 1,024
-// whether filled or not (340 atoms, 714 q: 85 us; 594 atoms, 1,037 q: 107 us,
-// against 50 us through the moments)
-double direct_cycles(double pairs, unsigned nq, double cus) {
-  return pairs * std::ceil(nq / 1024.0) * 1024.0 * (3.28 / 0.67) / 64.0 / cus + 60000.0;
-}
-
 template <int K>
 int launch_moments(hipStream_t st, unsigned nruns, size_t lds, const double *xyz, size_t n,
                    const Run *runs, double *slabs, const nodes::Bins &b, int s, unsigned shift) {
@@ -313,98 +263,18 @@ void launch_eval(hipStream_t st, dim3 grid, const double *M, const nodes::Bins &
 
 }  // namespace
 
-bool plan_moments(const MeshBox &in, const std::vector<uint32_t> &seg_cnt, unsigned n_el,
-                  unsigned nblocks, unsigned nq, int cus, MomentPlan *plan) {
-  if (!in.finite || !(in.R > 1e-100 && in.R < 1e100) || !(in.Q > 1e-100 && in.Q < 1e100))
-    return false;
-  const unsigned nparts = nblocks * (nblocks + 1) / 2;
-  const double rows = (double)ntypes_of(n_el) * nparts;
-  double n = 0.0;
-  for (uint32_t c : seg_cnt) n += c;
-  const double pairs = 0.5 * n * (n - 1.0);
-  const double rgroups = std::ceil(rows / 8.0);
-  // a chunk of nodes per work group in x, rows in z, q blocks in y
-  if (rows > 60000.0 || nq > 256u * 65535u) return false;
-  double best = direct_cycles(pairs, nq, cus);
-  bool found = false;
-  for (int K : kMoments) {
-    const nodes::Bins b = nodes::bins_for(in.R, in.Q, K);
-    if (b.nb > 1000000u || lds_bytes(b.nb, K) > kMLds) continue;
-    // each segment pair has at least one slab
-    const double slabs = (5.0 * rows + cus) * (double)b.entries() * 8.0;
-    if (slabs > (double)(size_t(1) << 30)) continue;
-    const double c = moments_cycles(pairs, rows, rgroups, nq, b, cus);
-    if (c < best) {
-      best = c;
-      plan->bins = b;
-      found = true;
-    }
-  }
-  return found;
-}
-
 int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n,
                 const std::vector<uint32_t> &seg_cnt, unsigned n_el, unsigned nblocks,
                 const MeshBox &in, const double *q, unsigned nq, double *S, void *work) {
   const nodes::Bins &b = plan.bins;
   const unsigned nparts = nblocks * (nblocks + 1) / 2;
   const unsigned nrows = ntypes_of(n_el) * nparts;
-  std::vector<uint32_t> off(seg_cnt.size() + 1, 0);
-  for (size_t s = 0; s < seg_cnt.size(); ++s) off[s + 1] = off[s] + seg_cnt[s];
-  // segment pairs by row: (element a, block i) with (element b, block j)
-  std::vector<SegPair> sp;
-  uint64_t total = 0;
-  auto tiles = [&](uint32_t s) { return (uint64_t)(seg_cnt[s] + kMTile - 1) / kMTile; };
-  auto pair_tiles = [&](const SegPair &v) {
-    return v.a == v.b ? tiles(v.a) * (tiles(v.a) + 1) / 2 : tiles(v.a) * tiles(v.b);
-  };
-  unsigned p = 0;
-  for (unsigned a = 0; a < n_el; ++a)
-    for (unsigned c = a; c < n_el; ++c, ++p)
-      for (unsigned i = 0; i < nblocks; ++i)
-        for (unsigned j = i; j < nblocks; ++j) {
-          const uint32_t row = p * nparts + nblocks * i - (i * (i + 1)) / 2 + j;
-          const uint32_t ai = a * nblocks + i, cj = c * nblocks + j;
-          sp.push_back(SegPair{row, ai, cj});
-          if (a != c && i != j) sp.push_back(SegPair{row, a * nblocks + j, c * nblocks + i});
-        }
-  for (const SegPair &v : sp) total += pair_tiles(v);
-  // shares of a tile pair, so that every wave of the chip has a few items
-  unsigned shift = 0;
-  while (shift < 3 && (total << shift) < 64ull * ctx->cu_count) ++shift;
-  // runs: the shortest longest run for which the segment pairs' runs fill one
-  // round of work groups (two runs a segment pair where those are many), at
-  // most 2^24 pairs each (the fixed-point sums)
-  const double cap = 16777216.0 / (kMTile * kMTile);
-  const uint64_t most = std::max<uint64_t>(ctx->cu_count, 2 * sp.size());
-  double low = 0.0, per = std::max(1.0, (double)total);
-  for (int it = 0; it < 50; ++it) {
-    const double mid = 0.5 * (low + per);
-    uint64_t nr = 0;
-    for (const SegPair &v : sp) nr += (uint64_t)std::ceil((double)pair_tiles(v) / mid);
-    (nr <= most ? per : low) = mid;
-  }
-  per = std::min(per, cap);
-  std::vector<Run> runs;
-  std::vector<uint32_t> row_run(nrows + 1, 0);
-  uint32_t longest = 1;
-  for (const SegPair &v : sp) {
-    const uint64_t t = pair_tiles(v) << shift;
-    if (t) {
-      const uint64_t nr = (uint64_t)std::ceil((double)pair_tiles(v) / per);
-      for (uint64_t k = 0; k < nr; ++k) {
-        const uint64_t f = t * k / nr, e = t * (k + 1) / nr;
-        if (e == f) continue;
-        runs.push_back(Run{(uint32_t)f, (uint32_t)(e - f), off[v.a], seg_cnt[v.a], off[v.b],
-                           seg_cnt[v.b], v.a == v.b ? 1u : 0u, 0u});
-        longest = std::max(longest, (uint32_t)(e - f));
-      }
-    }
-    row_run[v.row + 1] = (uint32_t)runs.size();
-  }
-  for (unsigned r = 0; r < nrows; ++r) row_run[r + 1] = std::max(row_run[r + 1], row_run[r]);
+  const RunTables T = plan_runs(seg_cnt, n_el, nblocks, ctx->cu_count);
+  const std::vector<Run> &runs = T.runs;
+  const std::vector<uint32_t> &row_run = T.row_run;
+  const unsigned shift = T.shift;
   // |T_k 2^s + ...| <= 2^s per pair: a run's sum stays below 2^62
-  const double run_pairs = (double)longest * kMTile * (kMTile >> shift);
+  const double run_pairs = (double)T.longest * kMTile * (kMTile >> shift);
   const int s = std::min(48, 62 - (int)std::ceil(std::log2(run_pairs + 1.0)));
 
   const size_t entries = b.entries();
@@ -430,7 +300,7 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
                      dim3(256), 0, st, q, nq, in.dq, in.uniform ? 1 : 0, qe, S, ssize);
   if (!runs.empty()) {
     const unsigned nr = (unsigned)runs.size();
-    const size_t lds = lds_bytes(b.nb, b.K);
+    const size_t lds = moments_lds_bytes(b.nb, b.K);
     switch (b.K) {
       case 6: XS_TRY(launch_moments<6>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
       case 8: XS_TRY(launch_moments<8>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;

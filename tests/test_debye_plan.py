@@ -1,0 +1,22 @@
+"""Host planning of the direct Debye sums through moments (no GPU): the runs cover
+every tile pair once, beyond 2^32 of them too.  The checks are C++ (tests/cpp/)
+compiled with g++ against the library's own header."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "softx-d-16-00083_amd", "csrc")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_runs_cover_every_tile_pair(tmp_path):
+    exe = tmp_path / "debye_plan_check"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-I", CSRC,
+                    os.path.join(HERE, "cpp", "debye_plan_check.cpp"), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip().endswith("ok")

@@ -382,7 +382,7 @@ static int run(xs_ctx *ctx, const double *xyz_in, size_t n, const unsigned *el_c
   MomentPlan mp;
   bool moments = false;
   if (plan_moments(in, seg_cnt, n_el, nblocks, nq, ctx->cu_count, &mp)) {
-    int e = ensure_aux(ctx, moments_table_bytes(seg_cnt, n_el, nblocks, ctx->cu_count));
+    int e = ensure_aux(ctx, moments_table_bytes((size_t)ntypes * nparts, ctx->cu_count));
     if (e == XS_OK) e = run_moments(ctx, mp, xyz, n, seg_cnt, n_el, nblocks, in, qd, nq, Sd, ctx->aux);
     if (e != XS_OK && e != XS_ERR_NOMEM) return e;
     moments = e == XS_OK;  // without memory for the moments (nothing launched): pair by pair

@@ -9,10 +9,6 @@
 namespace xs {
 namespace debye {
 
-// Bytes of the run tables, an upper bound.
-size_t moments_table_bytes(const std::vector<uint32_t> &seg_cnt, unsigned n_el, unsigned nblocks,
-                           int cus);
-
 // Enqueues the call (all pointers device memory; S is overwritten).  `work`
 // holds moments_table_bytes.  The pinned staging must be free.
 int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n,

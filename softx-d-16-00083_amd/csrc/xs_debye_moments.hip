@@ -5,13 +5,14 @@
 // (a pair type, or a pair type and block pair).  Three kernels:
 //   moments  one work group per run of 64 x 64-atom tile pairs of one segment
 //            pair; the moments of all bins live in LDS.  T_0 is a uint32
-//            count, T_k (k >= 1) a 64-bit fixed-point sum: T_k 2^s + 1.5 2^52
+//            count, T_k (k >= 1) a 64-bit fixed-point sum: T_k 2^48 + 1.5 2^52
 //            in one FMA leaves the integer in the low mantissa bits, so the
 //            raw bits are added with ds_add_u64 and count x bits(1.5 2^52) is
-//            subtracted once at the end.  s is as large as the run's pairs
-//            allow (62 - log2 of them, 48 at most), so the sum cannot overflow
-//            and a moment is rounded at 2^-(s+1) per pair; integer sums do
-//            not depend on their order.  ds_add_u64 on random bins takes 11.4
+//            subtracted at the end.  A moment is rounded at 2^-49 per pair
+//            whatever the structure's size: the waves meet every kStageJ J atoms,
+//            and before a bin could pass 32,767 pairs, where its sums could
+//            overflow, the sums go to the run's slab in FP64 and start again.
+//            ds_add_u64 on random bins takes 11.4
 //            CU cycles a wave, ds_add_u32 6.2, ds_add_f64 21.7 (measured;
 //            an odd 8-byte stride between bins, an even one takes 3 times as
 //            long): the kernel is bound by these LDS atomics, its ~45 VALU
@@ -38,6 +39,10 @@ namespace debye {
 constexpr int kMBlock = 1024;
 constexpr double kMagic = 6755399441055744.0;            // 1.5 * 2^52
 constexpr unsigned long long kMagicBits = 0x4338000000000000ull;
+constexpr unsigned kStageJ = 16;                     // J atoms between two looks at the counts
+constexpr unsigned kStagePairs = kMBlock * kStageJ;  // in one bin at most
+constexpr unsigned kMaxPairs = 32767;                // |sum of T_k 2^48| < 2^63
+static_assert(kStagePairs < kMaxPairs, "a stage must fit");
 constexpr double kTwoPi = 6.283185307179586476925286766559;
 
 __device__ __forceinline__ double lane_value(double v, int lane) {
@@ -63,7 +68,7 @@ template <int K>
 __global__ __launch_bounds__(kMBlock) void moments_kernel(
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const Run *__restrict__ runs, double *__restrict__ slabs, double inv_h, unsigned nb,
-    double scale, double unscale, unsigned sub_shift) {
+    unsigned sub_shift) {
   extern __shared__ unsigned long long mom[];  // [nb][K - 1], K - 1 odd
   uint32_t *cnt = reinterpret_cast<uint32_t *>(mom + (size_t)nb * (K - 1));
   double *near = reinterpret_cast<double *>(cnt + ((nb + 1) & ~1u));
@@ -75,10 +80,33 @@ __global__ __launch_bounds__(kMBlock) void moments_kernel(
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned TA = (run.cntA + kMTile - 1) / kMTile, TB = (run.cntB + kMTile - 1) / kMTile;
   const unsigned jr = kMTile >> sub_shift;
+  double *slab = slabs + (size_t)blockIdx.x * ((size_t)nb + 1) * K;
+  // The sums so far, added to the slab (the first time: stored) by the whole work
+  // group; they start again from zero.
+  bool stored = false;
+  auto flush = [&]() {
+    for (unsigned e = threadIdx.x; e < nb * K; e += kMBlock) {
+      const unsigned b = e / K, k = e % K;
+      const unsigned long long n = cnt[b];
+      double v = (double)n;
+      if (k) {
+        unsigned long long *p = mom + b * (K - 1) + k - 1;
+        v = (double)(long long)(*p - n * kMagicBits) * 0x1p-48;
+        *p = 0;
+      }
+      slab[e] = stored ? slab[e] + v : v;
+    }
+    stored = true;
+    __syncthreads();
+    for (unsigned b = threadIdx.x; b < nb; b += kMBlock) cnt[b] = 0;
+    __syncthreads();
+  };
   __syncthreads();
-  for (uint64_t m = run.first + wave; m < run.first + run.count; m += kMBlock / 64) {
+  for (uint64_t m0 = run.first; m0 < run.first + run.count; m0 += kMBlock / 64) {
+    const uint64_t m = m0 + wave;
+    const bool item = m < run.first + run.count;  // (else the wave only meets the others)
     const unsigned sub = (unsigned)m & ((1u << sub_shift) - 1);
-    const TilePair tp = tile_pair(m >> sub_shift, TB, run.diag);
+    const TilePair tp = tile_pair((item ? m : m0) >> sub_shift, TB, run.diag);
     const unsigned ti = __builtin_amdgcn_readfirstlane(tp.ti), tj = __builtin_amdgcn_readfirstlane(tp.tj);
     // a tile is every TA-th (TB-th) atom: the lanes' distances to a J atom then
     // spread over the bins
@@ -90,51 +118,50 @@ __global__ __launch_bounds__(kMBlock) void moments_kernel(
     // J atoms this lane pairs with: all, or those after its own atom
     const unsigned jmin = ia >= run.cntA ? 0xffffffffu
                           : (run.diag && ti == tj) ? lane + 1 : 0u;
-    const unsigned j1 = min(sub * jr + jr, (run.cntB - tj + TB - 1) / TB);
-    for (unsigned j = sub * jr; j < j1; ++j) {
-      const double dx = xi - lane_value(xj, j), dy = yi - lane_value(yj, j),
-                   dz = zi - lane_value(zj, j);
-      const double s = fma(dx, dx, fma(dy, dy, dz * dz));
-      if (j >= jmin && s > 0.0) {
-        const double r = root(s);
-        const double u = r * inv_h;
-        const unsigned b = min((unsigned)u, nb - 1);
-        const double t = fma(2.0, __builtin_amdgcn_fract(u), -1.0);
-        __hip_atomic_fetch_add(&cnt[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        unsigned long long *p = mom + b * (K - 1);
-        double tp0 = 1.0, tp1 = t;
-        const double t2 = t + t;
+    const unsigned jend = item ? min(sub * jr + jr, (run.cntB - tj + TB - 1) / TB) : 0u;
+    for (unsigned j0 = sub * jr; j0 < sub * jr + jr; j0 += kStageJ) {
+      const unsigned j1 = min(j0 + kStageJ, jend);
+      for (unsigned j = j0; j < j1; ++j) {
+        const double dx = xi - lane_value(xj, j), dy = yi - lane_value(yj, j),
+                     dz = zi - lane_value(zj, j);
+        const double s = fma(dx, dx, fma(dy, dy, dz * dz));
+        if (j >= jmin && s > 0.0) {
+          const double r = root(s);
+          const double u = r * inv_h;
+          const unsigned b = min((unsigned)u, nb - 1);
+          const double t = fma(2.0, __builtin_amdgcn_fract(u), -1.0);
+          __hip_atomic_fetch_add(&cnt[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          unsigned long long *p = mom + b * (K - 1);
+          double tp0 = 1.0, tp1 = t;
+          const double t2 = t + t;
 #pragma unroll
-        for (int k = 1; k < K; ++k) {
-          const unsigned long long v = __double_as_longlong(fma(tp1, scale, kMagic));
-          __hip_atomic_fetch_add(p + k - 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          const double tn = fma(t2, tp1, -tp0);
-          tp0 = tp1;
-          tp1 = tn;
-        }
-        if (b == 0) {
-          double a0 = 1.0, a1 = t;
-          const double ir = 1.0 / r;
-          for (int k = 0; k < K; ++k) {
-            __hip_atomic_fetch_add(near + k, a0 * ir, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            const double an = fma(t2, a1, -a0);
-            a0 = a1;
-            a1 = an;
+          for (int k = 1; k < K; ++k) {
+            const unsigned long long v = __double_as_longlong(fma(tp1, 0x1p48, kMagic));
+            __hip_atomic_fetch_add(p + k - 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            const double tn = fma(t2, tp1, -tp0);
+            tp0 = tp1;
+            tp1 = tn;
+          }
+          if (b == 0) {
+            double a0 = 1.0, a1 = t;
+            const double ir = 1.0 / r;
+            for (int k = 0; k < K; ++k) {
+              __hip_atomic_fetch_add(near + k, a0 * ir, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+              const double an = fma(t2, a1, -a0);
+              a0 = a1;
+              a1 = an;
+            }
           }
         }
       }
+      __syncthreads();
+      bool full = false;
+      for (unsigned b = threadIdx.x; b < nb; b += kMBlock) full |= cnt[b] > kMaxPairs - kStagePairs;
+      if (__syncthreads_or(full)) flush();
     }
   }
-  __syncthreads();
-  double *slab = slabs + (size_t)blockIdx.x * ((size_t)nb + 1) * K;
-  for (unsigned e = threadIdx.x; e < nb * K; e += kMBlock) {
-    const unsigned b = e / K, k = e % K;
-    const unsigned long long n = cnt[b];
-    double v = (double)n;
-    if (k) v = (double)(long long)(mom[b * (K - 1) + k - 1] - n * kMagicBits) * unscale;
-    slab[e] = v;
-  }
+  flush();
   if (threadIdx.x < K) slab[(size_t)nb * K + threadIdx.x] = near[threadIdx.x];
 }
 
@@ -245,12 +272,11 @@ namespace {
 
 template <int K>
 int launch_moments(hipStream_t st, unsigned nruns, size_t lds, const double *xyz, size_t n,
-                   const Run *runs, double *slabs, const nodes::Bins &b, int s, unsigned shift) {
+                   const Run *runs, double *slabs, const nodes::Bins &b, unsigned shift) {
   XS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&moments_kernel<K>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMLds));
   hipLaunchKernelGGL(moments_kernel<K>, dim3(nruns), dim3(kMBlock), lds, st, xyz, xyz + n,
-                     xyz + 2 * n, runs, slabs, 1.0 / b.h, b.nb, std::ldexp(1.0, s),
-                     std::ldexp(1.0, -s), shift);
+                     xyz + 2 * n, runs, slabs, 1.0 / b.h, b.nb, shift);
   return XS_OK;
 }
 
@@ -273,10 +299,6 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
   const std::vector<Run> &runs = T.runs;
   const std::vector<uint32_t> &row_run = T.row_run;
   const unsigned shift = T.shift;
-  // |T_k 2^s + ...| <= 2^s per pair: a run's sum stays below 2^62
-  const double run_pairs = (double)T.longest * kMTile * (kMTile >> shift);
-  const int s = std::min(48, 62 - (int)std::ceil(std::log2(run_pairs + 1.0)));
-
   const size_t entries = b.entries();
   char *w = static_cast<char *>(work);
   const size_t rb = runs.size() * sizeof(Run), wb = row_run.size() * 4;
@@ -302,13 +324,13 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
     const unsigned nr = (unsigned)runs.size();
     const size_t lds = moments_lds_bytes(b.nb, b.K);
     switch (b.K) {
-      case 6: XS_TRY(launch_moments<6>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      case 8: XS_TRY(launch_moments<8>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      case 10: XS_TRY(launch_moments<10>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      case 12: XS_TRY(launch_moments<12>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      case 14: XS_TRY(launch_moments<14>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      case 18: XS_TRY(launch_moments<18>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
-      default: XS_TRY(launch_moments<24>(st, nr, lds, xyz, n, runs_d, slabs, b, s, shift)); break;
+      case 6: XS_TRY(launch_moments<6>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 8: XS_TRY(launch_moments<8>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 10: XS_TRY(launch_moments<10>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 12: XS_TRY(launch_moments<12>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 14: XS_TRY(launch_moments<14>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 18: XS_TRY(launch_moments<18>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      default: XS_TRY(launch_moments<24>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
     }
     hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((entries + 63) / 64), nrows), dim3(1024), 0, st,
                        slabs, row_d, (unsigned)entries, M);
@@ -328,17 +350,6 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
   }
   XS_HIP_CHECK(hipGetLastError());
   return prof_end(ctx, "debye", ev);
-}
-
-size_t moments_table_bytes(const std::vector<uint32_t> &seg_cnt, unsigned n_el, unsigned nblocks,
-                           int cus) {
-  const size_t nparts = (size_t)nblocks * (nblocks + 1) / 2;
-  const size_t rows = (size_t)ntypes_of(n_el) * nparts;
-  double n = 0.0;
-  for (uint32_t c : seg_cnt) n += c;
-  const size_t tiles = (size_t)(n / kMTile) + seg_cnt.size();
-  const size_t by_cap = (size_t)((double)tiles * (double)tiles / 2 / 4096.0) + 1;
-  return align_up((6 * rows + cus + by_cap) * sizeof(Run), 256) + (rows + 1) * 4;
 }
 
 }  // namespace debye

@@ -44,7 +44,6 @@ struct RunTables {
   std::vector<Run> runs;
   std::vector<uint32_t> row_run;  // row r has the runs row_run[r] .. row_run[r + 1] - 1
   unsigned shift = 0;             // a tile pair is 2^shift items
-  uint64_t longest = 1;           // items of the longest run
 };
 
 inline size_t moments_lds_bytes(unsigned nb, int K) {
@@ -69,6 +68,12 @@ inline double direct_cycles(double pairs, unsigned nq, double cus) {
   return pairs * std::ceil(nq / 1024.0) * 1024.0 * (3.28 / 0.67) / 64.0 / cus + 60000.0;
 }
 
+// The runs of a call at most, and the bytes of their tables.
+inline size_t max_runs(size_t rows, int cus) { return std::max<size_t>((unsigned)cus, 4 * rows); }
+inline size_t moments_table_bytes(size_t rows, int cus) {
+  return (max_runs(rows, cus) * sizeof(Run) + 255) / 256 * 256 + (rows + 1) * 4;
+}
+
 // Whether the moments take fewer cycles than debye_kernel for these inputs
 // (and fit), and with how many of them.  seg_cnt: atoms of each (element,
 // block), element-major.
@@ -89,8 +94,8 @@ inline bool plan_moments(const MeshBox &in, const std::vector<uint32_t> &seg_cnt
   for (int K : kMoments) {
     const nodes::Bins b = nodes::bins_for(in.R, in.Q, K);
     if (b.nb > 1000000u || moments_lds_bytes(b.nb, K) > kMLds) continue;
-    // each segment pair has at least one slab
-    const double slabs = (5.0 * rows + cus) * (double)b.entries() * 8.0;
+    // (a slab per run, and the rows' sums)
+    const double slabs = ((double)max_runs((size_t)rows, cus) + rows) * (double)b.entries() * 8.0;
     if (slabs > (double)(size_t(1) << 30)) continue;
     const double c = moments_cycles(pairs, rows, rgroups, nq, b, cus);
     if (c < best) {
@@ -134,9 +139,7 @@ inline RunTables plan_runs(const std::vector<uint32_t> &seg_cnt, unsigned n_el, 
   // shares of a tile pair, so that every wave of the chip has a few items
   while (T.shift < 3 && (total << T.shift) < 64ull * (unsigned)cus) ++T.shift;
   // runs: the shortest longest run for which the segment pairs' runs fill one
-  // round of work groups (two runs a segment pair where those are many), at
-  // most 2^24 pairs each (the fixed-point sums)
-  const double cap = 16777216.0 / (kMTile * kMTile);
+  // round of work groups (two runs a segment pair where those are many)
   const uint64_t most = std::max<uint64_t>((unsigned)cus, 2 * sp.size());
   double low = 0.0, per = std::max(1.0, (double)total);
   for (int it = 0; it < 50; ++it) {
@@ -145,7 +148,6 @@ inline RunTables plan_runs(const std::vector<uint32_t> &seg_cnt, unsigned n_el, 
     for (const SegPair &v : sp) nr += (uint64_t)std::ceil((double)pair_tiles(v) / mid);
     (nr <= most ? per : low) = mid;
   }
-  per = std::min(per, cap);
   T.row_run.assign(nrows + 1, 0);
   for (const SegPair &v : sp) {
     const uint64_t t = pair_tiles(v) << T.shift;
@@ -157,7 +159,6 @@ inline RunTables plan_runs(const std::vector<uint32_t> &seg_cnt, unsigned n_el, 
         if (e == f) continue;
         T.runs.push_back(Run{f, e - f, off[v.a], seg_cnt[v.a], off[v.b], seg_cnt[v.b],
                              v.a == v.b ? 1u : 0u, 0u});
-        T.longest = std::max(T.longest, e - f);
         f = e;
       }
     }

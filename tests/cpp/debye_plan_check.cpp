@@ -40,7 +40,7 @@ static void check_runs(const std::vector<uint32_t> &cnt, unsigned n_el, unsigned
     const bool same = i && T.runs[i - 1].offA == r.offA && T.runs[i - 1].offB == r.offB;
     const uint64_t all = (r.diag ? tiles(r.cntA) * (tiles(r.cntA) + 1) / 2 : tiles(r.cntA) * tiles(r.cntB)) << T.shift;
     CHECK(r.first == (same ? next : 0), "run %zu starts at %llu", i, (unsigned long long)r.first);
-    CHECK(r.count > 0 && r.first + r.count <= all && r.count <= T.longest, "run %zu", i);
+    CHECK(r.count > 0 && r.first + r.count <= all, "run %zu", i);
     next = r.first + r.count;
     const bool last = i + 1 == T.runs.size() || T.runs[i + 1].offA != r.offA || T.runs[i + 1].offB != r.offB;
     CHECK(!last || next == all, "segment pair ends at %llu of %llu", (unsigned long long)next,
@@ -50,6 +50,7 @@ static void check_runs(const std::vector<uint32_t> &cnt, unsigned n_el, unsigned
   CHECK(total == expect, "%llu items of %llu", (unsigned long long)total, (unsigned long long)expect);
   const size_t rows = (size_t)n_el * (n_el + 1) / 2 * nblocks * (nblocks + 1) / 2;
   CHECK(T.row_run.size() == rows + 1 && T.row_run[rows] == T.runs.size(), "rows");
+  CHECK(T.runs.size() <= max_runs(rows, cus), "%zu runs", T.runs.size());
   for (size_t r = 0; r < rows; ++r) CHECK(T.row_run[r] <= T.row_run[r + 1], "row %zu", r);
   std::printf("runs of %zu segments: %zu, items %llu\n", cnt.size(), T.runs.size(),
               (unsigned long long)total);

@@ -151,7 +151,8 @@ int xs_pdf(xs_ctx *ctx, const uint64_t *hist, unsigned n_el,
 
 /* H5: direct Debye pair sums S[p*nq+iq] = sum_{pairs in p} sin(q r)/(q r + 1e-8)
  * with FP64 pair terms (xyz double).  Where that is cheaper the sums go
- * through Chebyshev moments of the pair distances (5e-13 a pair); else, on a
+ * through Chebyshev moments of the pair distances, to the FP64 rounding of a
+ * pair's term; else, on a
  * uniform q mesh (the reference's, ReadXML.cpp:220-222) sin(q r) advances
  * from q to q by a rotation, and other meshes evaluate the series per q.
  * Replaces the pair loop of calcIntDebye

@@ -43,25 +43,12 @@ constexpr unsigned kStageJ = 16;                     // J atoms between two look
 constexpr unsigned kStagePairs = kMBlock * kStageJ;  // in one bin at most
 constexpr unsigned kMaxPairs = 32767;                // |sum of T_k 2^48| < 2^63
 static_assert(kStagePairs < kMaxPairs, "a stage must fit");
-constexpr double kTwoPi = 6.283185307179586476925286766559;
 
 __device__ __forceinline__ double lane_value(double v, int lane) {
   const unsigned long long u = __double_as_longlong(v);
   const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)u, lane);
   const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
   return __longlong_as_double(((unsigned long long)hi << 32) | lo);
-}
-
-// sqrt(s) to within an ulp or two for normal s: v_rsq_f64, one Goldschmidt
-// step and one residual correction (the IEEE root's range scaling and its
-// last-bit fix are not needed: an ulp of r is the rounding of its inputs).
-__device__ __forceinline__ double root(double s) {
-  const double y = __builtin_amdgcn_rsq(s);
-  double g = s * y, h = 0.5 * y;
-  const double e = fma(-h, g, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  return fma(fma(-g, g, s), h, g);
 }
 
 template <int K>
@@ -126,7 +113,7 @@ __global__ __launch_bounds__(kMBlock) void moments_kernel(
                      dz = zi - lane_value(zj, j);
         const double s = fma(dx, dx, fma(dy, dy, dz * dz));
         if (j >= jmin && s > 0.0) {
-          const double r = root(s);
+          const double r = sqrt(s);
           const double u = r * inv_h;
           const unsigned b = min((unsigned)u, nb - 1);
           const double t = fma(2.0, __builtin_amdgcn_fract(u), -1.0);
@@ -184,37 +171,46 @@ __global__ __launch_bounds__(1024) void reduce_kernel(const double *__restrict__
   }
 }
 
-// Clears S; 1/q and e/q_c of every q.  On a uniform mesh q_c is the centre of
-// the q's group of 4, counted within blocks of 32 (debye_kernel's weights).
-__global__ void mesh_kernel(const double *__restrict__ q, unsigned nq, double dq, int uniform,
-                            double2 *__restrict__ qe, double *__restrict__ S, size_t ssize) {
-  const size_t n = gridDim.x * (size_t)blockDim.x;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < std::max<size_t>(nq, ssize);
-       i += n) {
-    if (i < ssize) S[i] = 0.0;
-    if (i < nq) {
-      const double v = q[i];
-      double c = v;
-      if (uniform) c = fma((double)((i % 32) / 4 * 4) + 1.5, dq, q[i / 32 * 32]);
-      qe[i] = make_double2(v == 0.0 ? 0.0 : 1.0 / v, c > 0.0 ? 1e-8 / c : 0.0);
-    }
-  }
+// e / q_c of q point i.  On a uniform mesh q_c is the centre of the point's group of
+// 4, counted within blocks of 32 (debye_kernel's weights).
+struct Mesh {
+  const double *q;
+  unsigned nq;
+  double dq;
+  int uniform;
+};
+__device__ __forceinline__ double eps_over_q(const Mesh &m, unsigned i) {
+  const double c = m.uniform ? fma((double)((i % 32) / 4 * 4) + 1.5, m.dq, m.q[i / 32 * 32]) : m.q[i];
+  return c > 0.0 ? 1e-8 / c : 0.0;
 }
 
-// S[row][q] += sum over a chunk's nodes; grid (chunks, q blocks, row groups).
+// hi + lo += v, without an error in hi + lo (Knuth's two-sum).
+__device__ __forceinline__ void add_exact(double &hi, double &lo, double v) {
+#pragma clang fp contract(off)
+  const double s = hi + v, b = s - hi;
+  lo += (hi - (s - b)) + (v - b);
+  hi = s;
+}
+
+// part[share][row][q] = q times the sum over a share's nodes, chunk by chunk (every
+// gridDim.x-th); grid (shares, q blocks, row groups).
+// A node stands for many pairs, so its phase q r is carried beyond FP64 (turn: h / 2 pi
+// in two parts): rounded, as a single pair's may be, its error would be the same for
+// all of them.  And the nodes run along r, so that the sum grows to many times its
+// end value and back at low q: the sums of 8 nodes are added up without rounding.
+// 1,500 atoms, q to 20 1/A: 1.2e-16 sqrt(pairs) at high q and 2e-15 max |S| at low q, as
+// the sums pair by pair; 2e-15 and 6e-14 with neither.
 constexpr int kEvalNodes = 64;
+constexpr unsigned kExactNodes = 4;  // whose sum is rounded
 template <int RG>
 __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M, unsigned nb, int K,
-                                                   unsigned cb, double h, unsigned nrows,
-                                                   const double *__restrict__ q,
-                                                   const double2 *__restrict__ qe, unsigned nq,
-                                                   double *__restrict__ S) {
+                                                   unsigned cb, double h, double2 turn, unsigned nrows,
+                                                   Mesh mesh, double *__restrict__ part) {
   __shared__ double2 tab[64];
   __shared__ double ct[kMaxMoments * kMaxMoments];  // T_k(t_m) 2/K (k = 0: 1/K)
-  __shared__ double4 node[kEvalNodes];              // r/2pi, weight of 1, weight of -e/q_c
+  __shared__ double4 node[kEvalNodes];              // r/2pi, weight of 1, of -e/q_c; rest of r/2pi
   __shared__ double W[kEvalNodes][RG];
-  const unsigned b0 = blockIdx.x * cb, nbin = min(cb, nb + 1 - b0);
-  const unsigned row0 = blockIdx.z * RG;
+  const unsigned row0 = blockIdx.z * RG, iq = blockIdx.y * 256 + threadIdx.x, nq = mesh.nq;
   if (threadIdx.x < 64) {
     double s, c;
     sincos_2pi((double)threadIdx.x / 64.0, &s, &c);
@@ -226,45 +222,80 @@ __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M,
     sincos_2pi((double)((k * (2 * m + 1)) % (4 * K)) / (double)(4 * K), &s, &c);
     ct[i] = (k ? 2.0 * c : 1.0) / K;
   }
-  __syncthreads();
-  for (unsigned i = threadIdx.x; i < nbin * K; i += 256) {
-    const unsigned b = b0 + i / K;
-    const int m = i % K;
-    const double t = 0.5 * K * ct[m * K + 1];
-    const double r = ((b == nb ? 0.0 : (double)b) + 0.5 + 0.5 * t) * h, ir = 1.0 / r;
-    node[i] = make_double4(r / kTwoPi, b == nb ? 0.0 : ir,
-                           b == nb ? ir : b == 0 ? 0.0 : ir * ir, 0.0);
-  }
-  for (unsigned i = threadIdx.x; i < nbin * K * RG; i += 256) {
-    const unsigned n = i / RG, g = i % RG, row = row0 + g;
-    double w = 0.0;
-    if (row < nrows) {
-      const double *mk = M + ((size_t)row * (nb + 1) + b0 + n / K) * K;
-      const double *c = ct + (n % K) * K;
-      for (int k = 0; k < K; ++k) w = fma(mk[k], c[k], w);
+  const double qv = iq < nq ? mesh.q[iq] : 0.0, eq = iq < nq ? eps_over_q(mesh, iq) : 0.0;
+  double sum[RG], rest[RG];
+#pragma unroll
+  for (int g = 0; g < RG; ++g) sum[g] = rest[g] = 0.0;
+  for (unsigned b0 = blockIdx.x * cb; b0 <= nb; b0 += gridDim.x * cb) {
+    const unsigned nbin = min(cb, nb + 1 - b0);
+    __syncthreads();
+    for (unsigned i = threadIdx.x; i < nbin * K; i += 256) {
+      const unsigned b = b0 + i / K;
+      const int m = i % K;
+      const double t = 0.5 * K * ct[m * K + 1];
+      // r / h as x + dx (t to FP64: its bin's share of the distance is small)
+      const double c = (b == nb ? 0.0 : (double)b) + 0.5, x = fma(0.5, t, c);
+      const double dx = fma(0.5, t, c - x), ir = 1.0 / (x * h), rt = x * turn.x;
+      node[i] = make_double4(rt, b == nb ? 0.0 : ir, b == nb ? ir : b == 0 ? 0.0 : ir * ir,
+                             fma(x, turn.x, -rt) + fma(x, turn.y, dx * turn.x));
     }
-    W[n][g] = w;
-  }
-  __syncthreads();
-  const unsigned iq = blockIdx.y * 256 + threadIdx.x;
-  const double qv = iq < nq ? q[iq] : 0.0;
-  const double2 e = iq < nq ? qe[iq] : make_double2(0.0, 0.0);
-  double acc[RG];
+    for (unsigned i = threadIdx.x; i < nbin * K * RG; i += 256) {
+      const unsigned n = i / RG, g = i % RG, row = row0 + g;
+      double w = 0.0;
+      if (row < nrows) {
+        const double *mk = M + ((size_t)row * (nb + 1) + b0 + n / K) * K;
+        const double *c = ct + (n % K) * K;
+        for (int k = 0; k < K; ++k) w = fma(mk[k], c[k], w);
+      }
+      W[n][g] = w;
+    }
+    __syncthreads();
+    for (unsigned n0 = 0; n0 < nbin * K; n0 += kExactNodes) {
+      double acc[RG];
 #pragma unroll
-  for (int g = 0; g < RG; ++g) acc[g] = 0.0;
-  for (unsigned n = 0; n < nbin * K; ++n) {
-    const double4 v = node[n];
-    double s, c;
-    sincos_2pi_tab(qv * v.x, tab, &s, &c);
-    const double f = s * fma(-e.y, v.z, v.y);
+      for (int g = 0; g < RG; ++g) acc[g] = 0.0;
+      for (unsigned n = n0; n < min(n0 + kExactNodes, nbin * K); ++n) {
+        const double4 v = node[n];
+        double s, c;
+        sincos_turn_tab(fma(qv, v.w, fma(qv, v.x, -rint(qv * v.x))), tab, &s, &c);
+        const double f = s * fma(-eq, v.z, v.y);
 #pragma unroll
-    for (int g = 0; g < RG; ++g) acc[g] = fma(W[n][g], f, acc[g]);
+        for (int g = 0; g < RG; ++g) acc[g] = fma(W[n][g], f, acc[g]);
+      }
+#pragma unroll
+      for (int g = 0; g < RG; ++g) add_exact(sum[g], rest[g], acc[g]);
+    }
   }
   if (iq >= nq) return;
 #pragma unroll
   for (int g = 0; g < RG; ++g)
-    if (row0 + g < nrows && acc[g] != 0.0)
-      atomicAdd(&S[(size_t)(row0 + g) * nq + iq], acc[g] * e.x);
+    if (row0 + g < nrows)
+      part[((size_t)blockIdx.x * nrows + row0 + g) * nq + iq] = sum[g] + rest[g];
+}
+
+// S[row][q] = sum of the shares / q (part may be S itself: one share); 64 q and 16
+// threads a q per work group, grid (q blocks, rows).
+__global__ __launch_bounds__(1024) void finish_kernel(const double *part, unsigned shares,
+                                                      const double *__restrict__ q, unsigned nq,
+                                                      double *S) {
+  __shared__ double ph[16][64], pl[16][64];
+  const unsigned i = threadIdx.x & 63, g = threadIdx.x >> 6, iq = blockIdx.x * 64 + i;
+  const size_t at = (size_t)blockIdx.y * nq + iq, stride = (size_t)gridDim.y * nq;
+  double hi = 0.0, lo = 0.0;
+  if (iq < nq) {
+#pragma unroll 4
+    for (unsigned x = g; x < shares; x += 16) add_exact(hi, lo, part[x * stride + at]);
+  }
+  ph[g][i] = hi;
+  pl[g][i] = lo;
+  __syncthreads();
+  if (g || iq >= nq) return;
+  for (unsigned k = 1; k < 16; ++k) {
+    add_exact(hi, lo, ph[k][i]);
+    lo += pl[k][i];
+  }
+  const double qv = q[iq];
+  S[at] = qv == 0.0 ? 0.0 : (hi + lo) / qv;
 }
 
 // ---------------------------------------------------------------- host side
@@ -276,15 +307,17 @@ int launch_moments(hipStream_t st, unsigned nruns, size_t lds, const double *xyz
   XS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&moments_kernel<K>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMLds));
   hipLaunchKernelGGL(moments_kernel<K>, dim3(nruns), dim3(kMBlock), lds, st, xyz, xyz + n,
-                     xyz + 2 * n, runs, slabs, 1.0 / b.h, b.nb, shift);
+                     xyz + 2 * n, runs, slabs, b.inv_h, b.nb, shift);
   return XS_OK;
 }
 
 template <int RG>
 void launch_eval(hipStream_t st, dim3 grid, const double *M, const nodes::Bins &b, unsigned cb,
-                 unsigned nrows, const double *q, const double2 *qe, unsigned nq, double *S) {
-  hipLaunchKernelGGL(eval_kernel<RG>, grid, dim3(256), 0, st, M, b.nb, b.K, cb, b.h, nrows, q, qe,
-                     nq, S);
+                 unsigned nrows, const Mesh &mesh, double *part) {
+  const long double h = b.h(), turn = h / 6.283185307179586476925286766559L;
+  const double hi = (double)turn;
+  hipLaunchKernelGGL(eval_kernel<RG>, grid, dim3(256), 0, st, M, b.nb, b.K, cb, (double)h,
+                     make_double2(hi, (double)(turn - hi)), nrows, mesh, part);
 }
 
 }  // namespace
@@ -307,47 +340,51 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
   std::memcpy(static_cast<char *>(ctx->pin) + align_up(rb, 256), row_run.data(), wb);
   Run *runs_d = reinterpret_cast<Run *>(w);
   uint32_t *row_d = reinterpret_cast<uint32_t *>(w + align_up(rb, 256));
-  XS_TRY(ensure_matrix(ctx, (runs.size() + nrows) * entries * 8 + (size_t)nq * 16 + 1024));
-  double *slabs = static_cast<double *>(ctx->mat);
-  double *M = slabs + runs.size() * entries;
-  double2 *qe = reinterpret_cast<double2 *>(
-      static_cast<char *>(ctx->mat) + align_up((runs.size() + nrows) * entries * 8, 256));
+  // the evaluation: chunks of cb bins (the near pairs' among them), up to 8 rows at once,
+  // as many shares of the chunks as give four work groups a CU
+  const size_t ssize = (size_t)nrows * nq;
+  const unsigned groups = (nrows + 7) / 8, rg = (nrows + groups - 1) / groups;
+  const unsigned cb = std::max(1, kEvalNodes / b.K), chunks = (b.nb + 1 + cb - 1) / cb;
+  const size_t eval_groups = (size_t)((nq + 255) / 256) * ((nrows + rg - 1) / rg);
+  const unsigned shares =
+      runs.empty() ? 0 : (unsigned)std::min<size_t>(chunks, std::max<size_t>(1, 4 * ctx->cu_count / eval_groups));
+  XS_TRY(ensure_matrix(ctx, Carver::need({runs.size() * entries * 8, nrows * entries * 8,
+                                          shares > 1 ? shares * ssize * 8 : 0})));
+  Carver cv(ctx->mat);
+  double *slabs = cv.take<double>(runs.size() * entries), *M = cv.take<double>(nrows * entries);
+  double *part = shares > 1 ? cv.take<double>(shares * ssize) : S;
   hipStream_t st = ctx->stream;
   XS_HIP_CHECK(hipMemcpyAsync(runs_d, ctx->pin, align_up(rb, 256) + wb, hipMemcpyHostToDevice, st));
-  const size_t ssize = (size_t)nrows * nq;
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "debye", &ev));
-  hipLaunchKernelGGL(mesh_kernel,
-                     dim3((unsigned)std::min<size_t>((std::max<size_t>(ssize, nq) + 255) / 256, 4096)),
-                     dim3(256), 0, st, q, nq, in.dq, in.uniform ? 1 : 0, qe, S, ssize);
   if (!runs.empty()) {
     const unsigned nr = (unsigned)runs.size();
     const size_t lds = moments_lds_bytes(b.nb, b.K);
     switch (b.K) {
-      case 6: XS_TRY(launch_moments<6>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
       case 8: XS_TRY(launch_moments<8>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
       case 10: XS_TRY(launch_moments<10>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
       case 12: XS_TRY(launch_moments<12>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
       case 14: XS_TRY(launch_moments<14>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
       case 18: XS_TRY(launch_moments<18>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
-      default: XS_TRY(launch_moments<24>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      case 24: XS_TRY(launch_moments<24>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
+      default: XS_TRY(launch_moments<32>(st, nr, lds, xyz, n, runs_d, slabs, b, shift)); break;
     }
     hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((entries + 63) / 64), nrows), dim3(1024), 0, st,
                        slabs, row_d, (unsigned)entries, M);
-    const unsigned groups = (nrows + 7) / 8, rg = (nrows + groups - 1) / groups;
-    const unsigned cb = std::max(1, kEvalNodes / b.K);
-    const dim3 grid((b.nb + 1 + cb - 1) / cb, (nq + 255) / 256, (nrows + rg - 1) / rg);
+    const dim3 grid(shares, (nq + 255) / 256, (nrows + rg - 1) / rg);
+    const Mesh mesh{q, nq, in.dq, in.uniform ? 1 : 0};
     switch (rg) {
-      case 1: launch_eval<1>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 2: launch_eval<2>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 3: launch_eval<3>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 4: launch_eval<4>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 5: launch_eval<5>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 6: launch_eval<6>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      case 7: launch_eval<7>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
-      default: launch_eval<8>(st, grid, M, b, cb, nrows, q, qe, nq, S); break;
+      case 1: launch_eval<1>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 2: launch_eval<2>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 3: launch_eval<3>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 4: launch_eval<4>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 5: launch_eval<5>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 6: launch_eval<6>(st, grid, M, b, cb, nrows, mesh, part); break;
+      case 7: launch_eval<7>(st, grid, M, b, cb, nrows, mesh, part); break;
+      default: launch_eval<8>(st, grid, M, b, cb, nrows, mesh, part); break;
     }
   }
+  hipLaunchKernelGGL(finish_kernel, dim3((nq + 63) / 64, nrows), dim3(1024), 0, st, part, shares, q, nq, S);
   XS_HIP_CHECK(hipGetLastError());
   return prof_end(ctx, "debye", ev);
 }

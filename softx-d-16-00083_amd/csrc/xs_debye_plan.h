@@ -17,8 +17,8 @@ namespace debye {
 
 constexpr int kMTile = 64;          // atoms per tile: one per lane
 constexpr size_t kMLds = 160000;    // of the CU's 163,840 bytes
-constexpr int kMaxMoments = 24;
-constexpr int kMoments[] = {6, 8, 10, 12, 14, 18, 24};
+constexpr int kMaxMoments = 32;
+constexpr int kMoments[] = {8, 10, 12, 14, 18, 24, 32};
 
 // What the host knows of the inputs: the bounding-box diagonal R, max |q|,
 // the mesh step and whether the mesh is uniform, and whether all coordinates
@@ -58,7 +58,7 @@ inline size_t moments_lds_bytes(unsigned nb, int K) {
 inline double moments_cycles(double pairs, double rows, double rgroups, unsigned nq,
                              const nodes::Bins &b, double cus) {
   const double per_pair = 20.0 * b.K / 64.0;
-  const double node_q = (double)b.entries() * nq * 2.0 * (26.0 * rgroups + 1.5 * rows) / 64.0;
+  const double node_q = (double)b.entries() * nq * 2.0 * (27.0 * rgroups + 3.5 * rows) / 64.0;
   return pairs * per_pair / cus + node_q / cus + (double)b.entries() * 1.5 + 60000.0;
 }
 // 3.28 VALU instructions per pair and q at 67% issue, for q in blocks of 1,024

@@ -57,17 +57,16 @@ __device__ __forceinline__ void sincos_2pi(double r, double *s, double *c) {
   *c = ((q ^ (q >> 1)) & 1) ? -cc : cc;
 }
 
-// sin and cos of 2 pi r for any double r, from a table of the 64 points
-// k/64 of a turn (tab[k] = (sin, cos) of 2 pi k/64, within an ulp) and a
-// short series: t = r - rint(r) and u = t - n/64 with n = rint(64 t) are
-// exact (u is a multiple of ulp(t), |u| <= |t|), |u| <= 1/128, so
+// sin and cos of 2 pi t for |t| <= 1/2 (and a little beyond), from a table of
+// the 64 points k/64 of a turn (tab[k] = (sin, cos) of 2 pi k/64, within an ulp)
+// and a short series: u = t - n/64 with n = rint(64 t) is exact (u is a multiple
+// of ulp(t), |u| <= |t|), |u| <= 1/128, so
 // x = 2 pi u lies within 0.0491 rad, where sin through x^9 and cos through
 // x^8 leave truncation errors below 1e-19 relative; then
 // sin(a + x) = sin a cos x + cos a sin x and likewise for cos.  24 VALU
-// instructions and one LDS read against 37 for the quarter-turn series of
-// sincos_2pi, with the same few-ulp result.
-__device__ __forceinline__ void sincos_2pi_tab(double r, const double2 *tab, double *s, double *c) {
-  const double t = r - rint(r);
+// instructions and one LDS read (of sincos_2pi_tab) against 37 for the
+// quarter-turn series of sincos_2pi, with the same few-ulp result.
+__device__ __forceinline__ void sincos_turn_tab(double t, const double2 *tab, double *s, double *c) {
   const double n = rint(64.0 * t);
   constexpr double kTwoPi = 6.283185307179586476925286766559;
   const double x = kTwoPi * fma(n, -1.0 / 64.0, t);
@@ -83,6 +82,11 @@ __device__ __forceinline__ void sincos_2pi_tab(double r, const double2 *tab, dou
   const double2 a = tab[(int)n & 63];
   *s = fma(a.x, cx, a.y * sx);
   *c = fma(a.y, cx, -(a.x * sx));
+}
+
+// The same for any double r: t = r - rint(r) is exact.
+__device__ __forceinline__ void sincos_2pi_tab(double r, const double2 *tab, double *s, double *c) {
+  sincos_turn_tab(r - rint(r), tab, s, c);
 }
 
 }  // namespace xs

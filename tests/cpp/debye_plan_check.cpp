@@ -5,6 +5,7 @@
 //    in order, also where a segment pair has 2^32 and more of them.
 // 2. tile_pair visits every tile pair of small segments once, and at the ends and
 //    the row boundaries of large ones gives the row and column that hold it.
+// 3. The inputs of the GPU tests of the moments take the moments.
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -56,7 +57,32 @@ static void check_runs(const std::vector<uint32_t> &cnt, unsigned n_el, unsigned
               (unsigned long long)total);
 }
 
+// Inputs of the GPU tests of the moments (tests/test_gpu_debye_moments.py, _coherent.py):
+// they must take them.  R: the diagonal of a box that the atoms nearly fill.
+static void check_taken(const std::vector<uint32_t> &cnt, unsigned n_el, unsigned nblocks, double box,
+                        double Q, unsigned nq) {
+  for (double fill : {0.95, 1.0}) {
+    MeshBox in;
+    in.R = fill * box * std::sqrt(3.0);
+    in.Q = Q;
+    in.finite = true;
+    MomentPlan plan;
+    CHECK(plan_moments(in, cnt, n_el, nblocks, nq, 256, &plan), "pair by pair: box %g, q to %g", box, Q);
+    CHECK(moments_lds_bytes(plan.bins.nb, plan.bins.K) <= kMLds, "LDS of %u bins", plan.bins.nb);
+    std::printf("box %g q %g: %u bins, %d moments\n", box, Q, plan.bins.nb, plan.bins.K);
+  }
+}
+
 int main() {
+  check_taken({1500}, 1, 1, 30.0, 6.0, 400);
+  check_taken({1, 1345, 63, 64, 65}, 5, 1, 40.0, 10.0, 1024);
+  check_taken({1281, 700}, 2, 1, 25.0, 12.0, 777);
+  check_taken({2000, 513}, 2, 1, 120.0, 25.0, 1000);
+  check_taken({3000}, 1, 1, 300.0, 20.0, 1500);
+  check_taken({1500, 321}, 2, 1, 35.0, 14.0, 300);
+  check_taken({400, 400, 400, 300, 300, 300}, 2, 3, 35.0, 14.0, 300);
+  check_taken({1000, 3000}, 2, 1, 10.03, 20.0, 300);
+  check_taken({8192, 8192}, 2, 1, 10.03, 2.0, 300);
   check_runs({1}, 1, 1, 256);
   check_runs({64, 65, 0, 1}, 4, 1, 256);
   check_runs({700, 30, 5000, 64, 0, 129}, 2, 3, 256);

@@ -193,6 +193,10 @@ inline void choose_equal_count(uint32_t ne, const double bbox[6], double cap, bo
         gy = (uint32_t)gb;
       }
     }
+  // No more slabs than atoms, nor columns than atoms of a slab: the others would be
+  // empty (the same tiles), and a few atoms over 2^31 bins have 10^10 of them.
+  gx = std::min(gx, std::max(ne, 1u));
+  gy = std::min(gy, std::max((ne + gx - 1) / gx, 1u));
 }
 
 // Tiles of the equal-count partition (positions from `pos`), column by column.

@@ -227,18 +227,20 @@ __global__ __launch_bounds__(kThreads) void sum_y(Work W) {
   sum_buckets(W.count + l.count0, l.nb, l.start);
 }
 
-__global__ __launch_bounds__(kThreads) void sum_z(Work W) {
-  unsigned lo = 0, hi = W.nslab - 1;
-  while (lo < hi) {
-    const unsigned mid = (lo + hi + 1) / 2;
-    if (W.slabs[mid].col0 <= blockIdx.x)
-      lo = mid;
-    else
-      hi = mid - 1;
+__global__ __launch_bounds__(kThreads) void sum_z(Work W, uint32_t ncols) {
+  for (uint32_t col = blockIdx.x; col < ncols; col += gridDim.x) {
+    unsigned lo = 0, hi = W.nslab - 1;
+    while (lo < hi) {
+      const unsigned mid = (lo + hi + 1) / 2;
+      if (W.slabs[mid].col0 <= col)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    const Slab l = W.slabs[lo];
+    const uint64_t c = col - l.col0;
+    sum_buckets(W.count + l.zcount0 + c * l.znb, l.znb, l.start + (uint32_t)(c * l.n / l.gy));
   }
-  const Slab l = W.slabs[lo];
-  const uint64_t c = blockIdx.x - l.col0;
-  sum_buckets(W.count + l.zcount0 + c * l.znb, l.znb, l.start + (uint32_t)(c * l.n / l.gy));
 }
 
 template <class S, class T>
@@ -341,6 +343,7 @@ template <class S, class T>
 int run(xs_ctx *ctx, const Tables &t, const char *tables, char *scratch, const S *x, const S *y,
         const S *z, T *sx, T *sy, T *sz) {
   if (!t.natoms) return XS_OK;
+  if (t.counters > 0xffffffffull) return fail(XS_ERR_RANGE, "histogram: too many atoms over too many bins");
   Carver cv(scratch);
   Work W{};
   W.segs = reinterpret_cast<const Seg *>(tables);
@@ -366,7 +369,7 @@ int run(xs_ctx *ctx, const Tables &t, const char *tables, char *scratch, const S
   hipLaunchKernelGGL((count_y<S>), atoms, block, 0, st, W, y);
   hipLaunchKernelGGL(sum_y, dim3(W.nslab), block, 0, st, W);
   hipLaunchKernelGGL((count_z<S>), atoms, block, 0, st, W, z);
-  hipLaunchKernelGGL(sum_z, dim3(t.ncols), block, 0, st, W);
+  hipLaunchKernelGGL(sum_z, dim3(std::min(t.ncols, 1u << 20)), block, 0, st, W, t.ncols);
   hipLaunchKernelGGL((put<S, T>), atoms, block, 0, st, W, x, y, z, sx, sy, sz);
   XS_HIP_CHECK(hipGetLastError());
   return XS_OK;

@@ -797,6 +797,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     Args<double> A) {
 #pragma clang fp contract(off)
   __shared__ uint32_t win[WCAP + kTrash];
+  __shared__ uint32_t over;  // pairs past nhist (an item has fewer than 2^32)
   __shared__ unsigned long long keys[kSortCap];
 
   const Item it = A.items[blockIdx.x];
@@ -826,12 +827,12 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
       }
     }
   }
+  unsigned long long *hp = A.hist + td.hist_off;
+  if (tid == 0) over = 0u;
+
   const uint32_t n = it.jcount;
   uint32_t npow = 1;
   while (npow < n) npow <<= 1;
-  unsigned long long *hp = A.hist + td.hist_off;
-  unsigned long long *ovf = A.overflow + td.ovf;
-
   for (uint32_t m = tid; m < npow; m += kTile) {
     unsigned long long key = ~0ull;
     if (m < n) {
@@ -862,8 +863,9 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     }
   }
 
-  // The window holds bins [B, B + WCAP), bin k in slot k - B.
-  uint32_t B = (uint32_t)(keys[0] >> 32);
+  // The window holds bins [B, B + WCAP), bin k in slot k - B; none at or past `top`
+  // has a count.
+  uint32_t B = (uint32_t)(keys[0] >> 32), top = B;
   for (uint32_t s = 0; s < n; ++s) {
     const uint32_t m = (uint32_t)(keys[s] & 0xffffffffu);
     const uint32_t tj = (it.jstart + m) % td.b_n;
@@ -878,12 +880,16 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
       if (ku - B >= (uint32_t)WCAP) {
         // no later tile reaches below kl (they are sorted by it): the window
         // moves up to there at once, so it moves rarely, and the waves meet
-        // only here and not at every tile
+        // only here and not at every tile; rotated if it has counts past kl
         __syncthreads();
-        flush_window<WCAP>(win, B, min(min(kl, B + (uint32_t)WCAP), nhist), 0u - B, hp);
-        rotate_window<WCAP>(win, kl, 0u - B);
+        flush_window<WCAP>(win, B, min(kl, top), 0u - B, hp);
+        if (kl < top)
+          rotate_window<WCAP>(win, kl, 0u - B);
+        else
+          __syncthreads();
         B = kl;
       }
+      top = max(top, ku + 1);
       wlim = min((uint32_t)WCAP, nhist - B);
     }
     const Tile J = A.tiles[tjg];
@@ -1070,14 +1076,15 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
             else if (k < nhist)
               atomicAdd(&hp[k], 1ull);
             else
-              atomicAdd(ovf, 1ull);
+              atomicAdd(&over, 1u);
           }
         }
       }
     }
   }
   __syncthreads();
-  flush_window<WCAP>(win, B, min(B + (uint32_t)WCAP, nhist), 0u - B, hp);
+  if (tid == 0 && over) atomicAdd(A.overflow + td.ovf, (unsigned long long)over);
+  flush_window<WCAP>(win, B, top, 0u - B, hp);
 }
 
 // ---------------------------------------------------------------- host planning

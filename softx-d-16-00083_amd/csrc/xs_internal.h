@@ -80,6 +80,7 @@ struct xs_batch {
   size_t ntypes_total = 0;
   size_t items8192 = 0, items32768 = 0;
   double pairs8192 = 0, pairs32768 = 0;  // pairs of each window class
+  bool few_tiles = false;  // most tiles hold a few atoms
   size_t natoms = 0;      // per axis in the sorted coordinate arrays
   void *coords = nullptr;  // sorted SoA (float or double)
   void *tiles = nullptr, *boxes = nullptr, *types = nullptr, *items = nullptr;

@@ -33,10 +33,10 @@ __global__ void fill_f64(double *__restrict__ p, size_t n) {
     p[i] = 0.0;
 }
 
-// The sums bin by bin, for calls that must not allocate: under stream capture (the
-// graph would keep a pointer to scratch that a later call may move) and where there
-// is no memory for the nodes' tables.  One thread per q and 2,048 bins, chunk sums
-// go to S with atomics: 97,251 bins x 4,096 q 94 us (nodes: 37).
+// The sums bin by bin, for short histograms and for calls that must not allocate:
+// under stream capture (the graph would keep a pointer to scratch that a later call may
+// move) and where there is no memory for the nodes' tables.  One thread per q and 2,048
+// bins, chunk sums go to S with atomics: 97,251 bins x 4,096 q 94 us (nodes: 37).
 //
 // Sum over one staged chunk of bins [k0, k0 + kn) for one q (qv != 0).
 // bins[b] = (h y, h y^2) with y = 1/(k0 + b + 1/2), so that the term
@@ -86,6 +86,15 @@ __device__ __forceinline__ void stage_chunk(double2 *bins, const unsigned long l
     const double y = 1.0 / ((double)(k0 + b) + 0.5), hy = (double)h[b] * y;
     bins[b] = make_double2(hy, hy * y);
   }
+}
+
+// Whether a call takes them: a chunk's time is its chain of bins (15 us a call and 2.9 us
+// per 100 bins, up to the work groups that run at once) against 22 (every bin a node) to
+// 28 us over the nodes.  1 histogram x 300 q: 30 bins 16 us (nodes 22-28), 100 18, 300 24;
+// 1,000 45 (23-29).
+constexpr unsigned kShortBins = 384;
+static bool short_sums(const xs_ctx *ctx, size_t nrows, unsigned nhist_max, unsigned nq) {
+  return nhist_max <= kShortBins && nrows * ((nq + kQBlock - 1) / kQBlock) <= 4 * (size_t)ctx->cu_count;
 }
 
 __global__ __launch_bounds__(kQBlock) void pairsum_kernel(const unsigned long long *__restrict__ hist,
@@ -268,7 +277,7 @@ extern "C" int xs_hist_pairsum(xs_ctx *ctx, const uint64_t *hist, unsigned ntype
   } else {
     const nodesum::Layout L =
         nodesum::layout((ntypes + nodesum::kRows - 1) / nodesum::kRows, nhist, nodesum::kBudget);
-    bool nodes = !(flags & XS_PAIRSUM_F32);
+    bool nodes = !(flags & XS_PAIRSUM_F32) && !iq::short_sums(ctx, ntypes, nhist, nq);
     if (nodes) {
       hipStreamCaptureStatus capture;
       XS_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));

@@ -39,7 +39,7 @@ constexpr unsigned kFew = 8;
 // as many groups and tiles at a time as fit `budget` bytes (at least 16 groups).
 struct Layout {
   size_t plan, rows, nmax, lagrange, node, weights, total;
-  unsigned ntiles, group_cap;  // groups of the longest tile
+  unsigned ntiles, nhist_max, group_cap;  // groups of the longest tile
   unsigned tiles_at_once, groups_at_once;
 };
 Layout layout(unsigned ntiles, unsigned nhist_max, size_t budget);

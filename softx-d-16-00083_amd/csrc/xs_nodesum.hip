@@ -46,10 +46,11 @@ struct PlanArgs {
   Row *rows;  // tables of ntypes histograms of nhist bins, or nullptr
   uint32_t *nmax;
   unsigned ntypes, nhist, ntiles;
+  unsigned limit;  // bins of a group at most
 };
 
-// Bins per group for |q| <= Q: the largest B with Q B bin / 4 <= c.  Every thread
-// of the work group gets the plan.
+// Bins per group for |q| <= Q: the largest B with Q B bin / 4 <= c, at most the limit.
+// Every thread of the work group gets the plan.
 __device__ Plan make_plan(const PlanArgs &A) {
   __shared__ double sh[16];
   double m = 0.0;
@@ -60,7 +61,7 @@ __device__ Plan make_plan(const PlanArgs &A) {
   for (unsigned i = 0; i < blockDim.x / 64; ++i) m = fmax(m, sh[i]);
   const double b = floor(4.0 * A.c / (m * A.bin));
   // (m = 0: infinite; an infinite q: 0)
-  const unsigned bins = b > (double)kMaxBins ? kMaxBins : b > 0.0 ? (unsigned)b : 0u;
+  const unsigned bins = b > (double)A.limit ? A.limit : b > 0.0 ? (unsigned)b : 0u;
   Plan P;
   P.compress = bins > kNodes + kNodes / 2;
   P.bins = P.compress ? bins : kNodes;
@@ -120,15 +121,15 @@ __global__ __launch_bounds__(4 * kNodes) void tables_kernel(PlanArgs A, Plan *__
     if (blockIdx.x == 0) store_plan(A, P, plan);
   }
   const unsigned m = threadIdx.x % kNodes, part = threadIdx.x / kNodes;
-  const unsigned zero0 = kMaxBins / 4 + (group_cap + 3) / 4;
+  const unsigned node0 = (A.limit + 3) / 4, zero0 = node0 + (group_cap + 3) / 4;
   if (blockIdx.x >= zero0) {
     for (size_t i = (blockIdx.x - zero0) * (size_t)blockDim.x + threadIdx.x; i < ssize;
          i += (size_t)(gridDim.x - zero0) * blockDim.x)
       S[i] = 0.0;
     return;
   }
-  if (blockIdx.x >= kMaxBins / 4) {
-    const unsigned g = (blockIdx.x - kMaxBins / 4) * 4 + part;
+  if (blockIdx.x >= node0) {
+    const unsigned g = (blockIdx.x - node0) * 4 + part;
     if (g >= group_cap) return;
     const double r = ((double)group_bins(g) + 0.5) * (double)P.bins + node_offset(P, m);
     const double y = 1.0 / r;
@@ -494,6 +495,7 @@ __global__ __launch_bounds__(256) void few_kernel(const double *__restrict__ W,
 Layout layout(unsigned ntiles, unsigned nhist_max, size_t budget) {
   Layout L{};
   L.ntiles = ntiles;
+  L.nhist_max = nhist_max;
   L.group_cap = align_groups(groups_for(nhist_max, kNodes));
   const size_t group = (size_t)kNodes * kRows * 8;
   L.groups_at_once = (unsigned)std::min<size_t>(L.group_cap, std::max<size_t>(16, budget / group / 16 * 16));
@@ -515,18 +517,27 @@ Layout layout(unsigned ntiles, unsigned nhist_max, size_t budget) {
   return L;
 }
 
-static int tables(xs_ctx *ctx, const Tables &T, double bin, const double *q, unsigned nq, double *S,
-                  size_t ssize) {
+// Bins per group at most.  The weights of a group are one work group's, so large groups
+// take time where there are few (4,096 bins: 85 us for one histogram of 3,000 bins that
+// 15 smaller groups do in 30), and for few_kernel 16 groups cost as much as one.  Where
+// the products are the larger part, only the bound of the tables.
+static unsigned group_limit(unsigned nrows, unsigned nq, unsigned nhist_max) {
+  if (nrows > kFew && (size_t)nrows * nq > 131072) return kMaxBins;
+  return std::min(1024u, std::max(kNodes + kNodes / 2 + 1, (nhist_max + 13) / 14));
+}
+
+static int tables(xs_ctx *ctx, const Tables &T, unsigned limit, double bin, const double *q, unsigned nq,
+                  double *S, size_t ssize) {
   const Layout &L = T.L;
   hipStream_t st = ctx->stream;
   // 2 c^64 / 64! = 1e-15
   const double c = nodes::reach((int)kNodes, 1e-15);
   const PlanArgs A{q, nq, bin, c, T.ntypes ? T.at<Row>(L.rows) : nullptr,
-                   T.ntypes ? T.at<uint32_t>(L.nmax) : nullptr, T.ntypes, T.nhist, L.ntiles};
+                   T.ntypes ? T.at<uint32_t>(L.nmax) : nullptr, T.ntypes, T.nhist, L.ntiles, limit};
   if (nq > kPlanAll)
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, st, A, T.at<Plan>(L.plan));
   const unsigned zb = (unsigned)std::min<size_t>((ssize + 1023) / 1024, 1024);
-  hipLaunchKernelGGL(tables_kernel, dim3(kMaxBins / 4 + (L.group_cap + 3) / 4 + zb), dim3(4 * kNodes), 0,
+  hipLaunchKernelGGL(tables_kernel, dim3((limit + 3) / 4 + (L.group_cap + 3) / 4 + zb), dim3(4 * kNodes), 0,
                      st, A, T.at<Plan>(L.plan), L.group_cap, T.at<double>(L.lagrange),
                      T.at<double2>(L.node), S, ssize);
   XS_HIP_CHECK(hipGetLastError());
@@ -592,7 +603,7 @@ static int sums(xs_ctx *ctx, const Tables &T, unsigned tile0, unsigned ntiles, u
 int run(xs_ctx *ctx, const Tables &T, const unsigned long long *hist, unsigned nrows, double bin,
         const double *q, unsigned nq, double *S) {
   const Layout &L = T.L;
-  XS_TRY(tables(ctx, T, bin, q, nq, S, (size_t)nrows * nq));
+  XS_TRY(tables(ctx, T, group_limit(nrows, nq, L.nhist_max), bin, q, nq, S, (size_t)nrows * nq));
   for (unsigned t = 0; t < L.ntiles; t += L.tiles_at_once)
     for (unsigned g = 0; g < L.group_cap; g += L.groups_at_once) {
       const unsigned nt = std::min(L.tiles_at_once, L.ntiles - t),

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void column_stats(const unsigned long long *__
 // Slices of the sine table: one thread per (q tile, kSincTiles k tiles, lane), 16
 // values a k tile, NA slices of 16 bytes.
 // A value v goes to N = rint(2^34 v) by one addition: 2^34 v + 1.5 2^52 + B holds
-// N + B in its low bits, B = 64 (1 + 2^7 + 2^14 + 2^21), so the slices are the 7-bit
+// N + B in its low bits, B = kSliceBias = 64 (1 + 2^7 + 2^14 + 2^21), so the slices are the 7-bit
 // fields of the low word less 64 and, signed, the bits from 28 on.  Four values share
 // a reciprocal (1/(abcd), two Newton steps), and the sine is advanced by a rotation
 // from bin to bin and over the other half-wave's 16 bins.
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void slice_sinc(const double *__restrict__ q, 
       unsigned lo[4], hi[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        constexpr double kBias = 6755399441055744.0 + 64.0 * (1 + 128 + 16384 + 2097152);
+        constexpr double kBias = 6755399441055744.0 + (double)kSliceBias;
         const bool in = qv != 0.0 && k0 + 4 * g + e < nhist;
         const unsigned long long n =
             (unsigned long long)__double_as_longlong(fma(in ? v[e] : 0.0, 17179869184.0, kBias));
@@ -335,9 +335,9 @@ __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i
     const v4i *bp = Bs + d.b_off;
     const unsigned col0 = d.col0 + wn * NT * 32, colend = min(ncols, d.col0 + d.ncol);
 
-    // Where |q| r > 129 for all of a q tile, every value is below 1/128 and its top slice
-    // is 0: no products with it from k tile ktop on, no loads from the largest ktop of the
-    // work group's q tiles on (kfetch).
+    // Where |q| r > kTopSliceX for all of a q tile, every value's top slice is 0: no
+    // products with it from k tile ktop on, no loads from the largest ktop of the work
+    // group's q tiles on (kfetch).
     unsigned ktop = 0, kfetch = 0;
 #pragma unroll
     for (unsigned m = 0; m < 4; ++m) {
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i
       double a = row < nq ? fabs(q[row]) : 0.0;
       a = a > 0.0 ? a : INFINITY;  // (q = 0: a row of zeros; NaN: as it comes)
       for (int o = 16; o > 0; o >>= 1) a = fmin(a, __shfl_xor(a, o, 64));
-      const double k = 129.0 / (a * bin) * (1.0 / 32.0) + 1.0;
+      const double k = kTopSliceX / (a * bin) * (1.0 / 32.0) + 1.0;
       const unsigned kk = __builtin_amdgcn_readfirstlane(k < 4294967295.0 ? (unsigned)k : ~0u);
       kfetch = max(kfetch, kk);
       if (m == wm) ktop = kk;

@@ -14,6 +14,12 @@ namespace xs {
 constexpr int kMfmaSlicesA = 5;      // int8 slices of the sinc matrix
 constexpr int kMfmaMaxSlicesB = 5;   // 7-bit count slices (counts below 2^35)
 
+// A sinc value v is sliced as N + kSliceBias, N = rint(2^34 v): four 7-bit fields (less
+// 64) and the bits from 28 on as the top slice.  That one is 0 for -127.0 < 1/v or
+// 1/v > 129.016 (N + bias from 0 to 2^28), so beyond |q| r = kTopSliceX whatever the sine.
+constexpr long long kSliceBias = 64ll * (1 + 128 + 16384 + 2097152);
+constexpr double kTopSliceX = 130.0;
+
 // Columns are the pair types, sorted by count slices (most first) and then
 // by bin count (largest first), so that every group of NT column tiles of 32
 // columns shares one slice count and one k range (its largest bin count).

@@ -91,6 +91,11 @@ __global__ __launch_bounds__(256) void column_stats(const unsigned long long *__
   __syncthreads();
   if (threadIdx.x) return;
   l = max(max(pl[0], pl[1]), max(pl[2], pl[3]));
+  if (gridDim.y == 1) {  // (nothing to add to, nothing cleared)
+    bits[blockIdx.x] = (pm[0] | pm[1]) | (pm[2] | pm[3]);
+    last[blockIdx.x] = l;
+    return;
+  }
   if (!l) return;
   atomicOr(&bits[blockIdx.x], (pm[0] | pm[1]) | (pm[2] | pm[3]));
   atomicMax(&last[blockIdx.x], l);
@@ -176,6 +181,20 @@ __global__ __launch_bounds__(256) void slice_sinc(const double *__restrict__ q, 
           (v4i){(int)w[i][0], (int)w[i][1], (int)w[i][2], (int)w[i][3]};
     rotate(js, jc);
   }
+}
+
+// The tables of few columns as arguments of a launch, which takes half the time of a copy.
+constexpr unsigned kInlineCols = 128, kInlineTiles = 16;
+struct InlineTables {
+  MfmaCol cols[kInlineCols];
+  MfmaTile tiles[kInlineTiles];
+};
+static_assert(sizeof(InlineTables) <= 3072, "kernel arguments");
+__global__ __launch_bounds__(128) void put_tables(InlineTables t, MfmaCol *__restrict__ cols, unsigned ncols,
+                                                  MfmaTile *__restrict__ tiles, unsigned ntiles) {
+  const unsigned i = threadIdx.x;
+  if (i < ncols) cols[i] = t.cols[i];
+  if (i < ntiles) tiles[i] = t.tiles[i];
 }
 
 static void launch_slice_sinc(xs_ctx *ctx, const double *q, unsigned nq, unsigned nhist, double bin,
@@ -337,18 +356,22 @@ __global__ __launch_bounds__(256 * WN, 2) void pairsum_mfma_lds_kernel(const v4i
 
     // Where |q| r > kTopSliceX for all of a q tile, every value's top slice is 0: no
     // products with it from k tile ktop on, no loads from the largest ktop of the work
-    // group's q tiles on (kfetch).
-    unsigned ktop = 0, kfetch = 0;
+    // group's q tiles on (kfetch).  (Not asked for 16 k tiles or fewer, whose
+    // products take no longer than finding out, 2 us.)
+    unsigned ktop = ~0u, kfetch = ~0u;
+    if (d.kt > 16) {
+      kfetch = 0;
 #pragma unroll
-    for (unsigned m = 0; m < 4; ++m) {
-      const unsigned row = (mg * 4 + m) * 32 + (lane & 31);
-      double a = row < nq ? fabs(q[row]) : 0.0;
-      a = a > 0.0 ? a : INFINITY;  // (q = 0: a row of zeros; NaN: as it comes)
-      for (int o = 16; o > 0; o >>= 1) a = fmin(a, __shfl_xor(a, o, 64));
-      const double k = kTopSliceX / (a * bin) * (1.0 / 32.0) + 1.0;
-      const unsigned kk = __builtin_amdgcn_readfirstlane(k < 4294967295.0 ? (unsigned)k : ~0u);
-      kfetch = max(kfetch, kk);
-      if (m == wm) ktop = kk;
+      for (unsigned m = 0; m < 4; ++m) {
+        const unsigned row = (mg * 4 + m) * 32 + (lane & 31);
+        double a = row < nq ? fabs(q[row]) : 0.0;
+        a = a > 0.0 ? a : INFINITY;  // (q = 0: a row of zeros; NaN: as it comes)
+        for (int o = 16; o > 0; o >>= 1) a = fmin(a, __shfl_xor(a, o, 64));
+        const double k = kTopSliceX / (a * bin) * (1.0 / 32.0) + 1.0;
+        const unsigned kk = __builtin_amdgcn_readfirstlane(k < 4294967295.0 ? (unsigned)k : ~0u);
+        kfetch = max(kfetch, kk);
+        if (m == wm) ktop = kk;
+      }
     }
     // The tiles of a stage go round the waves: the A tiles (q tile m, slice i > 0) as
     // m (NA - 1) + i - 1, the B tiles (slice j, column tile t) as kB0 + j NT WN + t, and
@@ -492,18 +515,23 @@ static int mm::products(xs_ctx *ctx, const MfmaBatchPlan &plan, const unsigned l
   const unsigned MT = (nq + 127) / 128 * 4, ncols = (unsigned)plan.cols.size();
   for (const MfmaLaunch &L : plan.launches) {
     const unsigned NTg = L.nt * L.wn;
-    const size_t tb = (size_t)L.ntiles * NTg * plan.kt_max * 64;
-    hipLaunchKernelGGL(slice_counts, dim3((unsigned)((tb + 255) / 256)), dim3(256), 0, ctx->stream, hist, cols,
-                       ncols, tiles, L.tile0, L.ntiles, plan.kt_max, (int)L.nb, (int)NTg, Bs,
-                       &L == &plan.launches[0] ? S : nullptr, (size_t)ncols * nq);
+    const size_t tb = (size_t)L.ntiles * NTg * plan.kt_max * 64, ssize = (size_t)ncols * nq;
+    // (the first one clears S: enough work groups for that too, 100 x 4,000 16 -> 3 us)
+    const bool first = &L == &plan.launches[0];
+    const size_t groups = std::max((tb + 255) / 256, first ? std::min<size_t>((ssize + 1023) / 1024, 2048) : 0);
+    hipLaunchKernelGGL(slice_counts, dim3((unsigned)groups), dim3(256), 0, ctx->stream, hist, cols, ncols,
+                       tiles, L.tile0, L.ntiles, plan.kt_max, (int)L.nb, (int)NTg, Bs, first ? S : nullptr,
+                       ssize);
   }
   for (const MfmaLaunch &L : plan.launches) {
-    // as many work groups as run at a time, of 16 k tiles at least
+    // as many work groups as run at a time, of 16 k tiles or one output at least (of
+    // short histograms, 9 x 50 bins x 2,000 q, 16 k tiles alone left 2 work groups)
     unsigned long long work = 0;
     for (uint32_t g = 0; g < L.ntiles; ++g) work += plan.tiles[L.tile0 + g].kt;
     work *= MT / 4;
     const unsigned slots = 2 / L.wn * (unsigned)ctx->cu_count;
-    const dim3 grid((unsigned)std::min<unsigned long long>(slots, std::max(1ull, work / 16)));
+    const unsigned long long outputs = (unsigned long long)L.ntiles * (MT / 4);
+    const dim3 grid((unsigned)std::min<unsigned long long>(slots, std::max(outputs, work / 16)));
     auto gemm = [&](auto launch) {
       launch(L.nb, grid, ctx->stream, As, Bs, MT, L.ntiles, KT, nq, ncols, S, tiles, cols, L.tile0, q, bin);
     };
@@ -527,7 +555,7 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   const unsigned KT = (nhist + 31) / 32;
   const size_t aBytes = (size_t)kNA * MT * KT * 1024;
   XS_TRY(ensure_matrix(ctx, Carver::need({aBytes, (size_t)ncols * 8, (size_t)ncols * 4})));
-  XS_TRY(ensure_pinned(ctx, (size_t)ncols * 12));
+  XS_TRY(ensure_pinned(ctx, align_up((size_t)ncols * 8, 256) + (size_t)ncols * 4));
   Carver cv(ctx->mat);
   v4i *As = cv.take<v4i>(aBytes / 16);
   unsigned long long *bits = cv.take<unsigned long long>(ncols);
@@ -535,16 +563,17 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   hipEvent_t ev;
   XS_TRY(prof_begin(ctx, "pairsum_slices", &ev));
   // every column's slices and extent, read back while the sine's slices are made
+  const unsigned parts = std::min(64u, (nhist + 4095) / 4096);
   const size_t nclear = (size_t)(last + ncols - reinterpret_cast<uint32_t *>(bits));
-  hipLaunchKernelGGL(clear_u32, dim3((unsigned)((nclear + 255) / 256)), dim3(256), 0, ctx->stream,
-                     reinterpret_cast<uint32_t *>(bits), nclear);
-  hipLaunchKernelGGL(column_stats, dim3(ncols, std::min(64u, (nhist + 4095) / 4096)), dim3(256), 0, ctx->stream,
-                     hist, nhist, bits, last);
+  if (parts > 1)
+    hipLaunchKernelGGL(clear_u32, dim3((unsigned)((nclear + 255) / 256)), dim3(256), 0, ctx->stream,
+                       reinterpret_cast<uint32_t *>(bits), nclear);
+  hipLaunchKernelGGL(column_stats, dim3(ncols, parts), dim3(256), 0, ctx->stream, hist, nhist, bits, last);
   XS_HIP_CHECK(hipGetLastError());
+  // (bits and last in one copy: they lie side by side)
   char *const pin = static_cast<char *>(ctx->pin);
-  XS_HIP_CHECK(hipMemcpyAsync(pin, bits, (size_t)ncols * 8, hipMemcpyDeviceToHost, ctx->stream));
-  XS_HIP_CHECK(hipMemcpyAsync(pin + (size_t)ncols * 8, last, (size_t)ncols * 4, hipMemcpyDeviceToHost,
-                              ctx->stream));
+  const size_t last_at = (size_t)(reinterpret_cast<char *>(last) - reinterpret_cast<char *>(bits));
+  XS_HIP_CHECK(hipMemcpyAsync(pin, bits, last_at + (size_t)ncols * 4, hipMemcpyDeviceToHost, ctx->stream));
   if (!ctx->read_back) XS_HIP_CHECK(hipEventCreateWithFlags(&ctx->read_back, hipEventDisableTiming));
   XS_HIP_CHECK(hipEventRecord(ctx->read_back, ctx->stream));
   launch_slice_sinc(ctx, q, nq, nhist, bin, MT, KT, As);
@@ -553,10 +582,19 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   std::vector<unsigned long long> off(ncols), bound(ncols);
   std::vector<uint32_t> extent(ncols);
   std::memcpy(bound.data(), pin, (size_t)ncols * 8);
-  std::memcpy(extent.data(), pin + (size_t)ncols * 8, (size_t)ncols * 4);
+  std::memcpy(extent.data(), pin + last_at, (size_t)ncols * 4);
   for (unsigned c = 0; c < ncols; ++c) off[c] = (unsigned long long)c * nhist;
+  // A small call (not 16 k tiles for every CU): one launch for all slice counts, no waves
+  // side by side, which would halve its few work groups (100 x 100 bins x 4,000 q: 59 us
+  // side by side and with one launch to clear S, 43 so)
+  const bool small = (size_t)(MT / 4) * ((ncols + 127) / 128) * KT < 16 * (size_t)ctx->cu_count;
+  if (small) {
+    unsigned long long all = 0;
+    for (unsigned long long b : bound) all |= b;
+    std::fill(bound.begin(), bound.end(), all);
+  }
   MfmaBatchPlan plan;
-  if (!mfma_batch_plan(off, extent, bound, nq, &plan, true)) {
+  if (!mfma_batch_plan(off, extent, bound, nq, &plan, !small)) {
     XS_TRY(prof_end(ctx, "pairsum_slices", ev));
     return fail(XS_ERR_RANGE, "xs_hist_pairsum: a bin count exceeds 2^35 (matrix-core path)");
   }
@@ -567,9 +605,18 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   MfmaCol *cols = ca.take<MfmaCol>(plan.cols.size());
   MfmaTile *tiles = ca.take<MfmaTile>(plan.tiles.size());
   v4i *Bs = ca.take<v4i>(plan.b_bytes / 16);
-  std::memcpy(ctx->pin, plan.cols.data(), colsb);
-  std::memcpy(static_cast<char *>(ctx->pin) + align_up(colsb, 256), plan.tiles.data(), tilesb);
-  XS_HIP_CHECK(hipMemcpyAsync(cols, ctx->pin, align_up(colsb, 256) + tilesb, hipMemcpyHostToDevice, ctx->stream));
+  if (plan.cols.size() <= kInlineCols && plan.tiles.size() <= kInlineTiles) {
+    InlineTables t{};
+    std::copy(plan.cols.begin(), plan.cols.end(), t.cols);
+    std::copy(plan.tiles.begin(), plan.tiles.end(), t.tiles);
+    hipLaunchKernelGGL(put_tables, dim3(1), dim3(128), 0, ctx->stream, t, cols, (unsigned)plan.cols.size(),
+                       tiles, (unsigned)plan.tiles.size());
+    XS_HIP_CHECK(hipGetLastError());
+  } else {
+    std::memcpy(ctx->pin, plan.cols.data(), colsb);
+    std::memcpy(static_cast<char *>(ctx->pin) + align_up(colsb, 256), plan.tiles.data(), tilesb);
+    XS_HIP_CHECK(hipMemcpyAsync(cols, ctx->pin, align_up(colsb, 256) + tilesb, hipMemcpyHostToDevice, ctx->stream));
+  }
   XS_TRY(prof_end(ctx, "pairsum_slices", ev));
   XS_TRY(prof_begin(ctx, "pairsum_mfma", &ev));
   XS_TRY(products(ctx, plan, hist, cols, tiles, As, Bs, KT, bin, q, nq, S));

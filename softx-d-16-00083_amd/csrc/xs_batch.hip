@@ -6,7 +6,8 @@
 // sorted coordinates, tiles and work items of all structures on the device,
 // so a run is a fixed sequence of launches with no host work:
 //   zero fills -> histogram kernels (8192- then 32768-bin windows)
-//   -> pair sums of all pair types over Chebyshev nodes
+//   -> pair sums of all pair types over Chebyshev nodes, or bin by bin where the
+//   histograms are short or there is no memory for the nodes' tables
 //   -> PDF kernel over all structures' bins.
 // With XS_BATCH_GRAPH the sequence is captured once into a hipGraph on the
 // context's stream and replayed while the output pointers, nq, the PDF type
@@ -33,9 +34,10 @@ void release_batch_run(BatchRunState &r) {
 namespace {
 
 // The run buffer of one call; host-mode staging only when needed, the
-// matrix-core slices when mm (a plan with mm.nq != 0) is given.
+// matrix-core slices when mm (a plan with mm.nq != 0) is given, else the nodes'
+// tables for a run with `nodes`.
 RunLayout layout(const xs_batch *b, unsigned nhist_max, unsigned nq, bool host, bool want_S,
-                 bool want_pdf, const MfmaBatchPlan *mm) {
+                 bool want_pdf, bool nodes, const MfmaBatchPlan *mm) {
   const size_t ntiles = (b->ntypes_total + nodesum::kRows - 1) / nodesum::kRows;
   RunSizes n;
   n.rows = ntiles * nodesum::kRows * sizeof(nodesum::Row);
@@ -53,7 +55,7 @@ RunLayout layout(const xs_batch *b, unsigned nhist_max, unsigned nq, bool host, 
   if (mm) {
     n.mm_a = mm->a_bytes;
     n.mm_b = mm->b_bytes;
-  } else if (want_S) {
+  } else if (nodes) {
     n.nodes = nodesum::layout((unsigned)ntiles, nhist_max, nodesum::kBudget).total;
   }
   return run_layout(n);
@@ -117,7 +119,7 @@ std::vector<unsigned long long> pair_counts(const xs_batch *b) {
 }
 
 int launch_all(xs_batch *b, const RunPtrs &P, const RunLayout &L, unsigned nhist_max, unsigned nq,
-               int pdf_type, unsigned pdf_blocks, bool cpu_radius, bool mfma, bool prof) {
+               int pdf_type, unsigned pdf_blocks, bool cpu_radius, bool mfma, bool nodes, bool prof) {
   char *buf = static_cast<char *>(b->run.buf);
   XS_TRY(batch_hist_launch(b, P.hist, prof));
   if (P.S && mfma)
@@ -128,11 +130,15 @@ int launch_all(xs_batch *b, const RunPtrs &P, const RunLayout &L, unsigned nhist
     hipEvent_t ev = nullptr;
     if (prof) XS_TRY(prof_begin(b->ctx, "batch_pairsum", &ev));
     const unsigned nrows = (unsigned)b->ntypes_total;
-    const nodesum::Tables T{nodesum::layout((nrows + nodesum::kRows - 1) / nodesum::kRows, nhist_max,
-                                            nodesum::kBudget),
-                            buf + L.nodes, 0, 0, reinterpret_cast<const nodesum::Row *>(buf + L.rows),
-                            reinterpret_cast<const uint32_t *>(buf + L.nmax)};
-    XS_TRY(nodesum::run(b->ctx, T, P.hist, nrows, b->bin, P.q, nq, P.S));
+    const auto *rows = reinterpret_cast<const nodesum::Row *>(buf + L.rows);
+    if (nodes) {
+      const nodesum::Tables T{nodesum::layout((nrows + nodesum::kRows - 1) / nodesum::kRows, nhist_max,
+                                              nodesum::kBudget),
+                              buf + L.nodes, 0, 0, rows, reinterpret_cast<const uint32_t *>(buf + L.nmax)};
+      XS_TRY(nodesum::run(b->ctx, T, P.hist, nrows, b->bin, P.q, nq, P.S));
+    } else {
+      XS_TRY(pairsum_rows(b->ctx, P.hist, rows, nrows, nhist_max, b->bin, P.q, nq, P.S));
+    }
     if (prof) XS_TRY(prof_end(b->ctx, "batch_pairsum", ev));
   }
   if (P.pdf)
@@ -182,7 +188,14 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
   unsigned pdf_blocks = 0;
   const std::vector<PdfDesc> desc = make_pdf_desc(plan, want_pdf ? rho0 : nullptr, want_pdf ? sl : nullptr,
                                                   &pdf_blocks);
-  const RunLayout L = layout(plan, rows[0].nhist, nq, !device, want_S, want_pdf, mfma ? &R.mm : nullptr);
+  const unsigned nhist_max = rows[0].nhist;
+  bool nodes = want_S && !mfma && !pairsum_short(ctx, plan->ntypes_total, nhist_max, nq);
+  RunLayout L = layout(plan, nhist_max, nq, !device, want_S, want_pdf, nodes, mfma ? &R.mm : nullptr);
+  auto without_nodes = [&]() {
+    nodes = false;
+    L = layout(plan, nhist_max, nq, !device, want_S, want_pdf, false, nullptr);
+  };
+  if (nodes && L.total >= R.refused) without_nodes();
 
   // (re)allocate the run buffer and upload the descriptors when they change
   if (L.total > R.buf_cap) {
@@ -194,7 +207,14 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
     if (R.buf) XS_HIP_CHECK(hipFree(R.buf));
     R.buf = nullptr;
     R.buf_cap = 0;
-    if (hipMalloc(&R.buf, L.total) != hipSuccess) {
+    hipError_t e = hipMalloc(&R.buf, L.total);
+    if (e != hipSuccess && nodes) {
+      (void)hipGetLastError();
+      R.refused = L.total;  // not asked for again by this plan
+      without_nodes();
+      e = hipMalloc(&R.buf, L.total);
+    }
+    if (e != hipSuccess) {
       R.buf = nullptr;
       (void)hipGetLastError();
       return fail(XS_ERR_NOMEM, "xs_batch_run: device allocation failed");
@@ -248,7 +268,7 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
   const bool cpu_radius = flags & XS_PDF_CPU_RADIUS;
 
   if (!graph) {
-    XS_TRY(launch_all(plan, P, L, rows[0].nhist, nq, pdf_type, pdf_blocks, cpu_radius, mfma, true));
+    XS_TRY(launch_all(plan, P, L, nhist_max, nq, pdf_type, pdf_blocks, cpu_radius, mfma, nodes, true));
   } else {
     const unsigned kflags = flags & (XS_DEVICE_PTRS | XS_PDF_CPU_RADIUS | (mfma ? XS_PAIRSUM_MFMA : 0u));
     const bool same = R.exec && R.key_hist == P.hist && R.key_S == P.S && R.key_pdf == P.pdf &&
@@ -262,7 +282,7 @@ extern "C" int xs_batch_run(xs_batch *plan, uint64_t *hist, const double *q, uns
       R.graph = nullptr;
       XS_HIP_CHECK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
       const int rc =
-          launch_all(plan, P, L, rows[0].nhist, nq, pdf_type, pdf_blocks, cpu_radius, mfma, false);
+          launch_all(plan, P, L, nhist_max, nq, pdf_type, pdf_blocks, cpu_radius, mfma, nodes, false);
       hipGraph_t g = nullptr;
       const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
       if (rc != XS_OK || ec != hipSuccess) {

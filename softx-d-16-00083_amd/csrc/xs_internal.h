@@ -55,6 +55,7 @@ struct BatchRunState {
   std::vector<double> key_rho0, key_sl;
   void *buf = nullptr;   // pair-sum and PDF descriptors, host-mode staging
   size_t buf_cap = 0;
+  size_t refused = SIZE_MAX;  // a size of buf, with the nodes' tables, that could not be had
   bool uploaded = false;     // buf holds the rows and descriptors of key_rho0, key_sl
   MfmaBatchPlan mm;      // XS_PAIRSUM_MFMA: columns, groups, buffer sizes (mm.nq = 0: none)
   bool mm_uploaded = false;  // its tables are in buf

@@ -115,6 +115,31 @@ __global__ __launch_bounds__(kQBlock) void pairsum_kernel(const unsigned long lo
   if (acc != 0.0) atomicAdd(&S[(size_t)p * nq + iq], acc / (qv * bin));
 }
 
+// The same for the rows of a batch plan, of any lengths.  Grid (blocks of 256 q, chunks of
+// the longest row, rows), the last two in strides.
+__global__ __launch_bounds__(kQBlock) void pairsum_rows_kernel(const unsigned long long *__restrict__ hist,
+                                                               const nodesum::Row *__restrict__ rows,
+                                                               unsigned nrows, const double *__restrict__ q,
+                                                               unsigned nq, double bin,
+                                                               double *__restrict__ S) {
+  __shared__ double2 bins[kChunk];
+  const unsigned iq = blockIdx.x * kQBlock + threadIdx.x;
+  const double qv = iq < nq ? q[iq] : 0.0;
+  for (unsigned p = blockIdx.z; p < nrows; p += gridDim.z) {
+    const nodesum::Row r = rows[p];
+    for (unsigned long long k0 = (unsigned long long)blockIdx.y * kChunk; k0 < r.nhist;
+         k0 += (unsigned long long)gridDim.y * kChunk) {
+      const unsigned kn = (unsigned)min((unsigned long long)kChunk, r.nhist - k0);
+      __syncthreads();
+      stage_chunk(bins, hist + r.hist_off + k0, (unsigned)k0, kn);
+      __syncthreads();
+      if (qv == 0.0) continue;
+      const double acc = pairsum_chunk(bins, (unsigned)k0, kn, qv, bin);
+      if (acc != 0.0) atomicAdd(&S[(size_t)r.srow * nq + iq], acc / (qv * bin));
+    }
+  }
+}
+
 // The plain FP32 form (XS_PAIRSUM_F32), for comparison: every term
 // h sin(q r)/(q r + 1e-8) evaluated in FP32 with the IEEE-accurate sinf, as
 // the reference GPU kernels evaluate theirs in FP32 (CalcFunctionsCUDA.cu:
@@ -227,6 +252,23 @@ __global__ void pdf_batch_kernel(const unsigned long long *__restrict__ hist, do
 }
 
 }  // namespace iq
+
+bool pairsum_short(const xs_ctx *ctx, size_t nrows, unsigned nhist_max, unsigned nq) {
+  return iq::short_sums(ctx, nrows, nhist_max, nq);
+}
+
+int pairsum_rows(xs_ctx *ctx, const unsigned long long *hist, const nodesum::Row *rows, unsigned nrows,
+                 unsigned nhist_max, double bin, const double *q, unsigned nq, double *S) {
+  const size_t ssize = (size_t)nrows * nq;
+  hipLaunchKernelGGL(iq::fill_f64, dim3((unsigned)std::min<size_t>((ssize + 255) / 256, 8192)), dim3(256), 0,
+                     ctx->stream, S, ssize);
+  const dim3 grid((nq + iq::kQBlock - 1) / iq::kQBlock,
+                  std::min(65535u, (nhist_max + iq::kChunk - 1) / iq::kChunk), std::min(65535u, nrows));
+  hipLaunchKernelGGL(iq::pairsum_rows_kernel, grid, dim3(iq::kQBlock), 0, ctx->stream, hist, rows, nrows, q, nq,
+                     bin, S);
+  XS_HIP_CHECK(hipGetLastError());
+  return XS_OK;
+}
 
 int batch_pdf_launch(xs_ctx *ctx, const unsigned long long *hist, const PdfDesc *desc,
                      unsigned nstruct, unsigned nblocks, int pdf_type, bool cpu_radius, double bin,

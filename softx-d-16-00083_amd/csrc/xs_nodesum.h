@@ -69,4 +69,11 @@ int run(xs_ctx *ctx, const Tables &T, const unsigned long long *hist, unsigned n
         const double *q, unsigned nq, double *S);
 
 }  // namespace nodesum
+
+// S (nrows x nq) of rows (on the device) bin by bin, overwritten (xs_iq.hip); launches
+// only, no memory of its own.  pairsum_short: where that is the faster form.
+bool pairsum_short(const xs_ctx *ctx, size_t nrows, unsigned nhist_max, unsigned nq);
+int pairsum_rows(xs_ctx *ctx, const unsigned long long *hist, const nodesum::Row *rows, unsigned nrows,
+                 unsigned nhist_max, double bin, const double *q, unsigned nq, double *S);
+
 }  // namespace xs

@@ -242,8 +242,9 @@ int grid_sort(xs_ctx *ctx, const double *x, const double *y, const double *z, si
               double min_cell, SortedPoints &out);
 
 // H3 as an int8 matrix-core product (device pointers, S[ncols * nq] overwritten).
+// host: the caller has just copied the inputs from the host.
 int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, unsigned nhist,
-                 double bin, const double *q, unsigned nq, double *S);
+                 double bin, const double *q, unsigned nq, double *S, bool host);
 
 // Launches only (no allocation, copy or wait; graph-capturable): slices of
 // the sinc matrix into a_buf, of the counts into b_buf, then the products;

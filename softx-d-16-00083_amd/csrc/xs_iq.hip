@@ -315,7 +315,7 @@ extern "C" int xs_hist_pairsum(xs_ctx *ctx, const uint64_t *hist, unsigned ntype
   if ((flags & XS_PAIRSUM_MFMA) && (flags & XS_PAIRSUM_F32))
     return fail(XS_ERR_ARG, "xs_hist_pairsum: XS_PAIRSUM_MFMA and XS_PAIRSUM_F32 exclude each other");
   if (flags & XS_PAIRSUM_MFMA) {
-    XS_TRY(pairsum_mfma(ctx, hd, ntypes, nhist, bin, qd, nq, Sd));
+    XS_TRY(pairsum_mfma(ctx, hd, ntypes, nhist, bin, qd, nq, Sd, !device));
   } else {
     const nodesum::Layout L =
         nodesum::layout((ntypes + nodesum::kRows - 1) / nodesum::kRows, nhist, nodesum::kBudget);

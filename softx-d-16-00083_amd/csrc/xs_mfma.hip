@@ -549,10 +549,14 @@ static int mm::products(xs_ctx *ctx, const MfmaBatchPlan &plan, const unsigned l
 }
 
 int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, unsigned nhist,
-                 double bin, const double *q, unsigned nq, double *S) {
+                 double bin, const double *q, unsigned nq, double *S, bool host) {
   using namespace mm;
   const unsigned MT = (nq + 127) / 128 * 4;
   const unsigned KT = (nhist + 31) / 32;
+  // A small call (not 16 k tiles for every CU): one launch for all slice counts, no waves
+  // side by side, which would halve its few work groups (100 x 100 bins x 4,000 q: 59 us
+  // side by side and with one launch to clear S, 43 so)
+  const bool small = (size_t)(MT / 4) * ((ncols + 127) / 128) * KT < 16 * (size_t)ctx->cu_count;
   const size_t aBytes = (size_t)kNA * MT * KT * 1024;
   XS_TRY(ensure_matrix(ctx, Carver::need({aBytes, (size_t)ncols * 8, (size_t)ncols * 4})));
   XS_TRY(ensure_pinned(ctx, align_up((size_t)ncols * 8, 256) + (size_t)ncols * 4));
@@ -574,20 +578,23 @@ int pairsum_mfma(xs_ctx *ctx, const unsigned long long *hist, unsigned ncols, un
   char *const pin = static_cast<char *>(ctx->pin);
   const size_t last_at = (size_t)(reinterpret_cast<char *>(last) - reinterpret_cast<char *>(bits));
   XS_HIP_CHECK(hipMemcpyAsync(pin, bits, last_at + (size_t)ncols * 4, hipMemcpyDeviceToHost, ctx->stream));
-  if (!ctx->read_back) XS_HIP_CHECK(hipEventCreateWithFlags(&ctx->read_back, hipEventDisableTiming));
-  XS_HIP_CHECK(hipEventRecord(ctx->read_back, ctx->stream));
-  launch_slice_sinc(ctx, q, nq, nhist, bin, MT, KT, As);
-  XS_HIP_CHECK(hipGetLastError());
-  XS_HIP_CHECK(hipEventSynchronize(ctx->read_back));
+  if (small && host) {
+    // (after copies from the host an event's wait takes 6 to 12 us longer than the stream's)
+    XS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    launch_slice_sinc(ctx, q, nq, nhist, bin, MT, KT, As);
+    XS_HIP_CHECK(hipGetLastError());
+  } else {
+    if (!ctx->read_back) XS_HIP_CHECK(hipEventCreateWithFlags(&ctx->read_back, hipEventDisableTiming));
+    XS_HIP_CHECK(hipEventRecord(ctx->read_back, ctx->stream));
+    launch_slice_sinc(ctx, q, nq, nhist, bin, MT, KT, As);
+    XS_HIP_CHECK(hipGetLastError());
+    XS_HIP_CHECK(hipEventSynchronize(ctx->read_back));
+  }
   std::vector<unsigned long long> off(ncols), bound(ncols);
   std::vector<uint32_t> extent(ncols);
   std::memcpy(bound.data(), pin, (size_t)ncols * 8);
   std::memcpy(extent.data(), pin + last_at, (size_t)ncols * 4);
   for (unsigned c = 0; c < ncols; ++c) off[c] = (unsigned long long)c * nhist;
-  // A small call (not 16 k tiles for every CU): one launch for all slice counts, no waves
-  // side by side, which would halve its few work groups (100 x 100 bins x 4,000 q: 59 us
-  // side by side and with one launch to clear S, 43 so)
-  const bool small = (size_t)(MT / 4) * ((ncols + 127) / 128) * KT < 16 * (size_t)ctx->cu_count;
   if (small) {
     unsigned long long all = 0;
     for (unsigned long long b : bound) all |= b;

@@ -121,6 +121,8 @@ __global__ __launch_bounds__(256) void slice_sinc(const double *__restrict__ q, 
   const unsigned lane = tid & 63, kg = (tid >> 6) % KG, mt = (unsigned)((tid >> 6) / KG);
   const unsigned row = mt * 32 + (lane & 31), half = 16 * (lane >> 5);
   const double qv = row < nq ? q[row] : 0.0, qb = qv * bin;
+  // (of four of which a product is taken: beyond 1e60 the values are 0 either way)
+  const double qd = fmin(fmax(qb, -1e60), 1e60);
   double s = 0, c = 1, ds = 0, dc = 1, js = 0, jc = 1;
   if (qv != 0.0) {
     const double turns = qb / (2.0 * kPi);
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(256) void slice_sinc(const double *__restrict__ q, 
       double d[4], v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        d[e] = fma((double)(k0 + 4 * g + e) + 0.5, qb, 1e-8);
+        d[e] = fma((double)(k0 + 4 * g + e) + 0.5, qd, 1e-8);
         v[e] = s;
         rotate(ds, dc);
       }

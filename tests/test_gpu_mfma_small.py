@@ -29,3 +29,17 @@ def test_small(ncols, nhist, nq):
     ref = O.hist_pairsum(h, 0.02, q[pick])
     bar = (2.0 ** -35 + 1e-13) * h.astype(np.float64).sum(axis=1, keepdims=True)
     assert np.all(np.abs(S[:, pick] - ref) <= bar)
+
+
+def test_huge_q():
+    """|q| r beyond 1e77, where the product of four denominators would overflow: terms of 0,
+    and the other q as without them."""
+    h = np.arange(1, 301, dtype=np.uint64).reshape(2, 150)
+    q = np.array([0.5, 1e78, 2.0, -1e90, 1e200, 3.0])
+    print("mfma: huge q", flush=True)
+    with xh.Context(0) as ctx:
+        S = ctx.hist_pairsum(h, 0.02, q, mfma=True)
+    small = np.abs(q) < 10
+    bar = (2.0 ** -35 + 1e-13) * h.astype(np.float64).sum(axis=1, keepdims=True)
+    assert np.all(np.abs(S[:, small] - O.hist_pairsum(h, 0.02, q[small])) <= bar)
+    assert np.all(np.abs(S[:, ~small]) <= bar)

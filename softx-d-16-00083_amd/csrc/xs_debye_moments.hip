@@ -192,6 +192,15 @@ __device__ __forceinline__ void add_exact(double &hi, double &lo, double v) {
   hi = s;
 }
 
+// The same while |hi| >= |v| (Dekker); where hi is smaller, near a zero of the sum, v is
+// rounded as it would be anyway.
+__device__ __forceinline__ void add_to_larger(double &hi, double &lo, double v) {
+#pragma clang fp contract(off)
+  const double s = hi + v;
+  lo += v - (s - hi);
+  hi = s;
+}
+
 // part[share][row][q] = q times the sum over a share's nodes, chunk by chunk (every
 // gridDim.x-th); grid (shares, q blocks, row groups).
 // A node stands for many pairs, so its phase q r is carried beyond FP64 (turn: h / 2 pi
@@ -201,6 +210,7 @@ __device__ __forceinline__ void add_exact(double &hi, double &lo, double v) {
 // 1,500 atoms, q to 20 1/A: 1.2e-16 sqrt(pairs) at high q and 2e-15 max |S| at low q, as
 // the sums pair by pair; 2e-15 and 6e-14 with neither.
 constexpr int kEvalNodes = 64;
+static_assert(kMaxMoments <= kEvalNodes, "a bin a chunk at least");
 constexpr unsigned kExactNodes = 4;  // whose sum is rounded
 template <int RG>
 __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M, unsigned nb, int K,
@@ -227,22 +237,23 @@ __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M,
 #pragma unroll
   for (int g = 0; g < RG; ++g) sum[g] = rest[g] = 0.0;
   for (unsigned b0 = blockIdx.x * cb; b0 <= nb; b0 += gridDim.x * cb) {
-    const unsigned nbin = min(cb, nb + 1 - b0);
+    const unsigned nbin = min(cb, nb + 1 - b0), nn = (nbin * K + kExactNodes - 1) / kExactNodes * kExactNodes;
     __syncthreads();
-    for (unsigned i = threadIdx.x; i < nbin * K; i += 256) {
+    for (unsigned i = threadIdx.x; i < nn; i += 256) {
       const unsigned b = b0 + i / K;
       const int m = i % K;
       const double t = 0.5 * K * ct[m * K + 1];
       // r / h as x + dx (t to FP64: its bin's share of the distance is small)
       const double c = (b == nb ? 0.0 : (double)b) + 0.5, x = fma(0.5, t, c);
       const double dx = fma(0.5, t, c - x), ir = 1.0 / (x * h), rt = x * turn.x;
+      // (beyond the last node: any, of weight 0)
       node[i] = make_double4(rt, b == nb ? 0.0 : ir, b == nb ? ir : b == 0 ? 0.0 : ir * ir,
                              fma(x, turn.x, -rt) + fma(x, turn.y, dx * turn.x));
     }
-    for (unsigned i = threadIdx.x; i < nbin * K * RG; i += 256) {
+    for (unsigned i = threadIdx.x; i < nn * RG; i += 256) {
       const unsigned n = i / RG, g = i % RG, row = row0 + g;
       double w = 0.0;
-      if (row < nrows) {
+      if (row < nrows && n < nbin * K) {
         const double *mk = M + ((size_t)row * (nb + 1) + b0 + n / K) * K;
         const double *c = ct + (n % K) * K;
         for (int k = 0; k < K; ++k) w = fma(mk[k], c[k], w);
@@ -250,11 +261,12 @@ __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M,
       W[n][g] = w;
     }
     __syncthreads();
-    for (unsigned n0 = 0; n0 < nbin * K; n0 += kExactNodes) {
+    for (unsigned n0 = 0; n0 < nn; n0 += kExactNodes) {
       double acc[RG];
 #pragma unroll
       for (int g = 0; g < RG; ++g) acc[g] = 0.0;
-      for (unsigned n = n0; n < min(n0 + kExactNodes, nbin * K); ++n) {
+#pragma unroll
+      for (unsigned n = n0; n < n0 + kExactNodes; ++n) {
         const double4 v = node[n];
         double s, c;
         sincos_turn_tab(fma(qv, v.w, fma(qv, v.x, -rint(qv * v.x))), tab, &s, &c);
@@ -263,7 +275,7 @@ __global__ __launch_bounds__(256) void eval_kernel(const double *__restrict__ M,
         for (int g = 0; g < RG; ++g) acc[g] = fma(W[n][g], f, acc[g]);
       }
 #pragma unroll
-      for (int g = 0; g < RG; ++g) add_exact(sum[g], rest[g], acc[g]);
+      for (int g = 0; g < RG; ++g) add_to_larger(sum[g], rest[g], acc[g]);
     }
   }
   if (iq >= nq) return;
@@ -341,13 +353,13 @@ int run_moments(xs_ctx *ctx, const MomentPlan &plan, const double *xyz, size_t n
   Run *runs_d = reinterpret_cast<Run *>(w);
   uint32_t *row_d = reinterpret_cast<uint32_t *>(w + align_up(rb, 256));
   // the evaluation: chunks of cb bins (the near pairs' among them), up to 8 rows at once,
-  // as many shares of the chunks as give four work groups a CU
+  // as many shares of the chunks as give eight work groups a CU
   const size_t ssize = (size_t)nrows * nq;
   const unsigned groups = (nrows + 7) / 8, rg = (nrows + groups - 1) / groups;
   const unsigned cb = std::max(1, kEvalNodes / b.K), chunks = (b.nb + 1 + cb - 1) / cb;
   const size_t eval_groups = (size_t)((nq + 255) / 256) * ((nrows + rg - 1) / rg);
   const unsigned shares =
-      runs.empty() ? 0 : (unsigned)std::min<size_t>(chunks, std::max<size_t>(1, 4 * ctx->cu_count / eval_groups));
+      runs.empty() ? 0 : (unsigned)std::min<size_t>(chunks, std::max<size_t>(1, 8 * ctx->cu_count / eval_groups));
   XS_TRY(ensure_matrix(ctx, Carver::need({runs.size() * entries * 8, nrows * entries * 8,
                                           shares > 1 ? shares * ssize * 8 : 0})));
   Carver cv(ctx->mat);

@@ -799,8 +799,8 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     Args<double> A) {
 #pragma clang fp contract(off)
   __shared__ uint32_t win[WCAP + kTrash];
-  __shared__ uint32_t over, kept;  // pairs past nhist (an item has fewer than 2^32); FEW: J tiles
   __shared__ unsigned long long keys[kSortCap];
+  __shared__ uint32_t over, kept;  // pairs past nhist (an item has fewer than 2^32); FEW: J tiles
 
   const Item it = A.items[blockIdx.x];
   const TypeDesc td = A.types[it.type];
@@ -830,8 +830,11 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     }
   }
   unsigned long long *hp = A.hist + td.hist_off;
-  if (tid == 0) over = kept = 0u;
-  if (FEW) __syncthreads();
+  if (tid == 0) over = 0u;
+  if constexpr (FEW) {
+    if (tid == 0) kept = 0u;
+    __syncthreads();
+  }
 
   // Tile pairs of few pairs: a wave each, pair by pair, exactly and straight to the
   // histogram.  (A few atoms over many bins have tiles of one atom, for which the loads
@@ -877,16 +880,14 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
         bool fits;
         box_bins(bu, A.boxes + 6 * (size_t)(td.b_base + tj), bin, nhist, kl, ku, fits);
         key = ((unsigned long long)kl << 32) | m;
-        if (FEW) atomicAdd(&kept, 1u);
+        if constexpr (FEW) atomicAdd(&kept, 1u);
       }
     }
     keys[m] = key;
   }
-  uint32_t n = it.jcount;
-  if (FEW) {
+  if constexpr (FEW) {
     __syncthreads();
-    n = __builtin_amdgcn_readfirstlane(kept);
-    if (n == 0) {
+    if (kept == 0) {
       if (tid == 0 && over) atomicAdd(A.overflow + td.ovf, (unsigned long long)over);
       return;
     }
@@ -910,6 +911,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     }
   }
 
+  const uint32_t n = FEW ? __builtin_amdgcn_readfirstlane(kept) : it.jcount;
   // The window holds bins [B, B + WCAP), bin k in slot k - B; none at or past `top`
   // has a count.
   uint32_t B = (uint32_t)(keys[0] >> 32), top = B;

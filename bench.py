@@ -49,10 +49,10 @@ OPS_PER_PAIR = 11                 # 3 sub, 3 mul, 2 add, sqrt, div, cvt
 # the two do not overlap.  A CU issues one 64-lane instruction per cycle (4 SIMDs x 16
 # lanes), so the fraction of the CUs' issue cycles at the 2.4 GHz peak clock the kernel
 # spends issuing is SLOTS_PER_PAIR * pairs / 64 / (256 * 2.4e9 * t).
-SLOTS_PER_PAIR = 14.08
+SLOTS_PER_PAIR = 14.07
 CU_ISSUE_PER_S = 256 * 2.4e9
 # FP32 binning kernel (hist_kernel_f32<32768, true>) on the same workload:
-# SQ_ACTIVE_INST_VALU reads 20.06 wave-instructions per 64 pairs.  Its
+# SQ_ACTIVE_INST_VALU reads 20.25 wave-instructions per 64 pairs.  Its
 # roofline fraction is the algorithmic one of the FP64 line: 11 ops per pair
 # x pairs / t against MI355X's FP32 vector peak (157.3 TFLOP/s).  Beside it,
 # the issue rate it reaches in wave-instructions per CU-cycle at 2.4 GHz:
@@ -60,7 +60,7 @@ CU_ISSUE_PER_S = 256 * 2.4e9
 # (measured), i.e. up to two FP32 wave-instructions per CU-cycle against one
 # for FP64, so each kernel's issue rate is read against the peak of its own
 # instruction type (2 for this one, 1 for the FP64 kernel).
-F32_ACTIVE_PER_64_PAIRS = 20.06
+F32_ACTIVE_PER_64_PAIRS = 20.25
 FP32_PEAK_TFLOPS = 157.3
 # Direct Debye: the direct form's unit is 4 ops per pair-q term (sin, q r, x 1/(q r),
 # accumulate).  The kernels go through moments of the pair distances and execute far
@@ -75,7 +75,7 @@ AMP2D_OPS_PER_TERM = 2 * 2 + 14 / 16
 # rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (KiB per dispatch), scaled by
 # the counters' reading for a 1 GiB device-to-device copy (FETCH_SIZE reads
 # 524,308 KiB for the 1,048,576 KiB copied, WRITE_SIZE 1,048,576 KiB).
-HIST_FETCH_KIB, HIST_WRITE_KIB = 7096870, 9979720
+HIST_FETCH_KIB, HIST_WRITE_KIB = 7075300, 9979410
 FETCH_SCALE, WRITE_SCALE = 1048576 / 524308, 1.0
 HIST_TRAFFIC_BYTES = int((HIST_FETCH_KIB * FETCH_SCALE + HIST_WRITE_KIB * WRITE_SCALE) * 1024)
 

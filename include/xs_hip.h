@@ -120,6 +120,7 @@ int xs_hist(xs_ctx *ctx, const void *xyz, size_t n_atoms,
  * r_k = (k+1/2) bin, S = 0 where q = 0.  FP64: groups of bins act through 64
  * Chebyshev nodes each, to FP64 rounding (every bin by itself where they are
  * wider than ~0.6 / max |q|); the sums over the nodes are matrix products.
+ * Up to 384 bins are summed bin by bin where that is faster.
  * Replaces the bin loop of calcInt1DHist (CalcFunctions.cpp:844-871) and
  * calcIntHistKernelXray/Neutron (CalcFunctionsCUDA.cu:923-985).
  * XS_PAIRSUM_MFMA evaluates the same sums as one product S = H A^T on the
@@ -127,7 +128,8 @@ int xs_hist(xs_ctx *ctx, const void *xyz, size_t n_atoms,
  * counts into exact 7-bit slices, int32 accumulation; the result differs
  * from the FP64 sum by about 2^-35 sum_k h[k] (needs counts < 2^35 and a
  * workspace of ~5 nq nhist bytes, and reads the counts' extents back).  The
- * FP64 form is faster where 64 nodes stand for more than ~300 bins.
+ * flag chooses the arithmetic, not the faster form: where 64 nodes stand for
+ * more than ~300 bins the FP64 form is faster.
  * On device arrays and without XS_PAIRSUM_MFMA the call may be captured: it
  * then sums bin by bin, without scratch (as it does where the node tables'
  * memory, at most ~260 MiB + 16 bytes a bin, cannot be had).
@@ -152,11 +154,11 @@ int xs_pdf(xs_ctx *ctx, const uint64_t *hist, unsigned n_el,
 /* H5: direct Debye pair sums S[p*nq+iq] = sum_{pairs in p} sin(q r)/(q r + 1e-8)
  * with FP64 pair terms (xyz double).  Where that is cheaper the sums go
  * through Chebyshev moments of the pair distances, to the FP64 rounding of a
- * pair's term; else, on a
- * uniform q mesh (the reference's, ReadXML.cpp:220-222) sin(q r) advances
- * from q to q by a rotation, and other meshes evaluate the series per q.
- * Replaces the pair loop of calcIntDebye
- * (CalcFunctions.cpp:561-591) and calcIntDebyeKernel (CalcFunctionsCUDA.cu:1163-1273). */
+ * pair's term; else, on a uniform q mesh (the reference's,
+ * ReadXML.cpp:220-222) sin(q r) advances from q to q by a recurrence, and
+ * other meshes evaluate the series per q.
+ * Replaces the pair loop of calcIntDebye (CalcFunctions.cpp:561-591) and
+ * calcIntDebyeKernel (CalcFunctionsCUDA.cu:1163-1273). */
 int xs_debye_pairsum(xs_ctx *ctx, const double *xyz, size_t n_atoms,
                      const unsigned *el_count, unsigned n_el, const double *q,
                      unsigned nq, double *S, unsigned flags);
@@ -202,12 +204,13 @@ int xs_amp2d(xs_ctx *ctx, const double *xyz, size_t n_atoms,
 
 /* H7 on a regular q grid: q(iu, iv) = q0 + iu du + iv dv (iu < nu, iv < nv),
  * point k = iv*nu + iu; otherwise as xs_amp2d (ff[el*nu*nv + k], I[k]).
- * Along a row the phase of an atom advances by (R^T du).x per point, so
- * runs of 8 points are evaluated from one FP32 hardware sine/cosine of the
- * FP64-reduced phase (the list kernel's accuracy) and FP64 complex
- * rotations.  q0, du, dv are host arrays of 3; the rest as xs_amp2d.  The
- * Cartesian q planes of 2D patterns are such grids; the reference's polar
- * (q, phi) mesh is not (use xs_amp2d). */
+ * Along a row the phase of an atom advances by (R^T du).x per point, so a
+ * run of 16 points takes one FP32 hardware sine/cosine of the FP64-reduced
+ * phase (the list kernel's accuracy), turned to the run's middle in FP64; the
+ * sums over the atoms of its product with the sines and cosines of the
+ * points' steps from there are FP64 matrix products.  q0, du, dv are host
+ * arrays of 3; the rest as xs_amp2d.  The Cartesian q planes of 2D patterns
+ * are such grids; the reference's polar (q, phi) mesh is not (use xs_amp2d). */
 int xs_amp2d_grid(xs_ctx *ctx, const double *xyz, size_t n_atoms, const unsigned *el_count,
                   unsigned n_el, const double *q0, const double *du, const double *dv,
                   unsigned nu, unsigned nv, const double *rot, unsigned nrot, const double *ff,
@@ -269,7 +272,8 @@ int xs_batch_info(const xs_batch *plan, unsigned *nhist,
 
 /* Histograms of every structure (as xs_hist), then, if S != NULL and nq > 0,
  * pair sums S[t*nq+iq] of every pair type t (as xs_hist_pairsum, one q mesh
- * for all), then, if pdf != NULL, PDFs of pdf_type (as xs_pdf) with rho0[s]
+ * for all; bin by bin where the memory for the node tables cannot be had),
+ * then, if pdf != NULL, PDFs of pdf_type (as xs_pdf) with rho0[s]
  * and sl[] in el_count order.  XS_DEVICE_PTRS: hist, q, S and pdf are device
  * pointers and the call returns without waiting; else host arrays and the
  * call is synchronous.  XS_BATCH_GRAPH: the launches are captured into a

@@ -14,8 +14,8 @@
 // are given out in shares, the amplitudes are.  Bound by the issue of one term:
 // three FMAs, v_fract_f64 (a floor and a subtraction took 5 cycles more), a
 // conversion to FP32, two hardware sines, two conversions back and two adds,
-// ~55 cycles of a SIMD for 64 points; 20,000 atoms x 92,160 points x 4 rotations
-// 2.87 ms (3.11 with floor and one share).
+// 53 cycles of a SIMD for 64 points, all of them issue; 20,000 atoms x 92,160
+// points x 4 rotations 2.87 ms (3.11 with floor and one share).
 #include <algorithm>
 #include <cmath>
 

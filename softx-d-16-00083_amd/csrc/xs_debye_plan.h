@@ -51,10 +51,10 @@ inline size_t moments_lds_bytes(unsigned nb, int K) {
 }
 
 // Cycles of the CUs for one call, to choose K and to leave small inputs to
-// debye_kernel.  Measured: 143 cycles a wave of 64 pairs for K = 8 on the
-// 8,000-atom rock-salt cube (1,560 bins) and 250 for K = 12 on 5,000 atoms
-// (290 bins), about 20 a moment; the evaluation's sines at half the issue
-// rate; 25 us for the launches and the copy of the tables.
+// debye_kernel.  Measured: 199 cycles a wave of 64 pairs for K = 10 on the
+// 8,000-atom rock-salt cube, the launch's start and end included, about 20 a
+// moment (172 for K = 12 on 50,000 atoms, 14 a moment); the evaluation's sines
+// at half the issue rate; 25 us for the launches and the copy of the tables.
 inline double moments_cycles(double pairs, double rows, double rgroups, unsigned nq,
                              const nodes::Bins &b, double cus) {
   const double per_pair = 20.0 * b.K / 64.0;

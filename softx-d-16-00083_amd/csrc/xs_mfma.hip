@@ -275,7 +275,7 @@ __device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
 // tile), 50%.  Two waves side by side (WN = 2) load 14 KiB instead of 24 for the
 // products of four waves.  A work group per group and 128 q left CUs idle 40% of the
 // time with two slices (a round and a quarter of work groups of unequal length): 530
-// us for the products, 400 in equal shares.  Particles of 500 to 8,000 atoms leave a
+// us for the products, 400 to 490 in equal shares.  Particles of 500 to 8,000 atoms leave a
 // third of the bins empty past each column's last, and half of the columns take one
 // slice: as columns of one k range and slice count the products took 790.
 //
